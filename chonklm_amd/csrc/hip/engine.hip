@@ -2680,6 +2680,20 @@ int32_t run_token(chonk_engine* e, int32_t token, bool need_logits, const chonk_
   return 0;
 }
 
+// tokens[0, n) appended to the context through the prompt pass: K/V, token
+// history and position on the host and the device.
+void append_rows(chonk_engine* e, const int32_t* tokens, size_t n) {
+  if (n == 0) return;
+  HIP_OK(hipMemcpy(e->hist + e->pos, tokens, n * 4, hipMemcpyHostToDevice));
+  prefill_rows(e, tokens, (int)n);
+  e->pos += (int)n;
+  DevState st = read_state(e);
+  st.pos = e->pos;
+  upload_state_fields(e, st);
+  e->known_token_pos = -1;
+  e->logits_valid = false;
+}
+
 int64_t common_prefix(const std::vector<int32_t>& a, const int32_t* b, size_t nb) {
   const size_t n = std::min(a.size(), nb);
   size_t i = 0;
@@ -2868,7 +2882,17 @@ void generate_stepped(chonk_engine* e, const int32_t* prompt, size_t n_prompt, i
   if (n_suffix == 0 && e->has_cached_next) {
     next = e->cached_next;
   } else {
-    for (size_t i = 0; i < n_suffix; ++i) {
+    size_t done = 0;
+    if (e->batched_prefill && n_suffix > 1) {
+      // all but the last prompt token as row batches (as generate does): a
+      // 300-token prompt of the Qwen3-0.6B shape in 6 ms instead of 300 steps
+      // of 0.7 ms. A prompt past the context fills it and then fails at the
+      // first token that does not fit, as token-by-token steps would.
+      const size_t room = (size_t)(e->cfg.ctx - e->pos);
+      done = std::min(n_suffix - 1, room);
+      append_rows(e, prompt + prefix, done);
+    }
+    for (size_t i = done; i < n_suffix; ++i) {
       const bool need = i + 1 == n_suffix;
       const size_t n_pen = (size_t)prefix + i + 1;
       next = run_token(e, prompt[prefix + i], need, &s, prompt, need ? n_pen : 0, prompt, need ? n_pen : 0);
@@ -3000,14 +3024,7 @@ int chonk_engine_prefill(chonk_engine* e, const int32_t* tokens, size_t n) {
       e->logits_valid = false;
       return;
     }
-    HIP_OK(hipMemcpy(e->hist + e->pos, tokens, n * 4, hipMemcpyHostToDevice));
-    prefill_rows(e, tokens, (int)n);
-    e->pos += (int)n;
-    DevState st = read_state(e);
-    st.pos = e->pos;
-    upload_state_fields(e, st);
-    e->known_token_pos = -1;
-    e->logits_valid = false;
+    append_rows(e, tokens, n);
   });
 }
 
