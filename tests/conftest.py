@@ -1,6 +1,7 @@
 """Shared fixtures. GPU tests carry @pytest.mark.gpu and run on an MI355X."""
 from __future__ import annotations
 
+import gc
 import os
 import sys
 from pathlib import Path
@@ -20,6 +21,15 @@ def pytest_configure(config):
 @pytest.fixture(scope="session")
 def model_dir(tmp_path_factory):
     return tmp_path_factory.mktemp("models")
+
+
+@pytest.fixture(autouse=True)
+def _free_engines():
+    """A test that keeps an ExceptionInfo leaves its frame, and the engine in it, in
+    a reference cycle: collected here, so that no engine outlives its test (how many
+    are alive decides which decode kernels the next test's engine takes)."""
+    yield
+    gc.collect()
 
 
 _CACHE: dict[str, str] = {}
