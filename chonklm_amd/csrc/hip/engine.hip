@@ -2122,13 +2122,15 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
   e->step_plain = e->kernels_plain;
   // CHONK_PREFILL=token keeps the reference's token-by-token prompt pass
   const char* pv = std::getenv("CHONK_PREFILL");
-  // (the row-batch glue kernels hold a row of at most 4096 elements in registers)
-  e->batched_prefill = !(pv && std::strcmp(pv, "token") == 0) && !c.gpt && !c.lfm && !c.granite &&
-                       std::max(c.hidden, std::max(c.heads * c.hd, c.ffn)) <= 4096;
+  // (the row-batch glue kernels hold a row of at most kPfRowMax elements in registers)
+  const int widest = std::max({c.hidden, c.heads * c.hd, c.ffn, c.ssm_inner});
+  e->batched_prefill = !(pv && std::strcmp(pv, "token") == 0) && widest <= kPfRowMax;
   // the no-allocation prompt pass: as many rows (a multiple of 16, at most one
-  // full pass) as fit the scratch with this model's row buffers
+  // full pass) as fit the scratch with this model's row buffers (the llama
+  // family, rows of at most 4096 elements)
   e->scratch = scratch_address(e->device);
-  e->noalloc_rows = e->batched_prefill ? noalloc_rows_for(c) : 0;
+  e->noalloc_rows =
+      e->batched_prefill && !c.gpt && !c.lfm && !c.granite && widest <= 4096 ? noalloc_rows_for(c) : 0;
   const char* ng = std::getenv("CHONK_NO_GRAPH");
   e->use_graph = !(ng && ng[0] == '1');
   for (const Launch& L : e->kernels_logits)
@@ -2315,7 +2317,9 @@ struct RowBufs {
 int64_t row_part_floats(const ModelCfg& c, int rows) {
   const int64_t R = rows;
   const int64_t qkv = (int64_t)(c.heads + 2 * c.kv_heads) * c.hd;
-  return std::max<int64_t>({kPartFloats, R * qkv, 2 * R * c.ffn, R * c.hidden});
+  // (the in_proj rows of a convolution or Mamba2 layer)
+  const int64_t in_proj = c.lfm ? 3 * c.hidden : c.ssm_inner ? c.ssm_inner + c.ssm_conv + c.ssm_heads : 0;
+  return std::max<int64_t>({kPartFloats, R * qkv, 2 * R * c.ffn, R * c.hidden, R * in_proj});
 }
 
 // Sizes the buffers of `rows` rows for the engine's model; returns the bytes
@@ -2323,8 +2327,10 @@ int64_t row_part_floats(const ModelCfg& c, int rows) {
 size_t row_bufs_layout(const ModelCfg& c, int rows, uint8_t* base, RowBufs* out) {
   const size_t R = rows;
   const size_t H = c.hidden, qdim = (size_t)c.heads * c.hd, kvdim = (size_t)c.kv_heads * c.hd, F = c.ffn;
-  const size_t kmax = gemm_kpad((int)std::max(H, std::max(qdim, F)));
-  const size_t sizes[12] = {R * H * 4, R * (qdim + 2 * kvdim) * 4, R * qdim * 4, R * F * 4, R * F * 4, R * F * 4,
+  // (Mamba2 layers: the convolved rows in g, the scan's output in u)
+  const size_t inner = c.ssm_inner, G = std::max(F, inner ? (size_t)pf_mamba_ld(c.ssm_conv, c.ssm_heads) : 0);
+  const size_t kmax = gemm_kpad((int)std::max({H, qdim, F, inner}));
+  const size_t sizes[12] = {R * H * 4, R * (qdim + 2 * kvdim) * 4, R * qdim * 4, R * G * 4, R * std::max(F, inner) * 4, R * F * 4,
                             R * H * 4, R * 4, (size_t)row_part_floats(c, rows) * 4, R * kmax * 2, R * kmax * 2, R * 4};
   size_t off = 0;
   void* ptr[12];
@@ -2376,7 +2382,8 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
   const int H = c.hidden;
   // split of x into the GEMM operand planes, after the pending residual update
   // (x += add, or the Gemma-3 sandwich with add_w) when add.p is set
-  auto split = [&](const float* x, int ld, int k, const float* w, int rows, PartSum add, const float* add_w) {
+  auto split = [&](const float* x, int ld, int k, const float* w, int rows, PartSum add, const float* add_w,
+                   const float* add_bias = nullptr, const float* norm_b = nullptr) {
     PfSplitArgs a{};
     a.x = x;
     a.ldx = ld;
@@ -2389,6 +2396,9 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
     a.xscale = b.xscale;
     a.add = add;
     a.add_w = add_w;
+    a.add_scale = c.res_scale;
+    a.add_bias = add_bias;
+    a.norm_b = norm_b;
     HIP_OK(launch_pf_split(a, rows, s));
   };
   // GEMM of the operand planes with the result left as partial sums in
@@ -2450,104 +2460,159 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
     return k;
   };
   const int64_t P = b.part_cap;
-  HIP_OK(launch_pf_embed(e->embed.q, b.tok, c.embed_scale, H, b.x, T, s));
+  HIP_OK(launch_pf_embed(e->embed.q, b.tok, c.embed_scale, c.gpt ? e->pos_embd : nullptr, pl.p0, H, b.x, T, s));
   PartSum pending{};                // the previous layer's ffn_down, not yet added to x
   const float* pending_w = nullptr; // its Gemma-3 post-ffn norm
+  const float* pending_b = nullptr; // its GPT-2 bias
   for (int i = 0; i < c.layers; ++i) {
     const LayerDev& L = e->layers[i];
     const LayerCfg& lc = c.layer[i];
     const int qdim = lc.heads * c.hd, kvdim = lc.kv_heads * c.hd, F = lc.ffn;
     const int ldqkv = qdim + 2 * kvdim;
-    split(b.x, H, H, L.in_norm, T, pending, pending_w);
+    const bool last_kv = i == c.layers - 1 && !logits;  // only the last layer's K/V (or state) are needed from it
+    split(b.x, H, H, L.in_norm, T, pending, pending_w, pending_b, L.in_norm_b);
     pending = PartSum{};
-    PfRopeArgs r{};
-    PartSum fused{};
-    if (c.openelm) {
-      // one fused q|k|v result; k and v are column ranges of it
-      const PartSum f = gemm(L.qkv, T, 0, P);
-      r.pq = columns(f, 0, qdim);
-      r.pk = columns(f, qdim, kvdim);
-      r.pv = columns(f, qdim + kvdim, kvdim);
-    } else if (gemm_fused({&L.q, &L.k, &L.v}, T, &fused)) {
-      r.pq = columns(fused, 0, qdim);
-      r.pk = columns(fused, qdim, kvdim);
-      r.pv = columns(fused, qdim + kvdim, kvdim);
+    PartSum po{};  // the block's output projection, not yet added to x
+    if (lc.conv) {
+      PfConvArgs cv{};
+      cv.p = gemm(L.conv_in, T, 0, P);
+      cv.k = H;
+      cv.kpad = gemm_kpad(H);
+      cv.w = L.conv_w;
+      cv.s1 = L.conv_s1;
+      cv.s2 = L.conv_s2;
+      cv.xh = b.h;
+      cv.xl = b.l;
+      cv.xscale = b.xscale;
+      if (!last_kv) HIP_OK(launch_pf_conv(cv, T, s));
+      HIP_OK(launch_pf_conv_state(cv, T, s));
+      if (last_kv) break;
+      po = gemm(L.conv_out, T, 0, P);
+    } else if (lc.mamba) {
+      PfMambaArgs m{};
+      m.p = gemm(L.ssm_in, T, 0, P);
+      m.rows = T;
+      m.inner = c.ssm_inner;
+      m.conv = c.ssm_conv;
+      m.heads = c.ssm_heads;
+      m.p0 = pl.p0;
+      m.conv_w = L.c1d_w;
+      m.conv_b = L.c1d_b;
+      m.dt_bias = L.dt_b;
+      m.a_neg = L.a_neg;
+      m.d = L.d_w;
+      m.conv_state = L.mconv_state;
+      m.ssm_state = L.ssm_state;
+      m.xbc = b.g;
+      m.y = b.u;
+      HIP_OK(launch_pf_mamba(m, s));
+      if (last_kv) break;
+      PfGateArgs gt{};
+      gt.z = columns(m.p, 0, c.ssm_inner);
+      gt.y = b.u;
+      gt.w = L.ssm_norm;
+      gt.k = c.ssm_inner;
+      gt.kpad = gemm_kpad(c.ssm_inner);
+      gt.eps = c.eps;
+      gt.xh = b.h;
+      gt.xl = b.l;
+      gt.xscale = b.xscale;
+      HIP_OK(launch_pf_gate(gt, T, s));
+      po = gemm(L.ssm_out, T, 0, P);
     } else {
-      // the partial-sum buffer shared out in proportion to each result's size
-      const int64_t pq = P * qdim / ldqkv, pk = P * kvdim / ldqkv;
-      r.pq = gemm(L.q, T, 0, pq);
-      r.pk = gemm(L.k, T, pq, pk);
-      r.pv = gemm(L.v, T, pq + pk, P - pq - pk);
+      PfRopeArgs r{};
+      PartSum fused{};
+      if (c.openelm || c.gpt) {
+        // one fused q|k|v result; k and v are column ranges of it
+        const PartSum f = gemm(L.qkv, T, 0, P);
+        r.pq = columns(f, 0, qdim);
+        r.pk = columns(f, qdim, kvdim);
+        r.pv = columns(f, qdim + kvdim, kvdim);
+        r.bias = L.qkv_b;
+      } else if (gemm_fused({&L.q, &L.k, &L.v}, T, &fused)) {
+        r.pq = columns(fused, 0, qdim);
+        r.pk = columns(fused, qdim, kvdim);
+        r.pv = columns(fused, qdim + kvdim, kvdim);
+      } else {
+        // the partial-sum buffer shared out in proportion to each result's size
+        const int64_t pq = P * qdim / ldqkv, pk = P * kvdim / ldqkv;
+        r.pq = gemm(L.q, T, 0, pq);
+        r.pk = gemm(L.k, T, pq, pk);
+        r.pv = gemm(L.v, T, pq + pk, P - pq - pk);
+      }
+      r.qkv = b.qkv;
+      r.ld = ldqkv;
+      r.hd = c.hd;
+      r.heads = lc.heads;
+      r.kv_heads = lc.kv_heads;
+      r.interleaved = c.interleaved ? 1 : 0;
+      r.kv16 = e->kv_elem == 2 ? 1 : 0;
+      r.qn_w = c.qk_norm ? L.q_norm : nullptr;
+      r.kn_w = c.qk_norm ? L.k_norm : nullptr;
+      r.eps = c.qk_eps;
+      r.rope_inv = rope_table(e, c.layer[i].theta, c.hd);
+      r.kv = kv_addr(i);
+      // decode batches: the page-walking attention (one workgroup per (kv head,
+      // row) walking all of its pages also does the rotary/K-V write)
+      const bool walk = pl.row_seq && c.hd >= 64 && lc.heads / lc.kv_heads <= 8 && kvs.max_pages <= 64;
+      const bool fuse_rope = walk && !last_kv && bd_attn_segments(T, lc.kv_heads, kvs.max_pages) == 1;
+      if (!fuse_rope) HIP_OK(launch_pf_rope_kv(r, T, s));
+      if (last_kv) break;
+      PfAttnArgs at{};
+      at.qkv = b.qkv;
+      at.ld = ldqkv;
+      at.out = b.att;
+      at.ldo = qdim;
+      at.heads = lc.heads;
+      at.kv_heads = lc.kv_heads;
+      at.hd = c.hd;
+      at.window = c.layer[i].window;
+      at.kv16 = r.kv16;
+      at.scale = c.scale;
+      at.kv = r.kv;
+      bool planes = false;  // the attention wrote the o-projection's operand planes
+      if (walk) {
+        at.oh = b.h;
+        at.ol = b.l;
+        at.oscale = b.xscale;
+        at.okpad = gemm_kpad(qdim);
+        HIP_OK(launch_bd_attn(at, T, b.part, P, s, &planes, fuse_rope ? &r : nullptr));
+      } else {
+        HIP_OK(launch_pf_attn(at, T, s));
+      }
+      if (!planes) split(b.att, qdim, qdim, nullptr, T, PartSum{}, nullptr);
+      po = gemm(L.o, T, 0, P);
     }
-    r.qkv = b.qkv;
-    r.ld = ldqkv;
-    r.hd = c.hd;
-    r.heads = lc.heads;
-    r.kv_heads = lc.kv_heads;
-    r.interleaved = c.interleaved ? 1 : 0;
-    r.kv16 = e->kv_elem == 2 ? 1 : 0;
-    r.qn_w = c.qk_norm ? L.q_norm : nullptr;
-    r.kn_w = c.qk_norm ? L.k_norm : nullptr;
-    r.eps = c.qk_eps;
-    r.rope_inv = rope_table(e, c.layer[i].theta, c.hd);
-    r.kv = kv_addr(i);
-    const bool last_kv = i == c.layers - 1 && !logits;  // only the last layer's K/V are needed from it
-    // decode batches: the page-walking attention (one workgroup per (kv head,
-    // row) walking all of its pages also does the rotary/K-V write)
-    const bool walk = pl.row_seq && c.hd >= 64 && lc.heads / lc.kv_heads <= 8 && kvs.max_pages <= 64;
-    const bool fuse_rope = walk && !last_kv && bd_attn_segments(T, lc.kv_heads, kvs.max_pages) == 1;
-    if (!fuse_rope) HIP_OK(launch_pf_rope_kv(r, T, s));
-    if (last_kv) break;
-    PfAttnArgs at{};
-    at.qkv = b.qkv;
-    at.ld = ldqkv;
-    at.out = b.att;
-    at.ldo = qdim;
-    at.heads = lc.heads;
-    at.kv_heads = lc.kv_heads;
-    at.hd = c.hd;
-    at.window = c.layer[i].window;
-    at.kv16 = r.kv16;
-    at.scale = c.scale;
-    at.kv = r.kv;
-    bool planes = false;  // the attention wrote the o-projection's operand planes
-    if (walk) {
-      at.oh = b.h;
-      at.ol = b.l;
-      at.oscale = b.xscale;
-      at.okpad = gemm_kpad(qdim);
-      HIP_OK(launch_bd_attn(at, T, b.part, P, s, &planes, fuse_rope ? &r : nullptr));
-    } else {
-      HIP_OK(launch_pf_attn(at, T, s));
-    }
-    if (!planes) split(b.att, qdim, qdim, nullptr, T, PartSum{}, nullptr);
-    const PartSum po = gemm(L.o, T, 0, P);
     // x += o (Gemma-3: x = clamp(x + RMSNorm(o) * post_norm)), then the ffn norm
-    split(b.x, H, H, c.gemma ? L.pre_ffn_norm : L.post_norm, T, po, c.gemma ? L.post_norm : nullptr);
+    split(b.x, H, H, c.gemma ? L.pre_ffn_norm : L.post_norm, T, po, c.gemma ? L.post_norm : nullptr, L.o_b,
+          L.post_norm_b);
     PfGluArgs gl{};
     PartSum gu{};
-    if (gemm_fused({&L.gate, &L.up}, T, &gu)) {
+    if (c.gpt) {
+      gl.pu = gemm(L.up, T, 0, P);
+      gl.bias = L.up_b;
+    } else if (gemm_fused({&L.gate, &L.up}, T, &gu)) {
       gl.pg = columns(gu, 0, F);
       gl.pu = columns(gu, F, F);
     } else {
       gl.pg = gemm(L.gate, T, 0, P / 2);
       gl.pu = gemm(L.up, T, P / 2, P - P / 2);
     }
-    gl.act = b.act;
     gl.k = F;
     gl.kpad = gemm_kpad(F);
-    gl.gelu = c.gemma ? 1 : 0;
+    gl.act = c.gpt ? PF_GELU_BIAS : c.gemma ? PF_GEGLU : PF_SWIGLU;
     gl.xh = b.h;
     gl.xl = b.l;
     gl.xscale = b.xscale;
     HIP_OK(launch_pf_glu_split(gl, T, s));
     pending = gemm(L.down, T, 0, P);
     pending_w = c.gemma ? L.post_ffn_norm : nullptr;
+    pending_b = L.down_b;
   }
   if (logits) {
     PartSum add = pending;
     if (add.p) add.p += (int64_t)lr0 * add.ld;  // rows [lr0, lr0 + nlr) of the result
-    split(b.x + (size_t)lr0 * H, H, H, e->final_norm, nlr, add, pending_w);
+    split(b.x + (size_t)lr0 * H, H, H, e->final_norm, nlr, add, pending_w, pending_b, e->final_norm_b);
     GemmArgs g{};
     g.w = e->lm_head.q;
     g.xh = b.h;

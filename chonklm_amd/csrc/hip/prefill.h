@@ -65,12 +65,53 @@ struct PfSplitArgs {
   // add_w (the Gemma-3 sandwich) x = clamp(x + RMSNorm(add) * add_w, +-65000)
   PartSum add;
   const float* add_w;
+  float add_scale;        // x += add_scale * add when not 0 (granitehybrid)
+  // GPT-2: x = sanitize(x + (add + add_bias)), and w / norm_b are a LayerNorm
+  const float *add_bias, *norm_b;
 };
+
+enum PfAct : int32_t { PF_SWIGLU = 0, PF_GEGLU = 1, PF_GELU_BIAS = 2 };
 
 struct PfGluArgs {
   PartSum pg, pu;         // gate and up rows [rows][k] (deferred GEMM results)
-  float* act;             // [rows][k]
-  int32_t k, kpad, gelu;
+  const float* bias;      // PF_GELU_BIAS: gelu(up + bias); pg is not read
+  int32_t k, kpad, act;
+  _Float16 *xh, *xl;
+  float* xscale;
+};
+
+// lfm2 short convolution over the rows of a pass, in_proj rows B | C | x of k
+// channels each, as operand planes; s1 / s2 are B * x two and one positions
+// before row 0, and after launch_pf_conv_state those before the next pass.
+struct PfConvArgs {
+  PartSum p;
+  int32_t k, kpad;
+  const float* w;         // [k][3] taps
+  float *s1, *s2;
+  _Float16 *xh, *xl;
+  float* xscale;
+};
+
+// granitehybrid Mamba2 layer over the rows of a pass; in_proj rows z | xBC | dt.
+struct PfMambaArgs {
+  PartSum p;              // in_proj rows (inner + conv + heads columns)
+  int32_t rows, inner, conv, heads, p0;
+  const float *conv_w, *conv_b, *dt_bias, *a_neg, *d;
+  float* conv_state;      // [2][conv][3], indexed by the position's parity
+  float* ssm_state;       // [heads][32][128]
+  float* xbc;             // [rows][pf_mamba_ld]: silu(conv(xBC)) | dt | decay
+  float* y;               // [rows][inner] scan output
+};
+
+// floats per row of PfMambaArgs.xbc (16-byte rows for the scan's loads)
+constexpr int pf_mamba_ld(int conv, int heads) { return (conv + 2 * heads + 3) / 4 * 4; }
+
+// y * silu(z), RMSNorm, operand planes (the Mamba2 gated norm)
+struct PfGateArgs {
+  PartSum z;
+  const float *y, *w;
+  int32_t k, kpad;
+  float eps;
   _Float16 *xh, *xl;
   float* xscale;
 };
@@ -80,6 +121,7 @@ struct PfRopeArgs {
   PartSum pq, pk, pv;
   int32_t ld, hd, heads, kv_heads, interleaved, kv16;
   const float *qn_w, *kn_w;  // per-head RMSNorm weights (null: none)
+  const float* bias;      // [q | k | v] added to the projections first (null: none)
   float eps;
   const float* rope_inv;  // [hd/2]
   KvAddr kv;
@@ -102,6 +144,10 @@ struct PfAttnArgs {
   int32_t okpad;
 };
 
+// Widest row the per-row glue kernels hold in registers (eight elements of
+// each of 1024 threads).
+constexpr int kPfRowMax = 8192;
+
 // K padded for the GEMM's activation planes.
 constexpr int gemm_kpad(int k) { return (k + 127) / 128 * 128; }
 
@@ -115,8 +161,14 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);
 // reduction is launched; *out describes the partials for the consumer.
 hipError_t launch_gemm_deferred(const GemmArgs& a, float* region, int64_t region_cap, PartSum* out, hipStream_t s);
 hipError_t launch_pf_split(const PfSplitArgs& a, int rows, hipStream_t s);
-hipError_t launch_pf_embed(const QMat& embed, const int32_t* tok, float scale, int k, float* x, int rows,
-                           hipStream_t s);
+// Embedding rows times scale, plus (pos != null, GPT-2) the rows of the
+// position table from position p0 on.
+hipError_t launch_pf_embed(const QMat& embed, const int32_t* tok, float scale, const float* pos, int p0, int k,
+                           float* x, int rows, hipStream_t s);
+hipError_t launch_pf_conv(const PfConvArgs& a, int rows, hipStream_t s);
+hipError_t launch_pf_conv_state(const PfConvArgs& a, int rows, hipStream_t s);
+hipError_t launch_pf_mamba(const PfMambaArgs& a, hipStream_t s);
+hipError_t launch_pf_gate(const PfGateArgs& a, int rows, hipStream_t s);
 hipError_t launch_pf_norm_add(const float* d, const float* w, float eps, int k, float* x, int rows, hipStream_t s);
 hipError_t launch_pf_glu_split(const PfGluArgs& a, int rows, hipStream_t s);
 hipError_t launch_pf_rope_kv(const PfRopeArgs& a, int rows, hipStream_t s);

@@ -104,22 +104,28 @@ __device__ __forceinline__ void part_gather(const PartSum& P, int t, const int (
   part_finish<N>(P, t, j, w, v);
 }
 
-// Row t of a deferred result, elements j0 + S * e for e < 4 (zero past n).
-template <int S = kWg>
-__device__ __forceinline__ void part_row4(const PartSum& P, int t, int j0, float (&v)[4]) {
-  int j[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) j[e] = min(j0 + S * e, P.n - 1);
-  part_gather<4>(P, t, j, v);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = j0 + S * e < P.n ? v[e] : 0.f;
-}
-
 // The per-row glue kernels run one workgroup of kRowT threads per token row
 // (a batch of decode rows is a few dozen workgroups; wide ones keep each
 // row's deferred partial sums to one or two rounds of loads).
 constexpr int kRowT = 1024;
 constexpr int kRowW = kRowT / 64;
+
+// Row t of a deferred result, elements j0 + kRowT * e for e < E (zero past n),
+// four at a time.
+template <int E>
+__device__ __forceinline__ void part_row(const PartSum& P, int t, int j0, float (&v)[E]) {
+  static_assert(E % 4 == 0, "groups of four");
+#pragma unroll
+  for (int g = 0; g < E; g += 4) {
+    int j[4];
+    float w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) j[e] = min(j0 + kRowT * (g + e), P.n - 1);
+    part_gather<4>(P, t, j, w);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[g + e] = j0 + kRowT * (g + e) < P.n ? w[e] : 0.f;
+  }
+}
 
 __device__ __forceinline__ float rowt_sum(float v, float* red) {
   v = wave_sum(v);
@@ -144,80 +150,120 @@ __device__ __forceinline__ float rowt_max(float v, float* red) {
 
 // ---- operand split ----------------------------------------------------------------
 
-// One workgroup per token row: optional RMSNorm (x * inv) * w with the
-// reference's fp32 operation order, then the row scaled by a power of two so
-// that |x| < 2^14 and split into fp16 hi + lo planes (zero-padded to kpad).
-// mode 0: plain; 1: RMSNorm with w.
-__global__ __launch_bounds__(kRowT) void k_pf_split(PfSplitArgs a) {
-  warm_kernarg<(int)(sizeof(PfSplitArgs))>();  // (dependent argument rounds hit the scalar cache)
-  // the row lives in registers: element tid + kRowT * e of this thread is v[e]
-  // (rows of at most 4 * kRowT elements; the launcher checks)
-  __shared__ float red[kRowW];
-  const int t = blockIdx.x, tid = threadIdx.x;
-  float* xw = const_cast<float*>(a.x + (size_t)t * a.ldx);
-  float v[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = xw[min(tid + kRowT * e, a.k - 1)];  // unconditional (no branch)
-#pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = tid + kRowT * e < a.k ? v[e] : 0.f;
-  if (a.add.p) {
-    float d[4];
-    part_row4<kRowT>(a.add, t, tid, d);
-    if (a.add_w) {
-      // the branch output goes through RMSNorm first (the Gemma-3 sandwich)
-      float ss = 0.f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ss += d[e] * d[e];
-      ss = rowt_sum(ss, red);
-      const float inv = 1.0f / sqrtf(ss / (float)a.k + a.eps);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = tid + kRowT * e;
-        if (i < a.k) v[e] = fminf(fmaxf(__fadd_rn(v[e], __fmul_rn(__fmul_rn(d[e], inv), a.add_w[i])), -65000.0f), 65000.0f);
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = __fadd_rn(v[e], d[e]);
-    }
-    // the updated residual row
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int i = tid + kRowT * e;
-      if (i < a.k) xw[i] = v[e];
-    }
-  }
-  if (a.w) {
-    float ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ss += v[e] * v[e];
-    ss = rowt_sum(ss, red);
-    const float inv = 1.0f / sqrtf(ss / (float)a.k + a.eps);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int i = tid + kRowT * e;
-      if (i < a.k) v[e] = __fmul_rn(__fmul_rn(v[e], inv), a.w[i]);
-    }
-  }
+// The row v (element threadIdx.x + kRowT * e of thread x is v[e], zero past the
+// row's end) scaled by a power of two so that |x| < 2^14 and split into fp16
+// hi + lo planes of kpad elements.
+template <int E>
+__device__ __forceinline__ void row_planes(const float (&v)[E], int t, int kpad, _Float16* xh, _Float16* xl,
+                                           float* xscale, float* red) {
+  const int tid = threadIdx.x;
   float mx = 0.f;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(v[e]));
+  for (int e = 0; e < E; ++e) mx = fmaxf(mx, fabsf(v[e]));
   mx = rowt_max(mx, red);
   int ex = 0;
   (void)frexpf(mx, &ex);  // mx < 2^ex
   const int rs = max(min(14 - ex, 60), -60);
-  _Float16* xh = a.xh + (size_t)t * a.kpad;
-  _Float16* xl = a.xl + (size_t)t * a.kpad;
+  xh += (size_t)t * kpad;
+  xl += (size_t)t * kpad;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
+  for (int e = 0; e < E; ++e) {
     const int i = tid + kRowT * e;
-    if (i < a.kpad) {
-      const float sv = ldexpf(v[e], rs);  // zero past k
+    if (i < kpad) {
+      const float sv = ldexpf(v[e], rs);  // zero past the row's end
       const _Float16 h = (_Float16)sv;
       xh[i] = h;
       xl[i] = (_Float16)(sv - (float)h);
     }
   }
-  if (tid == 0) a.xscale[t] = __builtin_isfinite(mx) ? ldexpf(1.0f, -rs) : __int_as_float(0x7fc00000);
+  if (tid == 0) xscale[t] = __builtin_isfinite(mx) ? ldexpf(1.0f, -rs) : __int_as_float(0x7fc00000);
+}
+
+// x := (x * inv) * w with the reference's fp32 operation order (RMSNorm)
+template <int E>
+__device__ __forceinline__ void row_rmsnorm(float (&v)[E], const float* w, int k, float eps, float* red) {
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < E; ++e) ss += v[e] * v[e];
+  ss = rowt_sum(ss, red);
+  const float inv = 1.0f / sqrtf(ss / (float)k + eps);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = threadIdx.x + kRowT * e;
+    if (i < k) v[e] = __fmul_rn(__fmul_rn(v[e], inv), w[i]);
+  }
+}
+
+// One workgroup per token row: the pending residual update, an optional
+// RMSNorm (GPT: LayerNorm), then the operand planes. The row lives in
+// registers: E = 4 elements per thread serve rows of up to 4096, E = 8 (the
+// LFM2 and OpenELM feed-forward widths) up to kPfRowMax.
+template <int E, bool GPT>
+__global__ __launch_bounds__(kRowT) void k_pf_split(PfSplitArgs a) {
+  warm_kernarg<(int)(sizeof(PfSplitArgs))>();  // (dependent argument rounds hit the scalar cache)
+  __shared__ float red[kRowW];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  float* xw = const_cast<float*>(a.x + (size_t)t * a.ldx);
+  float v[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = xw[min(tid + kRowT * e, a.k - 1)];  // unconditional (no branch)
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = tid + kRowT * e < a.k ? v[e] : 0.f;
+  if (a.add.p) {
+    float d[E];
+    part_row<E>(a.add, t, tid, d);
+    if (GPT) {
+      // bias, residual add, SANITIZE (gpt-wgsl-runtime.ts:1708-1746)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int i = tid + kRowT * e;
+        if (i < a.k) {
+          const float y = __fadd_rn(v[e], __fadd_rn(d[e], a.add_bias[i]));
+          v[e] = y != y ? 0.0f : fminf(fmaxf(y, -10000.0f), 10000.0f);
+        }
+      }
+    } else if (a.add_w) {
+      // the branch output goes through RMSNorm first (the Gemma-3 sandwich)
+      row_rmsnorm<E>(d, a.add_w, a.k, a.eps, red);
+#pragma unroll
+      for (int e = 0; e < E; ++e)
+        if (tid + kRowT * e < a.k) v[e] = fminf(fmaxf(__fadd_rn(v[e], d[e]), -65000.0f), 65000.0f);
+    } else {
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[e] = __fadd_rn(v[e], a.add_scale != 0.f ? __fmul_rn(d[e], a.add_scale) : d[e]);
+    }
+    // the updated residual row
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = tid + kRowT * e;
+      if (i < a.k) xw[i] = v[e];
+    }
+  }
+  if (GPT) {
+    if (a.w) {
+      // LAYER_NORM_WGSL (gpt-wgsl-runtime.ts:1658-1706): mean and E[x^2] in one
+      // pass, variance max(E[x^2] - mean^2, 0), ((x - mean) * inv_std) * w + b
+      float sm = 0.f, sq = 0.f;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        sm += v[e];
+        sq += v[e] * v[e];
+      }
+      sm = rowt_sum(sm, red);
+      sq = rowt_sum(sq, red);
+      const float mean = sm / (float)a.k;
+      const float var = fmaxf(__fsub_rn(sq / (float)a.k, __fmul_rn(mean, mean)), 0.0f);
+      const float inv = 1.0f / sqrtf(var + a.eps);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int i = tid + kRowT * e;
+        if (i < a.k) v[e] = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[e], mean), inv), a.w[i]), a.norm_b[i]);
+      }
+    }
+  } else if (a.w) {
+    row_rmsnorm<E>(v, a.w, a.k, a.eps, red);
+  }
+  row_planes<E>(v, t, a.kpad, a.xh, a.xl, a.xscale, red);
 }
 
 // ---- dequant-fused GEMM ----------------------------------------------------------
@@ -874,8 +920,10 @@ __global__ __launch_bounds__(kWg) void k_gemm_reduce(GemmArgs a) {
 
 // ---- per-token glue ---------------------------------------------------------------
 
-// Embedding rows of the prompt tokens times the embedding scale.
-__global__ __launch_bounds__(kWg) void k_pf_embed(QMat embed, const int32_t* tok, float scale, int k, float* x) {
+// Embedding rows of the prompt tokens times the embedding scale, plus (pos !=
+// null) row p0 + t of the learned position table.
+__global__ __launch_bounds__(kWg) void k_pf_embed(QMat embed, const int32_t* tok, float scale, const float* pos, int p0,
+                                                  int k, float* x) {
   const int t = blockIdx.x;
   const int id = tok[t];
   with_type(embed.type, [&]<int TE>() {
@@ -884,7 +932,11 @@ __global__ __launch_bounds__(kWg) void k_pf_embed(QMat embed, const int32_t* tok
       float v[32];
       dequant_unit<TE>(f, u, v);
 #pragma unroll
-      for (int e = 0; e < 32; ++e) x[(size_t)t * k + unit_col<TE>(u, e)] = __fmul_rn(v[e], scale);
+      for (int e = 0; e < 32; ++e) {
+        const int i = unit_col<TE>(u, e);
+        const float y = __fmul_rn(v[e], scale);
+        x[(size_t)t * k + i] = pos ? __fadd_rn(y, pos[(size_t)(p0 + t) * k + i]) : y;
+      }
     }
   });
 }
@@ -906,45 +958,267 @@ __global__ __launch_bounds__(kWg) void k_pf_norm_add(const float* d, const float
   }
 }
 
-// act = silu(g) * u or gelu_tanh(g) * u per element, then the split of the row
-// into fp16 planes (one workgroup per token row).
+// silu(g) * u, gelu_tanh(g) * u or (GPT-2) gelu_tanh(u + bias) per element, then
+// the operand planes (one workgroup per token row; E as for k_pf_split).
+template <int E>
 __global__ __launch_bounds__(kRowT) void k_pf_glu_split(PfGluArgs a) {
   warm_kernarg<(int)(sizeof(PfGluArgs))>();  // (dependent argument rounds hit the scalar cache)
-  // element tid + kRowT * e of the row is v[e] (at most 4 * kRowT elements)
   __shared__ float red[kRowW];
   const int t = blockIdx.x, tid = threadIdx.x;
-  float* y = a.act + (size_t)t * a.k;
-  float gv[4], uv[4], v[4];
-  part_row4<kRowT>(a.pg, t, tid, gv);
-  part_row4<kRowT>(a.pu, t, tid, uv);
-  float mx = 0.f;
+  float gv[E], uv[E], v[E];
+  if (a.act != PF_GELU_BIAS) {
+    part_row<E>(a.pg, t, tid, gv);
+  } else {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int i = tid + kRowT * e;
+    for (int e = 0; e < E; ++e) gv[e] = a.bias[min(tid + kRowT * e, a.k - 1)];
+  }
+  part_row<E>(a.pu, t, tid, uv);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
     v[e] = 0.f;
-    if (i < a.k) {
-      v[e] = a.gelu ? __fmul_rn(gelu_tanh(gv[e]), uv[e]) : silu_mul(gv[e], uv[e]);
-      y[i] = v[e];
-      mx = fmaxf(mx, fabsf(v[e]));
-    }
+    if (tid + kRowT * e < a.k)
+      v[e] = a.act == PF_SWIGLU  ? silu_mul(gv[e], uv[e])
+             : a.act == PF_GEGLU ? __fmul_rn(gelu_tanh(gv[e]), uv[e])
+                                 : gelu_tanh(__fadd_rn(uv[e], gv[e]));
   }
-  mx = rowt_max(mx, red);
-  int ex = 0;
-  (void)frexpf(mx, &ex);
-  const int rs = max(min(14 - ex, 60), -60);
-  _Float16* xh = a.xh + (size_t)t * a.kpad;
-  _Float16* xl = a.xl + (size_t)t * a.kpad;
+  row_planes<E>(v, t, a.kpad, a.xh, a.xl, a.xscale, red);
+}
+
+// ---- lfm2 short convolution ---------------------------------------------------------
+
+// C * (bx[t-2] w0 + bx[t-1] w1 + bx[t] w2) of every channel (CONV_BLOCK_WGSL,
+// lfm-wgsl-runtime.ts:1641-1672, each product and sum rounded as the decode
+// prologue does), bx = B * x of the in_proj rows, the two rows before the pass
+// from the state; then the operand planes. One workgroup per token row.
+template <int E>
+__global__ __launch_bounds__(kRowT) void k_pf_conv(PfConvArgs a) {
+  warm_kernarg<(int)(sizeof(PfConvArgs))>();
+  __shared__ float red[kRowW];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  float v[E];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int i = tid + kRowT * e;
-    if (i < a.kpad) {
-      const float sv = ldexpf(v[e], rs);
-      const _Float16 h = (_Float16)sv;
-      xh[i] = h;
-      xl[i] = (_Float16)(sv - (float)h);
+  for (int g = 0; g < E; g += 4) {
+    int i[4], j[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) i[e] = min(tid + kRowT * (g + e), a.k - 1);
+    auto part = [&](int row, int piece, float (&w)[4]) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) j[e] = piece * a.k + i[e];
+      part_gather<4>(a.p, row, j, w);
+    };
+    float b[4], x[4], c[4], p1[4], p2[4];
+    part(max(t - 2, 0), 0, b);
+    part(max(t - 2, 0), 2, x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p1[e] = __fmul_rn(b[e], x[e]);
+    part(max(t - 1, 0), 0, b);
+    part(max(t - 1, 0), 2, x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p2[e] = __fmul_rn(b[e], x[e]);
+    part(t, 0, b);
+    part(t, 2, x);
+    part(t, 1, c);
+    if (t < 2) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) p1[e] = t == 0 ? a.s1[i[e]] : a.s2[i[e]];
+      if (t == 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p2[e] = a.s2[i[e]];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float* w = a.w + 3 * (size_t)i[e];
+      const float y = __fadd_rn(__fadd_rn(__fmul_rn(p1[e], w[0]), __fmul_rn(p2[e], w[1])),
+                                __fmul_rn(__fmul_rn(b[e], x[e]), w[2]));
+      v[g + e] = tid + kRowT * (g + e) < a.k ? __fmul_rn(c[e], y) : 0.f;
     }
   }
-  if (tid == 0) a.xscale[t] = __builtin_isfinite(mx) ? ldexpf(1.0f, -rs) : __int_as_float(0x7fc00000);
+  row_planes<E>(v, t, a.kpad, a.xh, a.xl, a.xscale, red);
+}
+
+// s1, s2 = bx of the pass's last two rows (a launch of its own: k_pf_conv's
+// rows 0 and 1 read the old state). A thread reads its channel before it writes.
+__global__ __launch_bounds__(kWg) void k_pf_conv_state(PfConvArgs a, int rows) {
+  const int i = (int)blockIdx.x * kWg + (int)threadIdx.x;
+  if (i >= a.k) return;
+  const int j[2] = {i, 2 * a.k + i};
+  float w[2];
+  part_gather<2>(a.p, rows - 1, j, w);
+  const float cur = __fmul_rn(w[0], w[1]);
+  float prev = a.s2[i];
+  if (rows >= 2) {
+    part_gather<2>(a.p, rows - 2, j, w);
+    prev = __fmul_rn(w[0], w[1]);
+  }
+  a.s1[i] = prev;
+  a.s2[i] = cur;
+}
+
+// ---- granitehybrid Mamba2 ------------------------------------------------------------
+
+constexpr int kMbConvRows = 4;   // token rows per thread of k_pf_mamba_conv
+constexpr int kMbStates = 128;   // states per channel
+constexpr int kMbHd = 32;        // channels per head
+constexpr int kMbCh = 8;         // channels per workgroup of the scan
+constexpr int kMbSteps = 32;     // token rows staged in LDS at once
+
+// MAMBA_CONV_WGSL (granite-wgsl-runtime.ts:1476-1520) of every row: channel c of
+// xBC is silu(((p1 w0 + p2 w1) + p3 w2) + x w3 + bias) over its last four
+// inputs, those before row 0 from the window copy of p0's parity; and per head
+// dt = softplus(dt_raw + bias) and decay = exp(dt A) as MAMBA_SSM_WGSL forms
+// them. A thread walks kMbConvRows rows of one channel.
+__global__ __launch_bounds__(kWg) void k_pf_mamba_conv(PfMambaArgs a) {
+  warm_kernarg<(int)(sizeof(PfMambaArgs))>();
+  const int c = (int)blockIdx.x * kWg + (int)threadIdx.x, t0 = (int)blockIdx.y * kMbConvRows;
+  const int nt = min(kMbConvRows, a.rows - t0);
+  if (c >= a.conv + a.heads) return;
+  const int ld = pf_mamba_ld(a.conv, a.heads);
+  const int j[1] = {a.inner + c};
+  float x[kMbConvRows + 3];
+#pragma unroll
+  for (int r = 0; r < kMbConvRows + 3; ++r) {
+    float w[1];
+    part_gather<1>(a.p, min(max(t0 + r - 3, 0), a.rows - 1), j, w);
+    x[r] = w[0];
+  }
+  if (c >= a.conv) {
+    const int n = c - a.conv;
+    const float bias = a.dt_bias[n], an = a.a_neg[n];
+    for (int r = 0; r < nt; ++r) {
+      const float s = __fadd_rn(x[r + 3], bias);
+      const float dt = s > 20.0f ? __fadd_rn(s, logf(__fadd_rn(1.0f, expf(-s)))) : logf(__fadd_rn(1.0f, expf(s)));
+      float* o = a.xbc + (size_t)(t0 + r) * ld + a.conv;
+      o[n] = dt;
+      o[a.heads + n] = expf(__fmul_rn(dt, an));
+    }
+    return;
+  }
+  if (t0 == 0) {
+    const float* cs = a.conv_state + ((size_t)(a.p0 & 1) * a.conv + c) * 3;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) x[r] = cs[r];
+  }
+  const float4 w = reinterpret_cast<const float4*>(a.conv_w)[c];
+  const float bias = a.conv_b[c];
+#pragma unroll
+  for (int r = 0; r < kMbConvRows; ++r) {
+    if (r >= nt) break;
+    const float y = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(__fmul_rn(x[r], w.x), __fmul_rn(x[r + 1], w.y)),
+                                                  __fmul_rn(x[r + 2], w.z)),
+                                        __fmul_rn(x[r + 3], w.w)),
+                              bias);
+    a.xbc[(size_t)(t0 + r) * ld + c] = __fdiv_rn(y, __fadd_rn(1.0f, expf(-y)));
+  }
+}
+
+// MAMBA_SSM_WGSL's recurrence h = h decay + (dt x) B, y = C h + D x over the rows
+// of the pass. The chain over the rows is serial per state and its work small
+// (two multiplies and two fmas per state and row), so the split is over states:
+// a workgroup owns 8 channels of one head, 32 lanes per channel with 4 states
+// each in registers, and walks the rows with B, C (shared by every channel),
+// x dt, decay and x staged in LDS 32 rows at a time; the next rows' loads are in
+// flight while the staged ones are walked. Workgroups of one head and channel
+// group also leave the convolution window of the next pass (k_pf_mamba_conv has
+// read the old one; a thread reads its channel's window before it writes it).
+__global__ __launch_bounds__(kWg) void k_pf_mamba_scan(PfMambaArgs a) {
+  warm_kernarg<(int)(sizeof(PfMambaArgs))>();
+  __shared__ __align__(16) float sbc[kMbSteps][2 * kMbStates];
+  __shared__ float sx[kMbSteps][kMbCh], sxd[kMbSteps][kMbCh], sdec[kMbSteps], sy[kMbSteps][kMbCh];
+  const int n = (int)blockIdx.x, c0 = (int)blockIdx.y * kMbCh, tid = (int)threadIdx.x;
+  const int h = tid >> 5, l = tid & 31;
+  const int ld = pf_mamba_ld(a.conv, a.heads);
+  const int nx = n * kMbHd + c0;  // the workgroup's first channel
+  float4* sp = reinterpret_cast<float4*>(a.ssm_state + (size_t)(nx + h) * kMbStates) + l;
+  float4 s = *sp;
+  const float dsk = a.d[n];
+  // the next window: entry r is the input of row rows - 3 + r, or the old window's
+  auto window = [&](int c) {
+    const float* co = a.conv_state + ((size_t)(a.p0 & 1) * a.conv + c) * 3;
+    float* cn = a.conv_state + ((size_t)((a.p0 + a.rows) & 1) * a.conv + c) * 3;
+    const int j[1] = {a.inner + c};
+    float v[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      const int t = a.rows - 3 + r;
+      float w[1];
+      part_gather<1>(a.p, max(t, 0), j, w);
+      v[r] = t >= 0 ? w[0] : co[min(3 + t, 2)];
+    }
+#pragma unroll
+    for (int r = 0; r < 3; ++r) cn[r] = v[r];
+  };
+  if (tid < kMbCh) window(nx + tid);
+  if (n == 0 && c0 == 0) window(a.inner + tid);  // B and C: kWg == 2 * kMbStates channels
+
+  // staging roles: thread moves float4 (tid % 64) of rows tid / 64 + 4 i of
+  // B | C, and (row tid / 8, channel tid % 8) of x, dt and decay
+  float4 rb[kMbSteps / 4];
+  float rx, rdt, rdec;
+  auto fetch = [&](int t0) {
+#pragma unroll
+    for (int i = 0; i < kMbSteps / 4; ++i) {
+      const int t = min(t0 + (tid >> 6) + 4 * i, a.rows - 1);
+      rb[i] = *reinterpret_cast<const float4*>(a.xbc + (size_t)t * ld + a.inner + 4 * (tid & 63));
+    }
+    const float* r = a.xbc + (size_t)min(t0 + (tid >> 3), a.rows - 1) * ld;
+    rx = r[nx + (tid & 7)];
+    rdt = r[a.conv + n];
+    rdec = r[a.conv + a.heads + n];
+  };
+  fetch(0);
+  for (int t0 = 0; t0 < a.rows; t0 += kMbSteps) {
+    __syncthreads();  // the previous rows are consumed, their y written out
+#pragma unroll
+    for (int i = 0; i < kMbSteps / 4; ++i)
+      *reinterpret_cast<float4*>(&sbc[(tid >> 6) + 4 * i][4 * (tid & 63)]) = rb[i];
+    sx[tid >> 3][tid & 7] = rx;
+    // (steps past the last row leave the state as it is)
+    const bool live = t0 + (tid >> 3) < a.rows;
+    sxd[tid >> 3][tid & 7] = live ? __fmul_rn(rdt, rx) : 0.f;
+    if ((tid & 7) == 0) sdec[tid >> 3] = live ? rdec : 1.f;
+    __syncthreads();
+    fetch(min(t0 + kMbSteps, a.rows - 1));
+    const int nt = min(kMbSteps, a.rows - t0);
+    for (int tb = 0; tb < nt; tb += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int t = tb + u;
+        const float4 B = *reinterpret_cast<const float4*>(&sbc[t][4 * l]);
+        const float4 C = *reinterpret_cast<const float4*>(&sbc[t][kMbStates + 4 * l]);
+        const float dx = sxd[t][h], dec = sdec[t];
+        s.x = fmaf(s.x, dec, dx * B.x);
+        s.y = fmaf(s.y, dec, dx * B.y);
+        s.z = fmaf(s.z, dec, dx * B.z);
+        s.w = fmaf(s.w, dec, dx * B.w);
+        float acc = fmaf(s.x, C.x, s.y * C.y) + fmaf(s.z, C.z, s.w * C.w);
+        acc = group_sum<32>(acc);
+        if (l == 0) sy[t][h] = __fadd_rn(acc, __fmul_rn(dsk, sx[t][h]));
+      }
+    }
+    __syncthreads();
+    const int t = tid >> 3;
+    if (t < nt) a.y[(size_t)(t0 + t) * a.inner + nx + (tid & 7)] = sy[t][tid & 7];
+  }
+  *sp = s;
+}
+
+// MAMBA_GATE_NORM_WGSL (granite-wgsl-runtime.ts:1590-1606) of every row, then
+// the operand planes of out_proj.
+template <int E>
+__global__ __launch_bounds__(kRowT) void k_pf_gate(PfGateArgs a) {
+  warm_kernarg<(int)(sizeof(PfGateArgs))>();
+  __shared__ float red[kRowW];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  float v[E], z[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = a.y[(size_t)t * a.k + min(tid + kRowT * e, a.k - 1)];
+  part_row<E>(a.z, t, tid, z);
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    v[e] = tid + kRowT * e < a.k ? __fmul_rn(v[e], __fdiv_rn(z[e], __fadd_rn(1.0f, expf(-z[e])))) : 0.f;
+  row_rmsnorm<E>(v, a.w, a.k, a.eps, red);
+  row_planes<E>(v, t, a.kpad, a.xh, a.xl, a.xscale, red);
 }
 
 __device__ __forceinline__ int row_pos(const KvAddr& k, int t) { return k.row_pos ? k.row_pos[t] : k.p0 + t; }
@@ -1007,6 +1281,13 @@ __global__ __launch_bounds__(kWg) void k_pf_rope_kv(PfRopeArgs a) {
       x1[j] = row[col + ib[j]];
     }
   }
+  if (a.bias) {
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      x0[j] = __fadd_rn(x0[j], a.bias[col + ia[j]]);
+      x1[j] = __fadd_rn(x1[j], a.bias[col + ib[j]]);
+    }
+  }
   float r = 1.0f;
   if (a.qn_w) {
     float ss = 0.f;
@@ -1064,6 +1345,7 @@ __global__ __launch_bounds__(kWg) void k_pf_rope_kv(PfRopeArgs a) {
     for (int i = 0; i < 4; ++i) {
       const int d = lane + 64 * i;
       if (d >= hd) continue;
+      if (a.bias) vv[i] = __fadd_rn(vv[i], a.bias[vcol + d]);
       if (a.kv16)
         ((__half*)a.kv.vc)[base + d] = __float2half_rn(vv[i]);
       else
@@ -2000,24 +2282,60 @@ hipError_t init_gemm_attributes() {
   return hipSuccess;
 }
 
+// the instance of a per-row kernel that holds a row of kpad elements
+#define CHONK_ROW_CASE(kpad, ...)                       \
+  do {                                                  \
+    if ((kpad) > kPfRowMax) return hipErrorInvalidValue; \
+    if ((kpad) <= 4 * kRowT) {                          \
+      constexpr int E = 4;                              \
+      __VA_ARGS__;                                      \
+    } else {                                            \
+      constexpr int E = 8;                              \
+      __VA_ARGS__;                                      \
+    }                                                   \
+    return hipGetLastError();                           \
+  } while (0)
+
 hipError_t launch_pf_split(const PfSplitArgs& a, int rows, hipStream_t s) {
-  if (a.kpad > 4 * kRowT) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_pf_split, dim3(rows), dim3(kRowT), 0, s, a);
+  if (a.norm_b || a.add_bias) {
+    if ((a.w && !a.norm_b) || (a.add.p && !a.add_bias)) return hipErrorInvalidValue;
+    CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_split<E, true>), dim3(rows), dim3(kRowT), 0, s, a));
+  }
+  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_split<E, false>), dim3(rows), dim3(kRowT), 0, s, a));
+}
+hipError_t launch_pf_embed(const QMat& embed, const int32_t* tok, float scale, const float* pos, int p0, int k,
+                           float* x, int rows, hipStream_t s) {
+  hipLaunchKernelGGL(k_pf_embed, dim3(rows), dim3(kWg), 0, s, embed, tok, scale, pos, p0, k, x);
   return hipGetLastError();
 }
-hipError_t launch_pf_embed(const QMat& embed, const int32_t* tok, float scale, int k, float* x, int rows,
-                           hipStream_t s) {
-  hipLaunchKernelGGL(k_pf_embed, dim3(rows), dim3(kWg), 0, s, embed, tok, scale, k, x);
+hipError_t launch_pf_conv(const PfConvArgs& a, int rows, hipStream_t s) {
+  if (rows < 1 || a.p.n < 3 * a.k) return hipErrorInvalidValue;
+  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_conv<E>), dim3(rows), dim3(kRowT), 0, s, a));
+}
+hipError_t launch_pf_conv_state(const PfConvArgs& a, int rows, hipStream_t s) {
+  if (rows < 1 || a.p.n < 3 * a.k) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_pf_conv_state, dim3((a.k + kWg - 1) / kWg), dim3(kWg), 0, s, a, rows);
   return hipGetLastError();
+}
+hipError_t launch_pf_mamba(const PfMambaArgs& a, hipStream_t s) {
+  static_assert(kWg == 2 * kMbStates && kWg == kMbSteps * kMbCh && kWg == 32 * kMbCh, "scan geometry");
+  if (a.rows < 1 || a.inner != a.heads * kMbHd || a.conv != a.inner + 2 * kMbStates ||
+      a.p.n < a.inner + a.conv + a.heads)
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_pf_mamba_conv, dim3((a.conv + a.heads + kWg - 1) / kWg, (a.rows + kMbConvRows - 1) / kMbConvRows),
+                     dim3(kWg), 0, s, a);
+  hipLaunchKernelGGL(k_pf_mamba_scan, dim3(a.heads, kMbHd / kMbCh), dim3(kWg), 0, s, a);
+  return hipGetLastError();
+}
+hipError_t launch_pf_gate(const PfGateArgs& a, int rows, hipStream_t s) {
+  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_gate<E>), dim3(rows), dim3(kRowT), 0, s, a));
 }
 hipError_t launch_pf_norm_add(const float* d, const float* w, float eps, int k, float* x, int rows, hipStream_t s) {
   hipLaunchKernelGGL(k_pf_norm_add, dim3(rows), dim3(kWg), 0, s, d, w, eps, k, x);
   return hipGetLastError();
 }
 hipError_t launch_pf_glu_split(const PfGluArgs& a, int rows, hipStream_t s) {
-  if (a.kpad > 4 * kRowT) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_pf_glu_split, dim3(rows), dim3(kRowT), 0, s, a);
-  return hipGetLastError();
+  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_glu_split<E>), dim3(rows), dim3(kRowT), 0, s, a));
 }
 hipError_t launch_pf_rope_kv(const PfRopeArgs& a, int rows, hipStream_t s) {
   const int nh = a.heads + a.kv_heads;

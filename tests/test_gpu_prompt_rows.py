@@ -50,3 +50,58 @@ def test_streamed_prompt_past_the_context(synth):
         generate_llama_wgsl(loaded, prompt, 4, on_token=lambda info: None)
     assert loaded.engine.position == w.max_context
     loaded.engine.dispose()
+
+
+def _same_state(name, parts, synth, max_context=None):
+    """prefill of each part in turn, against the same tokens one by one: the logits of
+    the next two steps. With the fp32 cache both sides are fp32-class sums of the same
+    values in another order: 3e-7 apart per layer at most, over at most 32 layers and
+    two linear branches each, so 2e-5 bounds them."""
+    w = WORKLOADS[name]
+    md = w.model_def(synth(name), kv_dtype="f32")
+    if max_context:
+        md.max_context = max_context
+    tokens = np.random.default_rng(sum(parts)).integers(0, w.spec.vocab, sum(parts) + 2).tolist()
+    loaded = LOADERS.get(md.runtime, load_llama_wgsl_model)(md)
+    eng = loaded.engine
+    out = []
+    for rows in (True, False):
+        eng.reset()
+        at = 0
+        for n in parts:
+            if rows:
+                eng.prefill(tokens[at:at + n])
+            else:
+                for t in tokens[at:at + n]:
+                    eng.run_token(t, False)
+            at += n
+        assert eng.position == at
+        got = []
+        for t in tokens[at:]:
+            eng.run_token(t, True)
+            got.append(eng.read_logits().copy())
+        out.append(got)
+    eng.dispose()
+    for a, b in zip(*out):
+        assert np.isfinite(a).all()
+        assert rel_err(a, b) <= 2e-5
+
+
+# windows of two (lfm2) and three (granite) earlier inputs, the scan's 32 staged
+# rows, 64-row GEMM tiles; an odd and an even first part (the Mamba2 window's parity)
+@pytest.mark.parametrize("parts", [(1,), (2,), (3,), (1, 1, 2), (3, 32), (4, 33), (64, 1), (65, 64)])
+@pytest.mark.parametrize("name", ["tiny-gpt2", "tiny-lfm2", "tiny-lfm2-q8", "tiny-granite", "tiny-granite-q8"])
+def test_prompt_rows_equal_steps(name, parts, synth):
+    _same_state(name, parts, synth)
+
+
+@pytest.mark.parametrize("name", ["tiny-lfm2", "tiny-granite"])
+def test_prompt_of_two_passes_equals_steps(name, synth):
+    """2051 + 6 rows: the states cross the 2048-row pass boundary and a call's."""
+    _same_state(name, (2051, 6), synth, max_context=2200)
+
+
+@pytest.mark.parametrize("name", ["lfm2.5-350m-q4_k_m", "openelm-270m-q4_k_m", "granite-4.0-h-350m-q8_0"])
+def test_prompt_rows_of_the_workload_shapes_equal_steps(name, synth):
+    """Feed-forward rows over 4096 elements (eight per thread) and 48 SSM heads."""
+    _same_state(name, (70, 3), synth)
