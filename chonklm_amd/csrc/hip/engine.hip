@@ -596,9 +596,8 @@ struct chonk_engine {
   uint8_t* scratch = nullptr;  // device address of this GPU's no-allocation prompt-pass scratch
   int noalloc_rows = 0;        // rows one chonk_engine_prefill_noalloc call may take (0: none)
   void* pf_mem = nullptr;
-  float *pf_x = nullptr, *pf_qkv = nullptr, *pf_att = nullptr, *pf_g = nullptr, *pf_u = nullptr, *pf_act = nullptr,
-        *pf_d = nullptr, *pf_xscale = nullptr, *pf_part = nullptr;
-  _Float16 *pf_h = nullptr, *pf_l = nullptr;
+  float *pf_x = nullptr, *pf_qkv = nullptr, *pf_att = nullptr, *pf_g = nullptr, *pf_u = nullptr, *pf_d = nullptr, *pf_xscale = nullptr, *pf_part = nullptr;
+  _Float16 *pf_h = nullptr, *pf_l = nullptr, *pf_xs = nullptr;
   int32_t* pf_tok = nullptr;
   // status
   std::atomic<bool> busy{false};
@@ -2304,9 +2303,8 @@ constexpr int64_t kPartFloats = (int64_t)4 << 20;  // K-split partial sums
 
 // Device buffers of a row batch (rows <= cap).
 struct RowBufs {
-  float *x = nullptr, *qkv = nullptr, *att = nullptr, *g = nullptr, *u = nullptr, *act = nullptr, *d = nullptr,
-        *xscale = nullptr, *part = nullptr;
-  _Float16 *h = nullptr, *l = nullptr;
+  float *x = nullptr, *qkv = nullptr, *att = nullptr, *g = nullptr, *u = nullptr, *d = nullptr, *xscale = nullptr, *part = nullptr;
+  _Float16 *h = nullptr, *l = nullptr, *xs = nullptr;
   int32_t* tok = nullptr;
   int cap = 0;
   int64_t part_cap = 0;  // floats in part
@@ -2330,8 +2328,10 @@ size_t row_bufs_layout(const ModelCfg& c, int rows, uint8_t* base, RowBufs* out)
   // (Mamba2 layers: the convolved rows in g, the scan's output in u)
   const size_t inner = c.ssm_inner, G = std::max(F, inner ? (size_t)pf_mamba_ld(c.ssm_conv, c.ssm_heads) : 0);
   const size_t kmax = gemm_kpad((int)std::max({H, qdim, F, inner}));
-  const size_t sizes[12] = {R * H * 4, R * (qdim + 2 * kvdim) * 4, R * qdim * 4, R * G * 4, R * std::max(F, inner) * 4, R * F * 4,
-                            R * H * 4, R * 4, (size_t)row_part_floats(c, rows) * 4, R * kmax * 2, R * kmax * 2, R * 4};
+  const size_t sizes[12] = {R * H * 4, R * (qdim + 2 * kvdim) * 4, R * qdim * 4, R * G * 4,
+                            R * std::max(F, inner) * 4, std::max(R * F * 4, R * (kmax / 32) * 4),
+                            R * H * 4, R * 4, (size_t)row_part_floats(c, rows) * 4, plane_rows(rows) * kmax * 2,
+                            plane_rows(rows) * kmax * 2, R * 4};
   size_t off = 0;
   void* ptr[12];
   for (int i = 0; i < 12; ++i) {
@@ -2344,7 +2344,7 @@ size_t row_bufs_layout(const ModelCfg& c, int rows, uint8_t* base, RowBufs* out)
     out->att = (float*)ptr[2];
     out->g = (float*)ptr[3];
     out->u = (float*)ptr[4];
-    out->act = (float*)ptr[5];
+    out->xs = (_Float16*)ptr[5];
     out->d = (float*)ptr[6];
     out->xscale = (float*)ptr[7];
     out->part = (float*)ptr[8];
@@ -2394,6 +2394,7 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
     a.xh = b.h;
     a.xl = b.l;
     a.xscale = b.xscale;
+    a.xs = b.xs;
     a.add = add;
     a.add_w = add_w;
     a.add_scale = c.res_scale;
@@ -2409,6 +2410,7 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
     g.xh = b.h;
     g.xl = b.l;
     g.xscale = b.xscale;
+    g.xs = b.xs;
     g.t = rows;
     g.kpad = gemm_kpad(m.q.k);
     g.ws = m.ws;
@@ -2419,7 +2421,10 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
   // one launch over two or three matrices of one type and K whose results are
   // column ranges of one partial-sum row (segments start on 64-row tiles);
   // returns false (nothing launched) when the matrices do not qualify
-  auto gemm_fused = [&](std::initializer_list<const DevMat*> ms, int rows, PartSum* out) {
+  // (epi GEMM_SWIGLU / GEMM_GEGLU: gate and up, leaving the product, where a launch can)
+  auto gemm_fused = [&](std::initializer_list<const DevMat*> ms, int rows, PartSum* out, int epi = GEMM_STORE,
+                        int64_t cap = 0) {
+    if (cap == 0) cap = b.part_cap;
     std::vector<const DevMat*> m(ms);
     for (size_t i = 1; i < m.size(); ++i)
       if (m[i]->q.type != m[0]->q.type || m[i]->q.k != m[0]->q.k || m[i - 1]->q.n % 64 != 0) return false;
@@ -2433,11 +2438,17 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
     g.xh = b.h;
     g.xl = b.l;
     g.xscale = b.xscale;
+    g.xs = b.xs;
     g.t = rows;
     g.kpad = gemm_kpad(m[0]->q.k);
     g.ws = m[0]->ws;
     for (const DevMat* d : m) g.ws = std::min(g.ws, d->ws);  // every matrix stays below 2^14
-    HIP_OK(launch_gemm_deferred(g, b.part, b.part_cap, out, s));
+    if (epi != GEMM_STORE) {
+      g.epi = epi;
+      HIP_OK(launch_gemm_glu(g, b.part, cap, out, s));
+      return out->p != nullptr;
+    }
+    HIP_OK(launch_gemm_deferred(g, b.part, cap, out, s));
     return true;
   };
   // column range [c0, c0 + n) of a fused result
@@ -2484,6 +2495,7 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
       cv.xh = b.h;
       cv.xl = b.l;
       cv.xscale = b.xscale;
+      cv.xs = b.xs;
       if (!last_kv) HIP_OK(launch_pf_conv(cv, T, s));
       HIP_OK(launch_pf_conv_state(cv, T, s));
       if (last_kv) break;
@@ -2517,6 +2529,7 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
       gt.xh = b.h;
       gt.xl = b.l;
       gt.xscale = b.xscale;
+      gt.xs = b.xs;
       HIP_OK(launch_pf_gate(gt, T, s));
       po = gemm(L.ssm_out, T, 0, P);
     } else {
@@ -2535,10 +2548,18 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
         r.pv = columns(fused, qdim + kvdim, kvdim);
       } else {
         // the partial-sum buffer shared out in proportion to each result's size
-        const int64_t pq = P * qdim / ldqkv, pk = P * kvdim / ldqkv;
-        r.pq = gemm(L.q, T, 0, pq);
-        r.pk = gemm(L.k, T, pq, pk);
-        r.pv = gemm(L.v, T, pq + pk, P - pq - pk);
+        // (multiples of four floats, for 16-byte reads); v often has a type of its
+        // own, so q and k are fused without it where they can be
+        const int64_t pqk = P * (qdim + kvdim) / ldqkv & ~(int64_t)3;
+        if (gemm_fused({&L.q, &L.k}, T, &fused, GEMM_STORE, pqk)) {
+          r.pq = columns(fused, 0, qdim);
+          r.pk = columns(fused, qdim, kvdim);
+        } else {
+          const int64_t pq = P * qdim / ldqkv & ~(int64_t)3;
+          r.pq = gemm(L.q, T, 0, pq);
+          r.pk = gemm(L.k, T, pq, pqk - pq);
+        }
+        r.pv = gemm(L.v, T, pqk, P - pqk);
       }
       r.qkv = b.qkv;
       r.ld = ldqkv;
@@ -2572,10 +2593,13 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
       at.kv = r.kv;
       bool planes = false;  // the attention wrote the o-projection's operand planes
       if (walk) {
-        at.oh = b.h;
-        at.ol = b.l;
-        at.oscale = b.xscale;
-        at.okpad = gemm_kpad(qdim);
+        // (the walk writes no sums of x)
+        if (!gemm_needs_sums(L.o.q.type, qdim, T)) {
+          at.oh = b.h;
+          at.ol = b.l;
+          at.oscale = b.xscale;
+          at.okpad = gemm_kpad(qdim);
+        }
         HIP_OK(launch_bd_attn(at, T, b.part, P, s, &planes, fuse_rope ? &r : nullptr));
       } else {
         HIP_OK(launch_pf_attn(at, T, s));
@@ -2588,9 +2612,12 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
           L.post_norm_b);
     PfGluArgs gl{};
     PartSum gu{};
+    gl.act = c.gpt ? PF_GELU_BIAS : c.gemma ? PF_GEGLU : PF_SWIGLU;
     if (c.gpt) {
       gl.pu = gemm(L.up, T, 0, P);
       gl.bias = L.up_b;
+    } else if (gemm_fused({&L.gate, &L.up}, T, &gl.pu, c.gemma ? GEMM_GEGLU : GEMM_SWIGLU)) {
+      gl.act = PF_DONE;
     } else if (gemm_fused({&L.gate, &L.up}, T, &gu)) {
       gl.pg = columns(gu, 0, F);
       gl.pu = columns(gu, F, F);
@@ -2600,10 +2627,10 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
     }
     gl.k = F;
     gl.kpad = gemm_kpad(F);
-    gl.act = c.gpt ? PF_GELU_BIAS : c.gemma ? PF_GEGLU : PF_SWIGLU;
     gl.xh = b.h;
     gl.xl = b.l;
     gl.xscale = b.xscale;
+    gl.xs = b.xs;
     HIP_OK(launch_pf_glu_split(gl, T, s));
     pending = gemm(L.down, T, 0, P);
     pending_w = c.gemma ? L.post_ffn_norm : nullptr;
@@ -2618,6 +2645,7 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
     g.xh = b.h;
     g.xl = b.l;
     g.xscale = b.xscale;
+    g.xs = b.xs;
     g.y = logits;
     g.ldy = c.vocab;
     g.t = nlr;
@@ -2649,7 +2677,7 @@ void prefill_alloc(chonk_engine* e) {
   e->pf_att = b.att;
   e->pf_g = b.g;
   e->pf_u = b.u;
-  e->pf_act = b.act;
+  e->pf_xs = b.xs;
   e->pf_d = b.d;
   e->pf_xscale = b.xscale;
   e->pf_part = b.part;
@@ -2665,7 +2693,7 @@ RowBufs engine_row_bufs(const chonk_engine* e) {
   b.att = e->pf_att;
   b.g = e->pf_g;
   b.u = e->pf_u;
-  b.act = e->pf_act;
+  b.xs = e->pf_xs;
   b.d = e->pf_d;
   b.xscale = e->pf_xscale;
   b.part = e->pf_part;
@@ -3590,8 +3618,9 @@ int chonk_gemm(int32_t device, uint32_t ggml_type, const void* blocks, int64_t n
       }
       float* d_x = (float*)dev((size_t)n_tokens * row_len * 4);
       float* d_y = (float*)dev((size_t)n_tokens * n_rows * 4);
-      _Float16* d_h = (_Float16*)dev((size_t)n_tokens * kpad * 2);
-      _Float16* d_l = (_Float16*)dev((size_t)n_tokens * kpad * 2);
+      _Float16* d_h = (_Float16*)dev((size_t)plane_rows((int)n_tokens) * kpad * 2);
+      _Float16* d_l = (_Float16*)dev((size_t)plane_rows((int)n_tokens) * kpad * 2);
+      _Float16* d_xs = (_Float16*)dev((size_t)n_tokens * (kpad / 32) * 4);
       float* d_s = (float*)dev((size_t)n_tokens * 4);
       float* d_part = (float*)dev((size_t)kPartFloats * 4);
       HIP_OK(hipMemcpy(d_x, x, (size_t)n_tokens * row_len * 4, hipMemcpyHostToDevice));
@@ -3603,11 +3632,13 @@ int chonk_gemm(int32_t device, uint32_t ggml_type, const void* blocks, int64_t n
       sa.xh = d_h;
       sa.xl = d_l;
       sa.xscale = d_s;
+      sa.xs = d_xs;
       GemmArgs g{};
       g.w = q;
       g.xh = d_h;
       g.xl = d_l;
       g.xscale = d_s;
+      g.xs = d_xs;
       g.y = d_y;
       g.ldy = (int)n_rows;
       g.t = (int)n_tokens;

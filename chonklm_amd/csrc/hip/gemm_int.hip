@@ -1,19 +1,26 @@
-// Prompt GEMM over the weights' integer codes (Q4_K, Q6_K, Q8_0), gfx950.
+// Prompt GEMM over the weights' integer codes, gfx950.
 //
-//   Q4_K  W = d (sc (q - 8)) + c,   c = 8 d sc - dmin m per 32 k
-//   Q6_K  W = d (sc (q - 32))
-//   Q8_0  W = d q
+//   Q4_K, Q5_K  W = d (sc (q - z)) + c,   z = 8, 16,  c = z d sc - dmin m per 32 k
+//   Q6_K        W = d (sc (q - 32))
+//   Q8_0, Q5_0  W = d q,  d (q - 16)
+//   Q5_1        W = d q + m, formed in fp32
 //
-// sc (q - 8) of Q4_K is an integer below 2^9, exact in one fp16 plane, so the
-// matrix cores multiply it with the hi and lo activation planes (two products
+// sc (q - z) of Q4_K and Q5_K is an integer below 2^10, exact in one fp16 plane, so
+// the matrix cores multiply it with the hi and lo activation planes (two products
 // per 16x16x32 step where fp16 hi + lo weights take three, and no rounded
 // weight): the sums of a 256-k super-block are scaled by d once, and c, which
 // is constant over 32 k, meets the sums of x over those 32 k in one more MFMA
-// per super-block. sc (q - 32) of Q6_K has 13 bits and d q of Q8_0 up to 19, so
-// those keep two planes, split exactly (h = fp16(v), l = v - h by one fma).
+// per super-block. sc (q - 32) of Q6_K has 13 bits and d q up to 19, so the
+// other types keep two planes, split exactly (h = fp16(v), l = v - h by one fma).
 // Codes become fp16 by byte permutes under the exponent of 1024 and one or
-// two packed fp16 instructions per pair, about 1.5 VALU instructions per weight
-// (5 for the fp32 dequantization of k_gemm).
+// two packed fp16 instructions per pair, about 1.5 VALU instructions per weight.
+//
+// Against the three-product GEMM over fp32-dequantized hi + lo weights that it
+// replaces (MI355X, 2047 token rows): Q4_K 4096 x 1024 95.0 -> 47.9 us, 6144 x 1024
+// 139.5 -> 65.2, Q6_K 1024 x 3072 90.6 -> 41.2, Q8_0 3376 x 768 74.3 -> 41.1; error
+// against float64 3.6e-7 -> 1.4e-7 (Q4_K), 6.2e-7 -> 1.7e-7 (Q6_K). What is left:
+// 16 us of the 4096-row launch are its 34 MB of fp32 results, the rest is the
+// products at the rate the matrix cores sustain beside the staging.
 #include <hip/hip_runtime.h>
 
 #include "kernel_common.h"
@@ -61,6 +68,19 @@ struct Codes<QT_Q4_K, NG> {
   uint4 q[NG], hdr;
 };
 template <int NG>
+struct Codes<QT_Q5_K, NG> {
+  uint4 q[NG], qh[NG], hdr;
+};
+template <int NG>
+struct Codes<QT_Q5_0, NG> {
+  uint4 q[NG];
+  uint32_t qh[NG], d[NG];
+};
+template <int NG>
+struct Codes<QT_Q5_1, NG> {
+  Frag<QT_Q5_1> f[NG];
+};
+template <int NG>
 struct Codes<QT_Q6_K, NG> {
   uint4 ql[NG], qh;
   uint2 sc;
@@ -72,12 +92,17 @@ struct Codes<QT_Q8_0, NG> {
   uint32_t d[NG];
 };
 
+// sums of a super-block are scaled by d; block offsets c
 template <int T>
-constexpr int gemm_int_planes() { return T == QT_Q4_K ? 1 : 2; }
+constexpr bool gemm_int_sb = T == QT_Q4_K || T == QT_Q5_K || T == QT_Q6_K;
+template <int T>
+constexpr bool gemm_int_offsets = T == QT_Q4_K || T == QT_Q5_K;
+template <int T>
+constexpr int gemm_int_planes() { return gemm_int_offsets<T> ? 1 : 2; }
 template <int T, int NI>
 constexpr size_t gemm_int_shared() {
-  return sizeof(_Float16) * gemm_int_planes<T>() * 16 * NI * kIS + (T == QT_Q4_K ? 16 * NI * 16 * sizeof(_Float16) : 0) +
-         (T != QT_Q8_0 ? 16 * NI * sizeof(float) : 0);
+  return sizeof(_Float16) * gemm_int_planes<T>() * 16 * NI * kIS + (gemm_int_offsets<T> ? 16 * NI * 16 * sizeof(_Float16) : 0) +
+         (gemm_int_sb<T> ? 16 * NI * sizeof(float) : 0);
 }
 
 // 16 NI weight rows x 64 TJ token rows per workgroup; wave w owns token rows
@@ -87,15 +112,19 @@ constexpr size_t gemm_int_shared() {
 // through the vector cache and 32 KB of LDS reads under 512 cycles of MFMA,
 // half of what either can move in that time; 64 weight rows would need the
 // whole of the vector cache's rate. Codes of the next stage are in flight
-// while this one is multiplied.
-template <int T, int NI, int TJ>
+// while this one is multiplied, weight fragments are read from LDS three ahead
+// of their products, and the results leave through LDS as whole runs of a row
+// (64-byte pieces of 16 rows at a time cost 15 us more at 4096 x 1024 x 2047).
+// GLU: the first half of the weight rows are gate rows (a.w), the second the same
+// rows of up (a.w2).
+template <int T, int NI, int TJ, bool GLU>
 __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
   extern __shared__ __align__(16) _Float16 gism[];
   constexpr int R = 16 * NI, NP = gemm_int_planes<T>(), NG = NI / 4;
-  constexpr bool SB = T != QT_Q8_0;  // sums of a super-block are scaled by d
+  constexpr bool SB = gemm_int_sb<T>, OFF = gemm_int_offsets<T>;
   _Float16* wp = gism;                                   // [NP][R][kIS]
-  _Float16* cs = wp + NP * R * kIS;                      // Q4_K: [R][16], c of eight sub-blocks hi | lo
-  float* ds = (float*)(cs + (T == QT_Q4_K ? R * 16 : 0));  // [R] d 2^(ws - 5) (Q6_K: d 2^ws)
+  _Float16* cs = wp + NP * R * kIS;                      // OFF: [R][16], c of eight sub-blocks hi | lo
+  float* ds = (float*)(cs + (OFF ? R * 16 : 0));  // [R] d 2^(ws - 5) (Q6_K: d 2^ws)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * R, t0 = blockIdx.y * 64 * TJ;
@@ -110,30 +139,40 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
   // staging role: row wr, part wq of its 128 k (rows past N repeat the last row)
   constexpr int TPR = kWg / R;  // threads per row
   const int wr = tid / TPR, wq = tid % TPR;
-  const int gr = min(n0 + wr, N - 1);
-  const int seg = a.n_all ? (gr >= a.n2 ? 2 : (gr >= a.n1 ? 1 : 0)) : 0;
-  const size_t row = gr - (seg == 2 ? a.n2 : (seg == 1 ? a.n1 : 0));
+  const int gr = GLU ? min((int)blockIdx.x * (R / 2) + wr % (R / 2), a.n1 - 1) : min(n0 + wr, N - 1);
+  const int seg = GLU ? wr / (R / 2) : a.n_all ? (gr >= a.n2 ? 2 : (gr >= a.n1 ? 1 : 0)) : 0;
+  const size_t row = GLU ? gr : gr - (seg == 2 ? a.n2 : (seg == 1 ? a.n1 : 0));
 #define CHONK_PICK_S(f) (seg == 2 ? a.w3.f : (seg == 1 ? a.w2.f : a.w.f))
   const uint8_t *p0, *p1, *p2 = nullptr, *p3 = nullptr;
-  if constexpr (T == QT_Q4_K) {
+  if constexpr (OFF) {
     p0 = CHONK_PICK_S(s0) + row * (K / 2) + 16 * NG * wq;
     p1 = CHONK_PICK_S(s1) + row * (K / 16);
+    if constexpr (T == QT_Q5_K) p2 = CHONK_PICK_S(s2) + row * (K / 8) + (NG == 1 ? 16 * (wq & 1) : 0);
   } else if constexpr (T == QT_Q6_K) {
     // NI = 8: part wq = l / 16 of every quarter; NI = 4: also one ql run of the two
     p0 = CHONK_PICK_S(s0) + row * (K / 2) + 16 * (wq & 1) + (NG == 1 ? 32 * (wq >> 1) : 0);
     p1 = CHONK_PICK_S(s1) + row * (K / 4) + 16 * (wq & 1);
     p2 = CHONK_PICK_S(s2) + row * (K / 16);
     p3 = CHONK_PICK_S(s3) + row * (K / 256) * 2;
-  } else {
+  } else if constexpr (T == QT_Q8_0) {
     p0 = CHONK_PICK_S(s0) + row * K;
     p1 = CHONK_PICK_S(s1) + row * (K / 32) * 2;
+  } else {
+    p0 = CHONK_PICK_S(s0) + row * (K / 2);
+    p1 = CHONK_PICK_S(s1) + row * (K / 32) * 4;
+    p2 = CHONK_PICK_S(s2) + row * (K / 32) * 2;
+    if constexpr (T == QT_Q5_1) p3 = CHONK_PICK_S(s3) + row * (K / 32) * 2;
   }
 #undef CHONK_PICK_S
   Codes<T, NG> f;
   auto fetch = [&](int s) {
-    if constexpr (T == QT_Q4_K) {
+    if constexpr (OFF) {
 #pragma unroll
       for (int g = 0; g < NG; ++g) f.q[g] = ldg4(p0 + 64 * s + 16 * g);
+      if constexpr (T == QT_Q5_K) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) f.qh[g] = ldg4(p2 + 32 * (s >> 1) + 16 * g);
+      }
       f.hdr = ldg4(p1 + 16 * (s >> 1));
     } else if constexpr (T == QT_Q6_K) {
 #pragma unroll
@@ -145,36 +184,69 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
         const int u = min(4 * s + NG * wq + g, (K >> 5) - 1);  // (the last stage may hold fewer units)
-        f.q[2 * g] = ldg4(p0 + 32 * u);
-        f.q[2 * g + 1] = ldg4(p0 + 32 * u + 16);
-        f.d[g] = ld_u16(p1 + 2 * u);
+        if constexpr (T == QT_Q8_0) {
+          f.q[2 * g] = ldg4(p0 + 32 * u);
+          f.q[2 * g + 1] = ldg4(p0 + 32 * u + 16);
+          f.d[g] = ld_u16(p1 + 2 * u);
+        } else if constexpr (T == QT_Q5_0) {
+          f.q[g] = ldg4(p0 + 16 * u);
+          f.qh[g] = ldg1(p1 + 4 * u);
+          f.d[g] = ld_u16(p2 + 2 * u);
+        } else {
+          f.f[g].qs = ldg4(p0 + 16 * u);
+          f.f[g].qh = ldg1(p1 + 4 * u);
+          f.f[g].d = ld_u16(p2 + 2 * u);
+          f.f[g].m = ld_u16(p3 + 2 * u);
+        }
       }
     }
   };
-  auto stage = [&](int s) {
+  auto stage = [&]<int PAR>(int s) {
     _Float16* rh = wp + wr * kIS;
     _Float16* rl = rh + R * kIS;
-    if constexpr (T == QT_Q4_K) {
+    if constexpr (OFF) {
       const float d = h2f(f.hdr.x) * wsc, dm = h2f(f.hdr.x >> 16) * wsc;
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
         // bytes 16 p .. + 16 of sub-blocks 2 c, 2 c + 1 (low and high nibbles)
         const int gi = NG * wq + g, c = gi >> 1, p = gi & 1;
-        const int j = 4 * (s & 1) + 2 * c;
+        const int j = 4 * PAR + 2 * c;
         uint32_t sc[2], m[2];
-        scale_min(j, f.hdr.y, f.hdr.z, f.hdr.w, &sc[0], &m[0]);
-        scale_min(j + 1, f.hdr.y, f.hdr.z, f.hdr.w, &sc[1], &m[1]);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          // scale_min of sub-block j + h, in the half known here (bytes j, j + 4, j + 8 of the 12)
+          const int b = 8 * (2 * c + h);
+          if constexpr (PAR == 0) {
+            sc[h] = (f.hdr.y >> b) & 63u;
+            m[h] = (f.hdr.z >> b) & 63u;
+          } else {
+            const uint32_t lo = f.hdr.w >> b;
+            sc[h] = (lo & 15u) | (((f.hdr.y >> b) >> 2) & 48u);
+            m[h] = ((lo >> 4) & 15u) | (((f.hdr.z >> b) >> 2) & 48u);
+          }
+        }
         const uint32_t w[4] = {f.q[g].x, f.q[g].y, f.q[g].z, f.q[g].w};
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          // (1024 + 16 q) sc / 16 - 72 sc = sc (q - 8): every step exact
-          const half2_t k = splat((float)sc[h] * 0.0625f), z = splat((float)sc[h] * -72.0f);
           half2_t v[8];
+          if constexpr (T == QT_Q4_K) {
+            // (1024 + 16 q) sc / 16 - 72 sc = sc (q - 8): every step exact
+            const half2_t k = splat((float)sc[h] * 0.0625f), z = splat((float)sc[h] * -72.0f);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t b = (h ? w[i] : w[i] << 4) & 0xf0f0f0f0u;
-            v[2 * i] = __builtin_elementwise_fma(bytes01(b), k, z);
-            v[2 * i + 1] = __builtin_elementwise_fma(bytes23(b), k, z);
+            for (int i = 0; i < 4; ++i) {
+              const uint32_t b = (h ? w[i] : w[i] << 4) & 0xf0f0f0f0u;
+              v[2 * i] = __builtin_elementwise_fma(bytes01(b), k, z);
+              v[2 * i + 1] = __builtin_elementwise_fma(bytes23(b), k, z);
+            }
+          } else {
+            const half2_t k = splat((float)sc[h]);
+            const uint32_t hw[4] = {f.qh[g].x, f.qh[g].y, f.qh[g].z, f.qh[g].w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const uint32_t b = ((w[i] >> (4 * h)) & 0x0f0f0f0fu) | (((hw[i] >> (j + h)) & 0x01010101u) << 4);
+              v[2 * i] = (bytes01(b) - half2_t{1040, 1040}) * k;
+              v[2 * i + 1] = (bytes23(b) - half2_t{1040, 1040}) * k;
+            }
           }
           put16(rh + 64 * c + 32 * h + 16 * p, v);
         }
@@ -182,7 +254,7 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
           _Float16* cr = cs + wr * 16 + j;
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            const float cc = fmaf(8.0f * d, (float)sc[h], -(dm * (float)m[h]));
+            const float cc = fmaf((T == QT_Q4_K ? 8.0f : 16.0f) * d, (float)sc[h], -(dm * (float)m[h]));
             const _Float16 ch = (_Float16)cc;
             cr[h] = ch;
             cr[8 + h] = (_Float16)(cc - (float)ch);
@@ -218,6 +290,24 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
         }
       }
       if (wq == 0) ds[wr] = h2f(f.d) * wsc;
+    } else if constexpr (T == QT_Q5_1) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        const int u = NG * wq + g;
+        float v[32];
+        dequant_unit<QT_Q5_1>(f.f[g], 4 * s + u, v, 4 * s + u < (K >> 5) ? wsc : 0.f);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          half2_t vh[8], vl[8];
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            vh[i / 2][i % 2] = (_Float16)v[16 * p + i];
+            vl[i / 2][i % 2] = (_Float16)(v[16 * p + i] - (float)vh[i / 2][i % 2]);
+          }
+          put16(rh + 32 * u + 16 * p, vh);
+          put16(rl + 32 * u + 16 * p, vl);
+        }
+      }
     } else {
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
@@ -225,13 +315,21 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
         const half2_t d = splat(4 * s + u < (K >> 5) ? h2f(f.d[g]) * wsc : 0.f);
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-          const uint4 q4 = f.q[2 * g + p];
+          const uint4 q4 = f.q[T == QT_Q8_0 ? 2 * g + p : g];
           const uint32_t w[4] = {q4.x, q4.y, q4.z, q4.w};
+          const _Float16 z = T == QT_Q8_0 ? 1152 : 1040;
           half2_t vh[8], vl[8];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const uint32_t b = w[i] ^ 0x80808080u;  // q + 128
-            const half2_t x0 = bytes01(b) - half2_t{1152, 1152}, x1 = bytes23(b) - half2_t{1152, 1152};
+            uint32_t b;
+            if constexpr (T == QT_Q8_0) {
+              b = w[i] ^ 0x80808080u;  // q + 128
+            } else {
+              // element 16 p + 4 i + e: nibble p of byte 4 i + e, bit of qh under bit 4 of byte e
+              const uint32_t x = (f.qh[g] >> (16 * p + 4 * i)) & 15u;
+              b = ((w[i] >> (4 * p)) & 0x0f0f0f0fu) | (((x | x << 7 | x << 14 | x << 21) & 0x01010101u) << 4);
+            }
+            const half2_t x0 = bytes01(b) - half2_t{z, z}, x1 = bytes23(b) - half2_t{z, z};
             vh[2 * i] = x0 * d;
             vh[2 * i + 1] = x1 * d;
             vl[2 * i] = __builtin_elementwise_fma(x0, d, -vh[2 * i]);
@@ -245,14 +343,14 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
   };
 
   // operand role: lane l holds row (or token) l % 16 and k 8 (l / 16) .. + 8 of a
-  // 32-k step; plane rows as 32-bit byte offsets from the planes' bases, a token
-  // row past t reads row t - 1: its products are computed and dropped
+  // 32-k step; the lane's pieces as 32-bit byte offsets from the planes' bases, a
+  // row tile past the last one reads that: its products are computed and dropped
   const int col = lane & 15, quad = lane >> 4;
   uint32_t xo[TJ], so[TJ];
 #pragma unroll
   for (int j = 0; j < TJ; ++j) {
     const uint32_t t = min(t0 + 16 * (TJ * wave + j) + col, a.t - 1);
-    xo[j] = 2u * (t * (uint32_t)a.kpad + 8u * quad);
+    xo[j] = 2u * (uint32_t)plane_at(16 * min((t0 + 16 * (TJ * wave + j)) / 16, (a.t - 1) / 16), 0, a.kpad) + 16u * lane;
     // sums of x: [t][hi | lo][kpad / 32]; quads 0, 1: hi, 2: lo (3: times zero)
     so[j] = 2u * (uint32_t)(a.kpad / 32) * (2 * t + (quad == 2 ? 1u : 0u));
   }
@@ -266,158 +364,209 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < TJ; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-  if (s_lo < s_hi) fetch(s_lo);
-  for (int s = s_lo; s < s_hi; ++s) {
-    // the stage's activation operands: the first steps' ahead of the staging,
-    // the others' (when there is no register room for all) ahead of the products
-    constexpr int EARLY = TJ == 2 ? 2 : kIK / 32;
-    half8_t bh[kIK / 32][TJ], bl[kIK / 32][TJ];
-    auto load_x = [&](int k0, int k1) {
+  // The activation operands of 32-k step st sit in slot st % NS, requested LA
+  // steps ahead of their use (the last steps request the last one again).
+  constexpr int SPS = kIK / 32, NS = TJ == 2 ? 4 : 8, LA = TJ == 2 ? 2 : 6;
+  const int st_hi = SPS * s_hi - 1;
+  half8_t bh[NS][TJ], bl[NS][TJ];
+  auto load_x = [&](int st, int slot) {
 #pragma unroll
-      for (int ks = k0; ks < k1; ++ks)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-          const uint32_t o = xo[j] + 2u * (uint32_t)(s * kIK + ks * 32);
-          bh[ks][j] = *(const half8_t*)(xhb + o);
-          bl[ks][j] = *(const half8_t*)(xlb + o);
-        }
-    };
-    load_x(0, EARLY);
+    for (int j = 0; j < TJ; ++j) {
+      const uint32_t o = xo[j] + 1024u * (uint32_t)min(st, st_hi);
+      bh[slot][j] = *(const half8_t*)(xhb + o);
+      bl[slot][j] = *(const half8_t*)(xlb + o);
+    }
+  };
+  // one stage; PAR: its parity from s_lo on (for super-block types its half)
+  auto body = [&]<int PAR>(int s) {
     half8_t xb[TJ];
-    if constexpr (T == QT_Q4_K) {
+    if constexpr (OFF && PAR == 1) {
 #pragma unroll
       for (int j = 0; j < TJ; ++j) xb[j] = *(const half8_t*)(xsb + so[j] + 16u * (uint32_t)(s >> 1));
     }
     lds_barrier();  // the previous stage's tile is consumed
-    stage(s);
+    stage.template operator()<PAR>(s);
     fetch(min(s + 1, s_hi - 1));
     lds_barrier();  // (the codes and operands in flight are not waited for)
-    load_x(EARLY, kIK / 32);
-    if constexpr (SB) {
-      if (!(s & 1)) {
+    // the products: weight fragment f is plane f % NP of row tile f / NP % NI and
+    // 32-k step f / NP / NI; AD fragments are read from LDS ahead of their use
+    // (left alone, the compiler reads one at a time and waits for it)
+    constexpr int NF = SPS * NI * NP, AD = 3;
+    auto frag = [&](int fi) {
+      const int p = fi % NP, i = fi / NP % NI, ks = fi / NP / NI;
+      return *(const half8_t*)(wp + p * R * kIS + (16 * i + col) * kIS + ks * 32 + 8 * quad);
+    };
+    half8_t af[AD + 1];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+    for (int fi = 0; fi < AD; ++fi) af[fi] = frag(fi);
 #pragma unroll
-          for (int j = 0; j < TJ; ++j) tmp[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int fi = 0; fi < NF; ++fi) {
+      const int p = fi % NP, i = fi / NP % NI, ks = fi / NP / NI, sl = (SPS * PAR + ks) % NS;
+      if (fi + AD < NF) af[(fi + AD) % (AD + 1)] = frag(fi + AD);
+      if (p == 0 && i == 0) load_x(SPS * s + ks + LA, (SPS * PAR + ks + LA) % NS);
+      const half8_t w = af[fi % (AD + 1)];
+      auto& dst = [&]() -> auto& {
+        if constexpr (SB)
+          return tmp[i];
+        else
+          return acc[i];
+      }();
+      const bool first = SB && PAR == 0 && ks == 0 && p == 0;
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) dst[j] = mfma32(w, bh[sl][j], first ? float4_t{0.f, 0.f, 0.f, 0.f} : dst[j]);
+      if (p == 0) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) dst[j] = mfma32(w, bl[sl][j], dst[j]);
       }
     }
+    // (schedule: AD LDS reads, then per fragment one read and its products)
+    __builtin_amdgcn_sched_group_barrier(0x100, AD, 0);
 #pragma unroll
-    for (int ks = 0; ks < kIK / 32; ++ks)
+    for (int fi = 0; fi < NF; fi += NP) {
+      if (fi % (NP * NI) == 0) __builtin_amdgcn_sched_group_barrier(0x20, 2 * TJ, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x8, 2 * TJ, 0);
+      if constexpr (NP == 2) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x8, TJ, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (SB && PAR == 1) {
+      // the super-block's sums times d, and its c times the sums of x:
+      // k 0..7 c_hi Xh, 8..15 c_lo Xh, 16..23 c_hi Xl, 24..31 nothing
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        auto& dst = [&]() -> auto& {
-          if constexpr (SB)
-            return tmp[i];
-          else
-            return acc[i];
-        }();
-        const _Float16* ar = wp + (16 * i + col) * kIS + ks * 32 + 8 * quad;
-        const half8_t ah = *(const half8_t*)ar;
+        const float4_t d4 = *(const float4_t*)(ds + 16 * i + 4 * quad);
+        if constexpr (OFF) {
+          half8_t ca = *(const half8_t*)(cs + (16 * i + col) * 16 + (quad == 1 ? 8 : 0));
+          if (quad == 3) ca = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) dst[j] = mfma32(ah, bh[ks][j], dst[j]);
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) dst[j] = mfma32(ah, bl[ks][j], dst[j]);
-        if constexpr (NP == 2) {
-          const half8_t al = *(const half8_t*)(ar + R * kIS);
-#pragma unroll
-          for (int j = 0; j < TJ; ++j) dst[j] = mfma32(al, bh[ks][j], dst[j]);
+          for (int j = 0; j < TJ; ++j) acc[i][j] = mfma32(ca, xb[j], acc[i][j]);
         }
-      }
-    if constexpr (SB) {
-      if (s & 1) {
-        // the super-block's sums times d, and (Q4_K) its c times the sums of x:
-        // k 0..7 c_hi Xh, 8..15 c_lo Xh, 16..23 c_hi Xl, 24..31 nothing
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          const float4_t d4 = *(const float4_t*)(ds + 16 * i + 4 * quad);
-          if constexpr (T == QT_Q4_K) {
-            half8_t ca = *(const half8_t*)(cs + (16 * i + col) * 16 + (quad == 1 ? 8 : 0));
-            if (quad == 3) ca = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        for (int j = 0; j < TJ; ++j)
 #pragma unroll
-            for (int j = 0; j < TJ; ++j) acc[i][j] = mfma32(ca, xb[j], acc[i][j]);
-          }
-#pragma unroll
-          for (int j = 0; j < TJ; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[i][j][q] = fmaf(d4[q], tmp[i][j][q], acc[i][j][q]);
-        }
+          for (int q = 0; q < 4; ++q) acc[i][j][q] = fmaf(d4[q], tmp[i][j][q], acc[i][j][q]);
       }
     }
+  };
+  if (s_lo < s_hi) {
+#pragma unroll
+    for (int st = 0; st < LA; ++st) load_x(SPS * s_lo + st, st);
+    fetch(s_lo);
   }
-  // lane holds rows 4 quad + 0..3 of each 16-row tile, token col
-  const float wun = ldexpf(1.0f, (T == QT_Q4_K ? 5 : 0) - a.ws);
+  for (int s = s_lo; s < s_hi; s += 2) {
+    body.template operator()<0>(s);
+    if (SB || s + 1 < s_hi) body.template operator()<1>(s + 1);
+  }
+  // The lane holds rows 4 quad + 0..3 of each 16-row tile, token col. Each wave
+  // turns its 16-token tiles over in LDS, so that a store instruction writes
+  // whole runs of a token's row (512 bytes at NI = 8); the GLU launch stores
+  // silu(gate) * up (or GELU) of its two halves instead of both.
+  constexpr int RO = GLU ? R / 2 : R, NO = GLU ? NI / 2 : NI;  // columns and row tiles stored
+  constexpr int OS = RO + 4, LPT = RO / 4;                     // LDS stride; lanes per token row
+  const int ncols = GLU ? a.n1 : N, c0 = (int)blockIdx.x * RO;
+  const float wun = ldexpf(1.0f, (OFF ? 5 : 0) - a.ws);
   const bool part = a.ksplit > 1 || a.defer;
-  const bool vec = part && (N & 3) == 0 && ((uintptr_t)a.part & 15) == 0;
+  const bool vec = part && (ncols & 3) == 0 && ((uintptr_t)a.part & 15) == 0;
+  __syncthreads();  // the last stage's tile is consumed
+  float* tile = (float*)gism + wave * 16 * OS;
 #pragma unroll
   for (int j = 0; j < TJ; ++j) {
-    const int tt = t0 + 16 * (TJ * wave + j) + col;
-    if (tt >= a.t) continue;
-    const float sc = wun * a.xscale[tt];
+    const int tt0 = t0 + 16 * (TJ * wave + j);
+    const float sc = wun * a.xscale[min(tt0 + col, a.t - 1)];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int n = n0 + 16 * i + 4 * quad;
-      float* pp = a.part + ((size_t)blockIdx.z * a.t + tt) * N + n;
-      if (vec && n + 4 <= N) {
-        *(float4*)pp = make_float4(acc[i][j][0] * sc, acc[i][j][1] * sc, acc[i][j][2] * sc, acc[i][j][3] * sc);
+    for (int i = 0; i < NO; ++i) {
+      float4_t v = acc[i][j] * sc;
+      if constexpr (GLU) {
+        const float4_t u = acc[i + NO][j] * sc;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[q] = a.epi == GEMM_GEGLU ? __fmul_rn(gelu_tanh(v[q]), u[q]) : silu_mul(v[q], u[q]);
+      }
+      *(float4_t*)(tile + col * OS + 16 * i + 4 * quad) = v;
+    }
+    // (the wave's own LDS accesses are in order)
+#pragma unroll
+    for (int r = 0; r < 16; r += 64 / LPT) {
+      const int tr = r + lane / LPT, cc = 4 * (lane % LPT), tt = tt0 + tr, n = c0 + cc;
+      const float4_t v = *(const float4_t*)(tile + tr * OS + cc);
+      if (tt >= a.t || n >= ncols) continue;
+      float* pp = a.part + ((size_t)blockIdx.z * a.t + tt) * ncols + n;
+      if (vec) {
+        *(float4_t*)pp = v;
         continue;
       }
       float* y = a.y + (size_t)tt * a.ldy + n;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        if (n + q >= N) break;
-        const float v = acc[i][j][q] * sc;
+        if (n + q >= ncols) break;
         if (part)
-          pp[q] = v;
+          pp[q] = v[q];
         else
-          y[q] = a.epi == GEMM_ADD ? __fadd_rn(y[q], v) : v;
+          y[q] = a.epi == GEMM_ADD ? __fadd_rn(y[q], v[q]) : v[q];
       }
     }
   }
 }
 
-template <int T, int NI, int TJ>
+template <int T, int NI, int TJ, bool GLU>
 hipError_t launch_one(const GemmArgs& a, int n_rows, hipStream_t s) {
   const dim3 grid((n_rows + 16 * NI - 1) / (16 * NI), (a.t + 64 * TJ - 1) / (64 * TJ), a.ksplit);
-  hipLaunchKernelGGL((k_gemm_int<T, NI, TJ>), grid, dim3(kWg), (gemm_int_shared<T, NI>()), s, a);
+  hipLaunchKernelGGL((k_gemm_int<T, NI, TJ, GLU>), grid, dim3(kWg), (gemm_int_shared<T, NI>()), s, a);
   return hipGetLastError();
 }
 
 template <int T>
 hipError_t launch_type(const GemmArgs& a, int n_rows, int ni, int tj, hipStream_t s) {
-  if (ni == 8) return tj == 2 ? launch_one<T, 8, 2>(a, n_rows, s) : launch_one<T, 8, 1>(a, n_rows, s);
-  return tj == 2 ? launch_one<T, 4, 2>(a, n_rows, s) : launch_one<T, 4, 1>(a, n_rows, s);
+  if (a.epi == GEMM_SWIGLU || a.epi == GEMM_GEGLU) {
+    if (ni == 8) return tj == 2 ? launch_one<T, 8, 2, true>(a, n_rows, s) : launch_one<T, 8, 1, true>(a, n_rows, s);
+    return tj == 2 ? hipErrorInvalidValue : launch_one<T, 4, 1, true>(a, n_rows, s);
+  }
+  if (ni == 8) return tj == 2 ? launch_one<T, 8, 2, false>(a, n_rows, s) : launch_one<T, 8, 1, false>(a, n_rows, s);
+  return tj == 2 ? launch_one<T, 4, 2, false>(a, n_rows, s) : launch_one<T, 4, 1, false>(a, n_rows, s);
 }
 
+template <int T, int NI, int TJ, bool GLU>
+hipError_t init_one() {
+  return hipFuncSetAttribute((const void*)k_gemm_int<T, NI, TJ, GLU>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)gemm_int_shared<T, NI>());
+}
 template <int T>
 hipError_t init_type() {
-  const std::pair<const void*, size_t> f[4] = {{(const void*)k_gemm_int<T, 8, 2>, gemm_int_shared<T, 8>()},
-                                               {(const void*)k_gemm_int<T, 8, 1>, gemm_int_shared<T, 8>()},
-                                               {(const void*)k_gemm_int<T, 4, 2>, gemm_int_shared<T, 4>()},
-                                               {(const void*)k_gemm_int<T, 4, 1>, gemm_int_shared<T, 4>()}};
-  for (const auto& p : f) {
-    const hipError_t e = hipFuncSetAttribute(p.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.second);
+  for (hipError_t e : {init_one<T, 8, 2, false>(), init_one<T, 8, 1, false>(), init_one<T, 4, 2, false>(),
+                       init_one<T, 4, 1, false>(), init_one<T, 8, 2, true>(), init_one<T, 8, 1, true>(),
+                       init_one<T, 4, 1, true>()})
     if (e != hipSuccess) return e;
-  }
   return hipSuccess;
 }
 
 }  // namespace
 
-bool gemm_int_type(int type) { return type == QT_Q4_K || type == QT_Q6_K || type == QT_Q8_0; }
+bool gemm_int_sums(int type) { return type == QT_Q4_K || type == QT_Q5_K; }
 
 hipError_t launch_gemm_int(const GemmArgs& a, int n_rows, int ni, int tj, hipStream_t s) {
-  if (a.w.type == QT_Q4_K && (!a.xs || a.w.k % 256 != 0)) return hipErrorInvalidValue;
-  if (a.w.type == QT_Q6_K && a.w.k % 256 != 0) return hipErrorInvalidValue;
+  if (gemm_int_sums(a.w.type) && !a.xs) return hipErrorInvalidValue;
+  if (gemm_int_step(a.w.type) == 256 && a.w.k % 256 != 0) return hipErrorInvalidValue;
+  if ((a.epi == GEMM_SWIGLU || a.epi == GEMM_GEGLU) &&
+      (a.ksplit != 1 || !a.defer || a.n2 != 2 * a.n1 || n_rows != a.n2 || a.w.n != a.n1 || a.w2.n != a.n1))
+    return hipErrorInvalidValue;
   switch (a.w.type) {
     case QT_Q4_K: return launch_type<QT_Q4_K>(a, n_rows, ni, tj, s);
+    case QT_Q5_K: return launch_type<QT_Q5_K>(a, n_rows, ni, tj, s);
     case QT_Q6_K: return launch_type<QT_Q6_K>(a, n_rows, ni, tj, s);
     case QT_Q8_0: return launch_type<QT_Q8_0>(a, n_rows, ni, tj, s);
+    case QT_Q5_0: return launch_type<QT_Q5_0>(a, n_rows, ni, tj, s);
+    case QT_Q5_1: return launch_type<QT_Q5_1>(a, n_rows, ni, tj, s);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t init_gemm_int_attributes() {
-  for (hipError_t e : {init_type<QT_Q4_K>(), init_type<QT_Q6_K>(), init_type<QT_Q8_0>()})
+  for (hipError_t e : {init_type<QT_Q4_K>(), init_type<QT_Q5_K>(), init_type<QT_Q6_K>(), init_type<QT_Q8_0>(),
+                       init_type<QT_Q5_0>(), init_type<QT_Q5_1>()})
     if (e != hipSuccess) return e;
   return hipSuccess;
 }

@@ -8,7 +8,9 @@
 
 namespace chonk {
 
-enum GemmEpi : int32_t { GEMM_STORE = 0, GEMM_ADD = 1 };
+// GEMM_SWIGLU / GEMM_GEGLU: w is gate and w2 up (n2 = 2 n1), the result is
+// silu(gate) * up or gelu_tanh(gate) * up with n1 columns (gemm_int.hip)
+enum GemmEpi : int32_t { GEMM_STORE = 0, GEMM_ADD = 1, GEMM_SWIGLU = 2, GEMM_GEGLU = 3 };
 
 // y[t][n] (=|+=) 2^-ws * xscale[t] * sum_k (xh + xl)[t][k] * (W 2^ws)[n][k]
 struct GemmArgs {
@@ -18,9 +20,10 @@ struct GemmArgs {
   // segment starts are multiples of the 64-row tile. n_all = 0: w alone.
   QMat w2, w3;
   int32_t n1, n2, n_all, pad0;
-  const _Float16* xh;     // [t][kpad] activation planes, zero past K
+  const _Float16* xh;     // activation planes (plane_at), zero past K
   const _Float16* xl;
   const float* xscale;    // [t]
+  const _Float16* xs;     // [t][hi | lo][kpad / 32] sums of x over 32 k (pf_split's), or null
   float* y;               // [t][ldy]
   int32_t ldy, t, kpad, epi;
   int32_t ws;             // weight exponent
@@ -59,8 +62,9 @@ struct PfSplitArgs {
   int32_t ldx, k, kpad;
   const float* w;         // RMSNorm weight [k], or null for a plain split
   float eps;
-  _Float16 *xh, *xl;      // [rows][kpad]
+  _Float16 *xh, *xl;      // planes (plane_at)
   float* xscale;          // [rows]
+  _Float16* xs;           // [rows][hi | lo][kpad / 32]: sums of the scaled row over 32 k, times 2^-5
   // residual update first (x must then be writable): x += add, or with
   // add_w (the Gemma-3 sandwich) x = clamp(x + RMSNorm(add) * add_w, +-65000)
   PartSum add;
@@ -70,14 +74,15 @@ struct PfSplitArgs {
   const float *add_bias, *norm_b;
 };
 
-enum PfAct : int32_t { PF_SWIGLU = 0, PF_GEGLU = 1, PF_GELU_BIAS = 2 };
+enum PfAct : int32_t { PF_SWIGLU = 0, PF_GEGLU = 1, PF_GELU_BIAS = 2, PF_DONE = 3 };
 
 struct PfGluArgs {
   PartSum pg, pu;         // gate and up rows [rows][k] (deferred GEMM results)
-  const float* bias;      // PF_GELU_BIAS: gelu(up + bias); pg is not read
+  const float* bias;      // PF_GELU_BIAS: gelu(up + bias); pg is not read. PF_DONE: pu is the product already
   int32_t k, kpad, act;
   _Float16 *xh, *xl;
   float* xscale;
+  _Float16* xs;
 };
 
 // lfm2 short convolution over the rows of a pass, in_proj rows B | C | x of k
@@ -90,6 +95,7 @@ struct PfConvArgs {
   float *s1, *s2;
   _Float16 *xh, *xl;
   float* xscale;
+  _Float16* xs;
 };
 
 // granitehybrid Mamba2 layer over the rows of a pass; in_proj rows z | xBC | dt.
@@ -114,6 +120,7 @@ struct PfGateArgs {
   float eps;
   _Float16 *xh, *xl;
   float* xscale;
+  _Float16* xs;
 };
 
 struct PfRopeArgs {
@@ -135,7 +142,7 @@ struct PfAttnArgs {
   int32_t rows;           // rows of the pass (set by the launcher)
   float scale;
   KvAddr kv;
-  // batched decode: the next GEMM's operand planes [rows][okpad] (hi, lo) and
+  // batched decode: the next GEMM's operand planes (plane_at, okpad; hi, lo) and
   // row scales, written instead of `out` when set and the rows are not split
   // into segments (the output of attention needs no scaling: |x| <= max |V|)
   _Float16* oh;
@@ -144,14 +151,36 @@ struct PfAttnArgs {
   int32_t okpad;
 };
 
-// Widest row the per-row glue kernels hold in registers (eight elements of
-// each of 1024 threads).
+// Widest row the per-row glue kernels hold in registers (four runs of eight
+// elements in each of 256 threads).
 constexpr int kPfRowMax = 8192;
+
+// Operand planes hold the rows in MFMA operand order: 16 rows x 32 columns are
+// 512 consecutive halves, lane l of a wave finding its eight (row l % 16, columns
+// 8 (l / 16) .. + 8) at 8 l, so that a wave's operand load is one run of 1 KiB.
+// (Row after row, the load touched 64-byte pieces of 16 rows 2 kpad bytes apart:
+// the 2047-row Q4_K GEMMs of the Qwen3-0.6B shape took 51.0 us instead of 43.9.)
+// Rows are padded to a multiple of 16; the padding rows are never written and
+// only reach results that are dropped.
+constexpr int plane_rows(int rows) { return (rows + 15) / 16 * 16; }
+__host__ __device__ inline size_t plane_at(int row, int col, int kpad) {
+  return ((size_t)(row >> 4) * (kpad >> 5) + (col >> 5)) * 512 + ((col >> 3) & 3) * 128 + (row & 15) * 8 + (col & 7);
+}
 
 // K padded for the GEMM's activation planes.
 constexpr int gemm_kpad(int k) { return (k + 127) / 128 * 128; }
 
-size_t gemm_shared_bytes();
+// The GEMM over the weights' integer codes (gemm_int.hip): 16 ni weight rows x
+// 64 tj token rows per workgroup (ni 4 or 8, tj 1 or 2), a.ksplit and the output
+// as set by the caller. K splits are whole steps of gemm_int_step columns; types
+// with block offsets (gemm_int_sums) need a.xs.
+bool gemm_int_sums(int type);
+constexpr int gemm_int_step(int type) { return type == QT_Q4_K || type == QT_Q5_K || type == QT_Q6_K ? 256 : 128; }
+hipError_t launch_gemm_int(const GemmArgs& a, int n_rows, int ni, int tj, hipStream_t s);
+hipError_t init_gemm_int_attributes();
+// Whether a GEMM of `rows` token rows over a matrix of this type and K reads the
+// sums of x (GemmArgs.xs) beside the operand planes.
+bool gemm_needs_sums(int type, int k, int rows);
 hipError_t init_gemm_attributes();
 // Picks the K split for a launch (at least ~256 workgroups when the partial
 // buffer allows) and launches the GEMM and, when split, the ordered reduction.
@@ -160,6 +189,9 @@ hipError_t launch_gemm(const GemmArgs& a, hipStream_t s);
 // floats): the K split is chosen as in launch_gemm within the region, and no
 // reduction is launched; *out describes the partials for the consumer.
 hipError_t launch_gemm_deferred(const GemmArgs& a, float* region, int64_t region_cap, PartSum* out, hipStream_t s);
+// launch_gemm_deferred of gate | up (a.w, a.w2) leaving act(gate) * up; *out with
+// p null and nothing launched where the tiles would split K or have no instance.
+hipError_t launch_gemm_glu(const GemmArgs& a, float* region, int64_t region_cap, PartSum* out, hipStream_t s);
 hipError_t launch_pf_split(const PfSplitArgs& a, int rows, hipStream_t s);
 // Embedding rows times scale, plus (pos != null, GPT-2) the rows of the
 // position table from position p0 on.

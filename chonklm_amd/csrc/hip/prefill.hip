@@ -3,12 +3,12 @@
 // llama-wgsl-runtime.ts:276-289; the K/V it leaves in the cache and the last
 // prompt token's logits are what must match).
 //
-// Linear layers are dequant-fused GEMMs on the matrix cores. fp16 MFMA keeps
-// fp32-class accuracy by splitting both operands into hi + lo halves:
+// Linear layers are dequant-fused GEMMs on the matrix cores (gemm_int.hip; decode
+// batches of up to 64 rows below). fp16 MFMA keeps fp32-class accuracy by
+// splitting the operands into hi + lo halves:
 //   W * 2^ws = Wh + Wl,  x * 2^rs = xh + xl  (per token row),
 //   sum W x = 2^-(ws+rs) * (Wh xh + Wh xl + Wl xh)   (Wl xl ~ 2^-22, dropped)
-// with the weights dequantized bit-exactly (dequant_unit) into LDS tiles and
-// the products accumulated in fp32 by gfx950's v_mfma_f32_16x16x32_f16.
+// accumulated in fp32 by gfx950's v_mfma_f32_16x16x32_f16.
 #include <hip/hip_runtime.h>
 #include <cstdlib>
 #include <cstring>
@@ -24,15 +24,8 @@ namespace {
 
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
-
-constexpr int kGM = 64;          // weight rows per workgroup tile
-// token rows per workgroup tile: 128 for passes over 512 rows (each
-// dequantized weight stage serves more products), 64 up to 512 rows (twice the
-// tiles, so that short passes need no K split)
-__host__ __device__ constexpr int gemm_tokens(int tj) { return 64 * tj; }
-inline int gemm_tj(int rows) { return rows > 512 ? 2 : 1; }
-constexpr int kGK = 128;         // K per stage (whole units for every type)
-constexpr int kGS = kGK + 8;     // LDS row stride in halves (bank spread)
+typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 // gfx950's double-K shape: lane l holds row (or column) l % 16 and 8 consecutive
@@ -104,316 +97,252 @@ __device__ __forceinline__ void part_gather(const PartSum& P, int t, const int (
   part_finish<N>(P, t, j, w, v);
 }
 
-// The per-row glue kernels run one workgroup of kRowT threads per token row
-// (a batch of decode rows is a few dozen workgroups; wide ones keep each
-// row's deferred partial sums to one or two rounds of loads).
-constexpr int kRowT = 1024;
-constexpr int kRowW = kRowT / 64;
+// ---- per-row glue -----------------------------------------------------------------
+//
+// TPR threads of a 256-thread workgroup hold a token row in registers, E runs of
+// eight consecutive elements each (run c0 + TPR e is elements 8 (c0 + TPR e) ..
+// + 7): 16-byte loads and stores throughout, and the planes' 16-byte pieces are
+// written whole. With a wave per row (TPR = 64, passes of many rows) the four
+// rows of a workgroup write neighbouring pieces, and the row sums need no LDS or
+// barrier; short passes spread a row over two or four waves instead.
 
-// Row t of a deferred result, elements j0 + kRowT * e for e < E (zero past n),
-// four at a time.
-template <int E>
-__device__ __forceinline__ void part_row(const PartSum& P, int t, int j0, float (&v)[E]) {
-  static_assert(E % 4 == 0, "groups of four");
+template <int TPR>
+struct RowLane {
+  int t, c0, wave;  // token row (clamped), first run, wave of the workgroup
+  bool ok;          // false: past the last row (computes along, stores nothing)
+  __device__ __forceinline__ explicit RowLane(int rows) {
+    const int tid = threadIdx.x, r = (int)blockIdx.x * (kWg / TPR) + tid / TPR;
+    t = min(r, rows - 1);
+    c0 = tid % TPR;
+    wave = tid >> 6;
+    ok = r < rows;
+  }
+};
+
+template <int TPR, bool MAX>
+__device__ __forceinline__ float row_reduce(float v, const RowLane<TPR>& L, float* red) {
+  v = MAX ? wave_max(v) : wave_sum(v);
+  if constexpr (TPR > 64) {
+    constexpr int W = TPR / 64;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[L.wave] = v;
+    __syncthreads();
+    const float* r = red + L.wave / W * W;
+    v = r[0];
 #pragma unroll
-  for (int g = 0; g < E; g += 4) {
-    int j[4];
-    float w[4];
+    for (int w = 1; w < W; ++w) v = MAX ? fmaxf(v, r[w]) : v + r[w];
+  }
+  return v;
+}
+
+__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
+  const float4 a = ldg4f(p), b = ldg4f(p + 4);
+  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+  v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+}
+
+// 16-byte loads of the result's rows are aligned (uniform)
+__device__ __forceinline__ bool part_aligned(const PartSum& P) {
+  return ((P.ld | (int)P.zs) & 3) == 0 && ((uintptr_t)P.p & 15) == 0;
+}
+
+// Columns col .. col + 7 of row t of a deferred result, the splits added in
+// order, four splits' loads in flight (as part_gather).
+__device__ __forceinline__ void part8(const PartSum& P, bool vec, int t, int col, float (&v)[8]) {
+  const float* q = P.p + (int64_t)t * P.ld + col;
+  auto load = [&](int z, float (&w)[8]) {
+    const float* r = q + (int64_t)z * P.zs;
+    if (vec) {
+      load8(r, w);
+    } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) j[e] = min(j0 + kRowT * (g + e), P.n - 1);
-    part_gather<4>(P, t, j, w);
+      for (int i = 0; i < 8; ++i) w[i] = r[i];
+    }
+  };
+  load(0, v);
+  for (int z0 = 1; z0 < P.ks; z0 += 4) {
+    float w[4][8];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[g + e] = j0 + kRowT * (g + e) < P.n ? w[e] : 0.f;
+    for (int z = 0; z < 4; ++z) load(min(z0 + z, P.ks - 1), w[z]);
+#pragma unroll
+    for (int z = 0; z < 4; ++z)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = z0 + z < P.ks ? v[i] + w[z][i] : v[i];
   }
 }
 
-__device__ __forceinline__ float rowt_sum(float v, float* red) {
-  v = wave_sum(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float a = 0.f;
+// The row's runs of a deferred result from column 0 (zero past its columns).
+template <int TPR, int E>
+__device__ __forceinline__ void part_row(const PartSum& P, const RowLane<TPR>& L, float (&v)[E][8]) {
+  const bool vec = part_aligned(P);
 #pragma unroll
-  for (int w = 0; w < kRowW; w += 4) a += (red[w] + red[w + 1]) + (red[w + 2] + red[w + 3]);
-  return a;
-}
-__device__ __forceinline__ float rowt_max(float v, float* red) {
-  v = wave_max(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float a = 0.f;
+  for (int e = 0; e < E; ++e) {
+    const int col = 8 * (L.c0 + TPR * e);
+    part8(P, vec, L.t, min(col, P.n - 8), v[e]);
 #pragma unroll
-  for (int w = 0; w < kRowW; ++w) a = fmaxf(a, red[w]);
-  return a;
+    for (int i = 0; i < 8; ++i) v[e][i] = col < P.n ? v[e][i] : 0.f;
+  }
 }
 
-// ---- operand split ----------------------------------------------------------------
-
-// The row v (element threadIdx.x + kRowT * e of thread x is v[e], zero past the
-// row's end) scaled by a power of two so that |x| < 2^14 and split into fp16
-// hi + lo planes of kpad elements.
-template <int E>
-__device__ __forceinline__ void row_planes(const float (&v)[E], int t, int kpad, _Float16* xh, _Float16* xl,
-                                           float* xscale, float* red) {
-  const int tid = threadIdx.x;
+// The row v (zero past its end) scaled by a power of two so that |x| < 2^14 and
+// split into fp16 hi + lo planes of kpad columns; the sums of its 32-element
+// blocks (four threads each), which the block offsets of Q4_K weights multiply,
+// go to xs.
+template <int TPR, int E>
+__device__ __forceinline__ void row_planes(const float (&v)[E][8], const RowLane<TPR>& L, int kpad, _Float16* xh,
+                                           _Float16* xl, float* xscale, _Float16* xs, float* red) {
   float mx = 0.f;
 #pragma unroll
-  for (int e = 0; e < E; ++e) mx = fmaxf(mx, fabsf(v[e]));
-  mx = rowt_max(mx, red);
+  for (int e = 0; e < E; ++e)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(v[e][i]));
+  mx = row_reduce<TPR, true>(mx, L, red);
   int ex = 0;
   (void)frexpf(mx, &ex);  // mx < 2^ex
   const int rs = max(min(14 - ex, 60), -60);
-  xh += (size_t)t * kpad;
-  xl += (size_t)t * kpad;
+  const int nb = kpad / 32;
+  xs += (size_t)L.t * 2 * nb;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int i = tid + kRowT * e;
-    if (i < kpad) {
-      const float sv = ldexpf(v[e], rs);  // zero past the row's end
-      const _Float16 h = (_Float16)sv;
-      xh[i] = h;
-      xl[i] = (_Float16)(sv - (float)h);
+    const int col = 8 * (L.c0 + TPR * e);
+    half8_t h, l;
+    float bs = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float sv = ldexpf(v[e][i], rs);
+      h[i] = (_Float16)sv;
+      l[i] = (_Float16)(sv - (float)h[i]);
+      bs += sv;
+    }
+    bs = group_sum<4>(bs) * 0.03125f;
+    if (L.ok && col < kpad) {
+      const size_t at = plane_at(L.t, col, kpad);
+      *(half8_t*)(xh + at) = h;
+      *(half8_t*)(xl + at) = l;
+      if ((L.c0 & 3) == 0) {
+        const _Float16 bh = (_Float16)bs;
+        xs[col / 32] = bh;
+        xs[nb + col / 32] = (_Float16)(bs - (float)bh);
+      }
     }
   }
-  if (tid == 0) xscale[t] = __builtin_isfinite(mx) ? ldexpf(1.0f, -rs) : __int_as_float(0x7fc00000);
+  if (L.ok && L.c0 == 0) xscale[L.t] = __builtin_isfinite(mx) ? ldexpf(1.0f, -rs) : __int_as_float(0x7fc00000);
 }
 
 // x := (x * inv) * w with the reference's fp32 operation order (RMSNorm)
-template <int E>
-__device__ __forceinline__ void row_rmsnorm(float (&v)[E], const float* w, int k, float eps, float* red) {
+template <int TPR, int E>
+__device__ __forceinline__ void row_rmsnorm(float (&v)[E][8], const RowLane<TPR>& L, const float* w, int k, float eps,
+                                            float* red) {
   float ss = 0.f;
 #pragma unroll
-  for (int e = 0; e < E; ++e) ss += v[e] * v[e];
-  ss = rowt_sum(ss, red);
+  for (int e = 0; e < E; ++e)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss += v[e][i] * v[e][i];
+  ss = row_reduce<TPR, false>(ss, L, red);
   const float inv = 1.0f / sqrtf(ss / (float)k + eps);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int i = threadIdx.x + kRowT * e;
-    if (i < k) v[e] = __fmul_rn(__fmul_rn(v[e], inv), w[i]);
+    const int col = 8 * (L.c0 + TPR * e);
+    float wv[8];
+    load8(w + min(col, k - 8), wv);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[e][i] = __fmul_rn(__fmul_rn(v[e][i], inv), col < k ? wv[i] : 0.f);
   }
 }
 
-// One workgroup per token row: the pending residual update, an optional
-// RMSNorm (GPT: LayerNorm), then the operand planes. The row lives in
-// registers: E = 4 elements per thread serve rows of up to 4096, E = 8 (the
-// LFM2 and OpenELM feed-forward widths) up to kPfRowMax.
-template <int E, bool GPT>
-__global__ __launch_bounds__(kRowT) void k_pf_split(PfSplitArgs a) {
-  warm_kernarg<(int)(sizeof(PfSplitArgs))>();  // (dependent argument rounds hit the scalar cache)
-  __shared__ float red[kRowW];
-  const int t = blockIdx.x, tid = threadIdx.x;
-  float* xw = const_cast<float*>(a.x + (size_t)t * a.ldx);
-  float v[E];
+// The pending residual update of a token row, an optional RMSNorm (GPT:
+// LayerNorm), then the operand planes.
+template <int TPR, int E, bool GPT>
+__global__ __launch_bounds__(kWg) void k_pf_split(PfSplitArgs a, int rows) {
+  warm_kernarg<(int)(sizeof(PfSplitArgs) + 8)>();  // (dependent argument rounds hit the scalar cache)
+  __shared__ float red[4];
+  const RowLane<TPR> L(rows);
+  float* xw = const_cast<float*>(a.x + (size_t)L.t * a.ldx);
+  float v[E][8];
 #pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = xw[min(tid + kRowT * e, a.k - 1)];  // unconditional (no branch)
+  for (int e = 0; e < E; ++e) load8(xw + min(8 * (L.c0 + TPR * e), a.k - 8), v[e]);
 #pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = tid + kRowT * e < a.k ? v[e] : 0.f;
+  for (int e = 0; e < E; ++e)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[e][i] = 8 * (L.c0 + TPR * e) < a.k ? v[e][i] : 0.f;
   if (a.add.p) {
-    float d[E];
-    part_row<E>(a.add, t, tid, d);
-    if (GPT) {
+    float d[E][8];
+    part_row<TPR, E>(a.add, L, d);
+    if constexpr (GPT) {
       // bias, residual add, SANITIZE (gpt-wgsl-runtime.ts:1708-1746)
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        const int i = tid + kRowT * e;
-        if (i < a.k) {
-          const float y = __fadd_rn(v[e], __fadd_rn(d[e], a.add_bias[i]));
-          v[e] = y != y ? 0.0f : fminf(fmaxf(y, -10000.0f), 10000.0f);
+        const int col = 8 * (L.c0 + TPR * e);
+        float b[8];
+        load8(a.add_bias + min(col, a.k - 8), b);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float y = __fadd_rn(v[e][i], __fadd_rn(d[e][i], b[i]));
+          v[e][i] = col >= a.k || y != y ? 0.0f : fminf(fmaxf(y, -10000.0f), 10000.0f);
         }
       }
     } else if (a.add_w) {
       // the branch output goes through RMSNorm first (the Gemma-3 sandwich)
-      row_rmsnorm<E>(d, a.add_w, a.k, a.eps, red);
+      row_rmsnorm<TPR, E>(d, L, a.add_w, a.k, a.eps, red);
 #pragma unroll
       for (int e = 0; e < E; ++e)
-        if (tid + kRowT * e < a.k) v[e] = fminf(fmaxf(__fadd_rn(v[e], d[e]), -65000.0f), 65000.0f);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[e][i] = fminf(fmaxf(__fadd_rn(v[e][i], d[e][i]), -65000.0f), 65000.0f);
     } else {
 #pragma unroll
-      for (int e = 0; e < E; ++e) v[e] = __fadd_rn(v[e], a.add_scale != 0.f ? __fmul_rn(d[e], a.add_scale) : d[e]);
+      for (int e = 0; e < E; ++e)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          v[e][i] = __fadd_rn(v[e][i], a.add_scale != 0.f ? __fmul_rn(d[e][i], a.add_scale) : d[e][i]);
     }
     // the updated residual row
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int i = tid + kRowT * e;
-      if (i < a.k) xw[i] = v[e];
+      const int col = 8 * (L.c0 + TPR * e);
+      if (L.ok && col < a.k) {
+        *(float4*)(xw + col) = make_float4(v[e][0], v[e][1], v[e][2], v[e][3]);
+        *(float4*)(xw + col + 4) = make_float4(v[e][4], v[e][5], v[e][6], v[e][7]);
+      }
     }
   }
-  if (GPT) {
+  if constexpr (GPT) {
     if (a.w) {
       // LAYER_NORM_WGSL (gpt-wgsl-runtime.ts:1658-1706): mean and E[x^2] in one
       // pass, variance max(E[x^2] - mean^2, 0), ((x - mean) * inv_std) * w + b
       float sm = 0.f, sq = 0.f;
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        sm += v[e];
-        sq += v[e] * v[e];
-      }
-      sm = rowt_sum(sm, red);
-      sq = rowt_sum(sq, red);
+      for (int e = 0; e < E; ++e)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          sm += v[e][i];
+          sq += v[e][i] * v[e][i];
+        }
+      sm = row_reduce<TPR, false>(sm, L, red);
+      sq = row_reduce<TPR, false>(sq, L, red);
       const float mean = sm / (float)a.k;
       const float var = fmaxf(__fsub_rn(sq / (float)a.k, __fmul_rn(mean, mean)), 0.0f);
       const float inv = 1.0f / sqrtf(var + a.eps);
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        const int i = tid + kRowT * e;
-        if (i < a.k) v[e] = __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[e], mean), inv), a.w[i]), a.norm_b[i]);
+        const int col = 8 * (L.c0 + TPR * e);
+        float w[8], b[8];
+        load8(a.w + min(col, a.k - 8), w);
+        load8(a.norm_b + min(col, a.k - 8), b);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          v[e][i] = col < a.k ? __fadd_rn(__fmul_rn(__fmul_rn(__fsub_rn(v[e][i], mean), inv), w[i]), b[i]) : 0.f;
       }
     }
   } else if (a.w) {
-    row_rmsnorm<E>(v, a.w, a.k, a.eps, red);
+    row_rmsnorm<TPR, E>(v, L, a.w, a.k, a.eps, red);
   }
-  row_planes<E>(v, t, a.kpad, a.xh, a.xl, a.xscale, red);
-}
-
-// ---- dequant-fused GEMM ----------------------------------------------------------
-
-// y[t][n] (=|+=) sum_k x[t][k] W[n][k] for a kGM x 64 TJ tile. The tile's
-// weights are dequantized once per stage into LDS (fp16 hi + lo of W * 2^ws)
-// and serve 64 TJ token rows; wave w owns token rows 16 TJ w .. 16 TJ (w + 1) - 1
-// against all 64 weight rows (4 x TJ MFMA tiles of 16 x 16, three products each) and
-// reads its activation operands straight from the planes (each element is
-// read by one lane of one wave, so staging them through LDS would only add a
-// copy). With only the weights in LDS (35 KB) the registers bound the
-// workgroups per CU: at TJ = 2 three for the Q4_K instance, two for Q6_K.
-template <int T, int TJ>
-__global__ __launch_bounds__(kWg) void k_gemm(GemmArgs a) {
-  extern __shared__ __align__(16) _Float16 gsm[];
-  _Float16* wh = gsm;
-  _Float16* wl = wh + kGM * kGS;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * kGM, t0 = blockIdx.y * gemm_tokens(TJ);
-  const int N = a.n_all ? a.n_all : a.w.n;
-  // the tile's matrix of a fused launch (segments start on tile boundaries)
-  const int seg = a.n_all ? (n0 >= a.n2 ? 2 : (n0 >= a.n1 ? 1 : 0)) : 0;
-  const int sb = seg == 2 ? a.n2 : (seg == 1 ? a.n1 : 0);
-  // picked field by field (a selected struct copy would live in scratch)
-  QMat wm = a.w;
-#define CHONK_PICK_W(f) wm.f = seg == 2 ? a.w3.f : (seg == 1 ? a.w2.f : a.w.f)
-  CHONK_PICK_W(s0);
-  CHONK_PICK_W(s1);
-  CHONK_PICK_W(s2);
-  CHONK_PICK_W(s3);
-  CHONK_PICK_W(n);
-#undef CHONK_PICK_W
-  const int U = a.w.k >> 5;
-  const int nst = (a.w.k + kGK - 1) / kGK;
-  // this workgroup's stages: part blockIdx.z of ksplit
-  const int s_lo = (int)((int64_t)nst * blockIdx.z / a.ksplit);
-  const int s_hi = (int)((int64_t)nst * (blockIdx.z + 1) / a.ksplit);
-  // staging role: weight unit (row wr, unit j of the stage)
-  const int wr = tid >> 2, wj = tid & 3;
-  const bool w_ok = n0 + wr < N;
-  const float wsc = ldexpf(1.0f, a.ws);
-  // operand role: lane l holds row (or token) l % 16 and k 8 (l / 16) .. + 8 of a 32-k step
-  const int col = lane & 15, kq = (lane >> 4) * 8;
-  // the lane's plane rows as 32-bit byte offsets from the planes' (uniform)
-  // bases; a token row past t reads row t - 1: its products are computed and
-  // dropped (the launcher checks that a plane fits 32-bit offsets)
-  uint32_t xo[TJ];
-#pragma unroll
-  for (int j = 0; j < TJ; ++j)
-    xo[j] = 2u * ((uint32_t)min(t0 + 16 * (TJ * wave + j) + col, a.t - 1) * (uint32_t)a.kpad + (uint32_t)kq);
-  const char* xhb = (const char*)a.xh;
-  const char* xlb = (const char*)a.xl;
-
-  float4_t acc[4][TJ];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-  Frag<T> f{};
-  auto fetch_w = [&](int st) {
-    const int u = st * 4 + wj;
-    if (w_ok && u < U) f = load_unit<T>(wm, n0 - sb + wr, u);
-  };
-  fetch_w(s_lo);
-  for (int s = s_lo; s < s_hi; ++s) {
-    // this stage's activation operands (awaited after the weight staging)
-    half8_t bh[kGK / 32][TJ], bl[kGK / 32][TJ];
-#pragma unroll
-    for (int ks = 0; ks < kGK / 32; ++ks)
-#pragma unroll
-      for (int j = 0; j < TJ; ++j) {
-        const uint32_t o = xo[j] + 2u * (uint32_t)(s * kGK + ks * 32);
-        bh[ks][j] = *(const half8_t*)(xhb + o);
-        bl[ks][j] = *(const half8_t*)(xlb + o);
-      }
-    // weights: the unit's 32 values at their K offsets, hi and lo
-    const int u = s * 4 + wj;
-    float v[32];
-    if (w_ok && u < U) {
-      dequant_unit<T>(f, u, v, wsc);  // W * 2^ws (the unit's factors scaled: exact)
-    } else {
-#pragma unroll
-      for (int e = 0; e < 32; ++e) v[e] = 0.f;
-    }
-    // the next stage's unit goes out as soon as this one is decoded (the last
-    // stage requests itself again rather than branching on the stage index)
-    fetch_w(min(s + 1, s_hi - 1));
-    __syncthreads();  // the previous stage's tile is consumed
-    _Float16* rh = wh + wr * kGS;
-    _Float16* rl = wl + wr * kGS;
-#pragma unroll
-    for (int e = 0; e < 32; e += 4) {
-      const int kk = (u < U ? unit_col<T>(u, e) : 32 * u + e) - s * kGK;
-      half4_t h, l;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float sv = v[e + i];
-        h[i] = (_Float16)sv;
-        l[i] = (_Float16)(sv - (float)h[i]);
-      }
-      *(half4_t*)(rh + kk) = h;
-      *(half4_t*)(rl + kk) = l;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < kGK / 32; ++ks) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const half8_t ah = *(const half8_t*)(wh + (16 * i + col) * kGS + ks * 32 + kq);
-        const half8_t al = *(const half8_t*)(wl + (16 * i + col) * kGS + ks * 32 + kq);
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-          acc[i][j] = mfma32(ah, bh[ks][j], acc[i][j]);
-          acc[i][j] = mfma32(ah, bl[ks][j], acc[i][j]);
-          acc[i][j] = mfma32(al, bh[ks][j], acc[i][j]);
-        }
-      }
-    }
-  }
-  // lane holds rows 4 * (lane / 16) + 0..3 of each row tile, token lane % 16
-  const float wun = ldexpf(1.0f, -a.ws);
-#pragma unroll
-  for (int j = 0; j < TJ; ++j) {
-    const int tt = t0 + 16 * (TJ * wave + j) + col;
-    if (tt >= a.t) continue;
-    const float sc = wun * a.xscale[tt];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int n = n0 + 16 * i + 4 * (lane >> 4);
-      float* y = a.y + (size_t)tt * a.ldy + n;
-      float* pp = a.part + ((size_t)blockIdx.z * a.t + tt) * N + n;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (n + q >= N) break;
-        const float v = acc[i][j][q] * sc;
-        if (a.ksplit > 1 || a.defer)
-          pp[q] = v;
-        else
-          y[q] = a.epi == GEMM_ADD ? __fadd_rn(y[q], v) : v;
-      }
-    }
-  }
+  row_planes<TPR, E>(v, L, a.kpad, a.xh, a.xl, a.xscale, a.xs, red);
 }
 
 // ---- decode-batch GEMM (at most 64 token rows) ------------------------------------
 //
 // With 64 or fewer token rows the GEMM streams weights: every weight is used
-// by at most 64 products, so staging dequantized tiles through LDS (k_gemm)
+// by at most 64 products, so staging weight tiles through LDS (k_gemm_int)
 // costs more than the products. Here each wave owns 64 weight rows x all 64
 // token rows over a quarter of the workgroup's K range, with no LDS for the
 // operands: the x planes are loaded straight into MFMA A operands (lane l:
@@ -553,11 +482,11 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk(GemmArgs a) {
   int rows[4];
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) rows[rt] = min(n0 + 16 * rt + r16, N - 1) - sb0;
-  // token rows of the lane's A operands, clamped: rows past a.t load a valid row
-  // and their sums are never written
-  int xrow[4];
+  // the lane's piece of each token tile's A operands; a tile past a.t loads the
+  // last one and its sums are never written
+  size_t xo[4];
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt) xrow[tt] = min(16 * tt + r16, a.t - 1);
+  for (int tt = 0; tt < 4; ++tt) xo[tt] = plane_at(16 * min(tt, (a.t - 1) / 16), 0, a.kpad) + 8 * lane;
   // the epilogue's operand scales, requested up front (read from LDS at the end)
   if (tid < a.t) ssm[4 * 64 * kSkRows + tid] = a.xscale[tid];
 
@@ -581,11 +510,11 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk(GemmArgs a) {
     for (int rt = 0; rt < 4; ++rt) nxt[rt] = sk_load<T>(wm, rows[rt], bn, g);
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
-      const int k0 = sk_col<T>(blk, s2) + 8 * g;  // this lane's 8 k of the step
+      const int k0 = sk_col<T>(blk, s2);
       half8_t ah[4], al[4];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {
-        const size_t off = (size_t)xrow[tt] * a.kpad + k0;
+        const size_t off = xo[tt] + 16 * k0;  // (512 halves per 32 columns)
         ah[tt] = *gbl((const half8_t*)(a.xh + off));
         al[tt] = *gbl((const half8_t*)(a.xl + off));
       }
@@ -665,19 +594,17 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
   const int blk = (int)blockIdx.z * 4 + wave;
   _Float16* xw = (_Float16*)ssm + (size_t)wave * (2 * 2 * 64 * 32);  // this wave's x operands
   float* xs = ssm + 4 * 64 * kSkRed;                                 // the token rows' operand scales
-  // x: 16 copies of 1 KiB (16 tokens x 64 bytes each); lane l moves token
-  // 16 i + l / 4, piece l % 4 (token rows past a.t repeat the last row: their
-  // sums are never written)
+  // x: 16 copies of 1 KiB (a token tile's 32 columns, in operand order; tiles
+  // past a.t repeat the last one: their sums are never written)
   {
-    const int tok = lane >> 2, pc = lane & 3;
 #pragma unroll
     for (int p = 0; p < 2; ++p)
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int t = min(16 * i + tok, a.t - 1);
-          const _Float16* src = (p ? a.xl : a.xh) + (size_t)t * a.kpad + sk_col<T>(blk, s2) + 8 * pc;
+          const _Float16* src =
+              (p ? a.xl : a.xh) + plane_at(16 * min(i, (a.t - 1) / 16), sk_col<T>(blk, s2), a.kpad) + 8 * lane;
           __builtin_amdgcn_global_load_lds((gmem_void*)src, (lds_void*)(xw + ((p * 2 + s2) * 64 + 16 * i) * 32), 16,
                                            0, 0);
         }
@@ -699,8 +626,8 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
     half8_t ah[4], al[4];
 #pragma unroll
     for (int tt = 0; tt < 4; ++tt) {
-      ah[tt] = *(const half8_t*)(xw + ((0 * 2 + s2) * 64 + 16 * tt + r16) * 32 + 8 * g);
-      al[tt] = *(const half8_t*)(xw + ((1 * 2 + s2) * 64 + 16 * tt + r16) * 32 + 8 * g);
+      ah[tt] = *(const half8_t*)(xw + ((0 * 2 + s2) * 64 + 16 * tt) * 32 + 8 * lane);
+      al[tt] = *(const half8_t*)(xw + ((1 * 2 + s2) * 64 + 16 * tt) * 32 + 8 * lane);
     }
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
@@ -784,13 +711,12 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) rows[rt] = min(n0 + 16 * rt + r16, N - 1);
   // x of block b into buffer b & 1: this wave's four of its sixteen 1-KiB copies
-  const int tok = lane >> 2, pc = lane & 3;
   auto copy_x = [&](int b) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int c = wave * 4 + j, p = c >> 3, s2 = (c >> 2) & 1, i = c & 3;
-      const int t = min(16 * i + tok, a.t - 1);
-      const _Float16* src = (p ? a.xl : a.xh) + (size_t)t * a.kpad + sk_col<T>(b, s2) + 8 * pc;
+      const _Float16* src =
+          (p ? a.xl : a.xh) + plane_at(16 * min(i, (a.t - 1) / 16), sk_col<T>(b, s2), a.kpad) + 8 * lane;
       __builtin_amdgcn_global_load_lds((gmem_void*)src,
                                        (lds_void*)(xb + (((b & 1) * 4 + p * 2 + s2) * 64 + 16 * i) * 32), 16, 0, 0);
     }
@@ -829,8 +755,8 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
       half8_t ah[4], al[4];
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {
-        ah[tt] = *(const half8_t*)(xc + ((0 * 2 + s2) * 64 + 16 * tt + r16) * 32 + 8 * g);
-        al[tt] = *(const half8_t*)(xc + ((1 * 2 + s2) * 64 + 16 * tt + r16) * 32 + 8 * g);
+        ah[tt] = *(const half8_t*)(xc + ((0 * 2 + s2) * 64 + 16 * tt) * 32 + 8 * lane);
+        al[tt] = *(const half8_t*)(xc + ((1 * 2 + s2) * 64 + 16 * tt) * 32 + 8 * lane);
       }
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
@@ -878,14 +804,14 @@ size_t gemm_lm_shared_bytes() { return sizeof(_Float16) * 2 * (2 * 2 * 64 * 32) 
 size_t gemm_sk_shared_bytes() { return sizeof(float) * (4 * 64 * kSkRed + 64); }
 
 // The decode-batch GEMM applies: at most 64 token rows and a K-quant type it covers.
-bool gemm_sk_applies(const GemmArgs& a) {
+bool gemm_sk_applies(int type, int k, int rows) {
   static const bool off = [] {
     const char* v = std::getenv("CHONK_GEMM");
     return v && std::strcmp(v, "tiles") == 0;
   }();
-  return !off && a.t >= 1 && a.t <= 64 && (a.w.type == QT_Q4_K || a.w.type == QT_Q6_K) && a.w.k % 256 == 0 &&
-         a.kpad >= a.w.k;
+  return !off && rows >= 1 && rows <= 64 && (type == QT_Q4_K || type == QT_Q6_K) && k % 256 == 0;
 }
+bool gemm_sk_applies(const GemmArgs& a) { return gemm_sk_applies(a.w.type, a.w.k, a.t) && a.kpad >= a.w.k; }
 
 // K split of a decode-batch GEMM: about 256 workgroups (one per CU), at least
 // one block per wave.
@@ -958,30 +884,37 @@ __global__ __launch_bounds__(kWg) void k_pf_norm_add(const float* d, const float
   }
 }
 
-// silu(g) * u, gelu_tanh(g) * u or (GPT-2) gelu_tanh(u + bias) per element, then
-// the operand planes (one workgroup per token row; E as for k_pf_split).
-template <int E>
-__global__ __launch_bounds__(kRowT) void k_pf_glu_split(PfGluArgs a) {
-  warm_kernarg<(int)(sizeof(PfGluArgs))>();  // (dependent argument rounds hit the scalar cache)
-  __shared__ float red[kRowW];
-  const int t = blockIdx.x, tid = threadIdx.x;
-  float gv[E], uv[E], v[E];
+// silu(g) * u, gelu_tanh(g) * u or (GPT-2) gelu_tanh(u + bias) per element (or
+// that product as the GEMM left it), then the operand planes.
+template <int TPR, int E>
+__global__ __launch_bounds__(kWg) void k_pf_glu_split(PfGluArgs a, int rows) {
+  warm_kernarg<(int)(sizeof(PfGluArgs) + 8)>();  // (dependent argument rounds hit the scalar cache)
+  __shared__ float red[4];
+  const RowLane<TPR> L(rows);
+  float gv[E][8], v[E][8];
+  if (a.act == PF_DONE) {
+    part_row<TPR, E>(a.pu, L, v);
+    row_planes<TPR, E>(v, L, a.kpad, a.xh, a.xl, a.xscale, a.xs, red);
+    return;
+  }
   if (a.act != PF_GELU_BIAS) {
-    part_row<E>(a.pg, t, tid, gv);
+    part_row<TPR, E>(a.pg, L, gv);
   } else {
 #pragma unroll
-    for (int e = 0; e < E; ++e) gv[e] = a.bias[min(tid + kRowT * e, a.k - 1)];
+    for (int e = 0; e < E; ++e) load8(a.bias + min(8 * (L.c0 + TPR * e), a.k - 8), gv[e]);
   }
-  part_row<E>(a.pu, t, tid, uv);
+  part_row<TPR, E>(a.pu, L, v);
 #pragma unroll
-  for (int e = 0; e < E; ++e) {
-    v[e] = 0.f;
-    if (tid + kRowT * e < a.k)
-      v[e] = a.act == PF_SWIGLU  ? silu_mul(gv[e], uv[e])
-             : a.act == PF_GEGLU ? __fmul_rn(gelu_tanh(gv[e]), uv[e])
-                                 : gelu_tanh(__fadd_rn(uv[e], gv[e]));
-  }
-  row_planes<E>(v, t, a.kpad, a.xh, a.xl, a.xscale, red);
+  for (int e = 0; e < E; ++e)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float g = gv[e][i], u = v[e][i];
+      const float y = a.act == PF_SWIGLU  ? silu_mul(g, u)
+                      : a.act == PF_GEGLU ? __fmul_rn(gelu_tanh(g), u)
+                                          : gelu_tanh(__fadd_rn(u, g));
+      v[e][i] = 8 * (L.c0 + TPR * e) < a.k ? y : 0.f;
+    }
+  row_planes<TPR, E>(v, L, a.kpad, a.xh, a.xl, a.xscale, a.xs, red);
 }
 
 // ---- lfm2 short convolution ---------------------------------------------------------
@@ -989,52 +922,45 @@ __global__ __launch_bounds__(kRowT) void k_pf_glu_split(PfGluArgs a) {
 // C * (bx[t-2] w0 + bx[t-1] w1 + bx[t] w2) of every channel (CONV_BLOCK_WGSL,
 // lfm-wgsl-runtime.ts:1641-1672, each product and sum rounded as the decode
 // prologue does), bx = B * x of the in_proj rows, the two rows before the pass
-// from the state; then the operand planes. One workgroup per token row.
-template <int E>
-__global__ __launch_bounds__(kRowT) void k_pf_conv(PfConvArgs a) {
-  warm_kernarg<(int)(sizeof(PfConvArgs))>();
-  __shared__ float red[kRowW];
-  const int t = blockIdx.x, tid = threadIdx.x;
-  float v[E];
+// from the state; then the operand planes.
+template <int TPR, int E>
+__global__ __launch_bounds__(kWg) void k_pf_conv(PfConvArgs a, int rows) {
+  warm_kernarg<(int)(sizeof(PfConvArgs) + 8)>();
+  __shared__ float red[4];
+  const RowLane<TPR> L(rows);
+  const bool vec = part_aligned(a.p) && (a.k & 3) == 0;
+  const int t = L.t;
+  float v[E][8];
 #pragma unroll
-  for (int g = 0; g < E; g += 4) {
-    int i[4], j[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) i[e] = min(tid + kRowT * (g + e), a.k - 1);
-    auto part = [&](int row, int piece, float (&w)[4]) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) j[e] = piece * a.k + i[e];
-      part_gather<4>(a.p, row, j, w);
-    };
-    float b[4], x[4], c[4], p1[4], p2[4];
-    part(max(t - 2, 0), 0, b);
-    part(max(t - 2, 0), 2, x);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) p1[e] = __fmul_rn(b[e], x[e]);
-    part(max(t - 1, 0), 0, b);
-    part(max(t - 1, 0), 2, x);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) p2[e] = __fmul_rn(b[e], x[e]);
-    part(t, 0, b);
-    part(t, 2, x);
-    part(t, 1, c);
-    if (t < 2) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) p1[e] = t == 0 ? a.s1[i[e]] : a.s2[i[e]];
-      if (t == 0) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) p2[e] = a.s2[i[e]];
+  for (int e = 0; e < E; ++e) {
+    const int col = min(8 * (L.c0 + TPR * e), a.k - 8);
+    // B * x of row r, or of a row before the pass
+    auto bx = [&](int r, float (&w)[8]) {
+      if (r < 0) {
+        load8((r == -2 ? a.s1 : a.s2) + col, w);
+        return;
       }
-    }
+      float b[8];
+      part8(a.p, vec, r, col, b);
+      part8(a.p, vec, r, 2 * a.k + col, w);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float* w = a.w + 3 * (size_t)i[e];
-      const float y = __fadd_rn(__fadd_rn(__fmul_rn(p1[e], w[0]), __fmul_rn(p2[e], w[1])),
-                                __fmul_rn(__fmul_rn(b[e], x[e]), w[2]));
-      v[g + e] = tid + kRowT * (g + e) < a.k ? __fmul_rn(c[e], y) : 0.f;
+      for (int i = 0; i < 8; ++i) w[i] = __fmul_rn(b[i], w[i]);
+    };
+    float p1[8], p2[8], p3[8], c[8], w[24];
+    bx(t - 2, p1);
+    bx(t - 1, p2);
+    bx(t, p3);
+    part8(a.p, vec, t, a.k + col, c);
+#pragma unroll
+    for (int i = 0; i < 24; ++i) w[i] = a.w[3 * (size_t)col + i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float y = __fadd_rn(__fadd_rn(__fmul_rn(p1[i], w[3 * i]), __fmul_rn(p2[i], w[3 * i + 1])),
+                                __fmul_rn(p3[i], w[3 * i + 2]));
+      v[e][i] = 8 * (L.c0 + TPR * e) < a.k ? __fmul_rn(c[i], y) : 0.f;
     }
   }
-  row_planes<E>(v, t, a.kpad, a.xh, a.xl, a.xscale, red);
+  row_planes<TPR, E>(v, L, a.kpad, a.xh, a.xl, a.xscale, a.xs, red);
 }
 
 // s1, s2 = bx of the pass's last two rows (a launch of its own: k_pf_conv's
@@ -1205,20 +1131,22 @@ __global__ __launch_bounds__(kWg) void k_pf_mamba_scan(PfMambaArgs a) {
 
 // MAMBA_GATE_NORM_WGSL (granite-wgsl-runtime.ts:1590-1606) of every row, then
 // the operand planes of out_proj.
-template <int E>
-__global__ __launch_bounds__(kRowT) void k_pf_gate(PfGateArgs a) {
-  warm_kernarg<(int)(sizeof(PfGateArgs))>();
-  __shared__ float red[kRowW];
-  const int t = blockIdx.x, tid = threadIdx.x;
-  float v[E], z[E];
+template <int TPR, int E>
+__global__ __launch_bounds__(kWg) void k_pf_gate(PfGateArgs a, int rows) {
+  warm_kernarg<(int)(sizeof(PfGateArgs) + 8)>();
+  __shared__ float red[4];
+  const RowLane<TPR> L(rows);
+  float v[E][8], z[E][8];
 #pragma unroll
-  for (int e = 0; e < E; ++e) v[e] = a.y[(size_t)t * a.k + min(tid + kRowT * e, a.k - 1)];
-  part_row<E>(a.z, t, tid, z);
+  for (int e = 0; e < E; ++e) load8(a.y + (size_t)L.t * a.k + min(8 * (L.c0 + TPR * e), a.k - 8), v[e]);
+  part_row<TPR, E>(a.z, L, z);
 #pragma unroll
   for (int e = 0; e < E; ++e)
-    v[e] = tid + kRowT * e < a.k ? __fmul_rn(v[e], __fdiv_rn(z[e], __fadd_rn(1.0f, expf(-z[e])))) : 0.f;
-  row_rmsnorm<E>(v, a.w, a.k, a.eps, red);
-  row_planes<E>(v, t, a.kpad, a.xh, a.xl, a.xscale, red);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      v[e][i] = 8 * (L.c0 + TPR * e) < a.k ? __fmul_rn(v[e][i], __fdiv_rn(z[e][i], __fadd_rn(1.0f, expf(-z[e][i])))) : 0.f;
+  row_rmsnorm<TPR, E>(v, L, a.w, a.k, a.eps, red);
+  row_planes<TPR, E>(v, L, a.kpad, a.xh, a.xl, a.xscale, a.xs, red);
 }
 
 __device__ __forceinline__ int row_pos(const KvAddr& k, int t) { return k.row_pos ? k.row_pos[t] : k.p0 + t; }
@@ -1228,6 +1156,12 @@ __device__ __forceinline__ size_t kv_row(const KvAddr& k, int kv_heads, int hd, 
   if (!k.pages) return ((size_t)kv * k.ctx + pos) * hd;
   const int page = k.pages[(size_t)seq * k.max_pages + pos / kKvPage];
   return (((size_t)page * kv_heads + kv) * kKvPage + (pos & (kKvPage - 1))) * hd;
+}
+
+// (cos, sin) of rotary pair d at a position.
+__device__ __forceinline__ float2 rope_cs(const PfRopeArgs& a, int pos, int d, int half) {
+  const float ang = __fmul_rn((float)pos, a.rope_inv[d]);
+  return make_float2(cosf(ang), sinf(ang));
 }
 
 // Per-head q/k RMSNorm and rotary embedding of every prompt row (position
@@ -1253,11 +1187,13 @@ __global__ __launch_bounds__(kWg) void k_pf_rope_kv(PfRopeArgs a) {
   const int pcol = is_k ? kv * hd : hh * hd;                 // ... in its projection's result
   int ia[NP], ib[NP];
   float x0[NP], x1[NP];
+  float2 cs[NP];
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
     const int d = min(lane + 64 * j, half - 1);
     ia[j] = a.interleaved ? 2 * d : d;
     ib[j] = a.interleaved ? 2 * d + 1 : d + half;
+    cs[j] = rope_cs(a, pos, d, half);
   }
   if (P.p) {
     // both elements of every pair in one round of loads
@@ -1309,8 +1245,7 @@ __global__ __launch_bounds__(kWg) void k_pf_rope_kv(PfRopeArgs a) {
       v0 = __fmul_rn(__fmul_rn(v0, r), w[ia[j]]);
       v1 = __fmul_rn(__fmul_rn(v1, r), w[ib[j]]);
     }
-    const float ang = __fmul_rn((float)pos, a.rope_inv[d]);
-    const float co = cosf(ang), si = sinf(ang);
+    const float co = cs[j].x, si = cs[j].y;
     const float y0 = __fsub_rn(__fmul_rn(v0, co), __fmul_rn(v1, si));
     const float y1 = __fadd_rn(__fmul_rn(v0, si), __fmul_rn(v1, co));
     if (is_k) {
@@ -1901,8 +1836,8 @@ __global__ __launch_bounds__(kWg) void k_bd_walk(PfAttnArgs a, float* part, int 
           v0 = __fmul_rn(__fmul_rn(v0, rn), w[ia[j]]);
           v1 = __fmul_rn(__fmul_rn(v1, rn), w[ib[j]]);
         }
-        const float ang = __fmul_rn((float)pos, ra.rope_inv[d]);
-        const float co = cosf(ang), si = sinf(ang);
+        const float2 cs = rope_cs(ra, pos, d, HALF);
+        const float co = cs.x, si = cs.y;
         const float y0 = __fsub_rn(__fmul_rn(v0, co), __fmul_rn(v1, si));
         const float y1 = __fadd_rn(__fmul_rn(v0, si), __fmul_rn(v1, co));
         if (is_k) {
@@ -1984,8 +1919,9 @@ __global__ __launch_bounds__(kWg) void k_bd_walk(PfAttnArgs a, float* part, int 
           // spacing 2^-24), so the relative error grows to ~2^-24 / |y|
           // (2^-17 at 0.01, 2^-14 at 1e-3), still far inside the 1e-3 logits bar
           const _Float16 h = (_Float16)y;
-          a.oh[(size_t)r * a.okpad + i] = h;
-          a.ol[(size_t)r * a.okpad + i] = (_Float16)(y - (float)h);
+          const size_t at = plane_at(r, (int)i, a.okpad);
+          a.oh[at] = h;
+          a.ol[at] = (_Float16)(y - (float)h);
         } else {
           a.out[(size_t)r * a.ldo + i] = y;
         }
@@ -1994,8 +1930,8 @@ __global__ __launch_bounds__(kWg) void k_bd_walk(PfAttnArgs a, float* part, int 
     if (a.oh && kv == 0) {
       // the planes past the row's last column are zero; its scale is 1
       for (int i = a.heads * HD + tid; i < a.okpad; i += kWg) {
-        a.oh[(size_t)r * a.okpad + i] = (_Float16)0.f;
-        a.ol[(size_t)r * a.okpad + i] = (_Float16)0.f;
+        a.oh[plane_at(r, i, a.okpad)] = (_Float16)0.f;
+        a.ol[plane_at(r, i, a.okpad)] = (_Float16)0.f;
       }
       if (tid == 0) a.oscale[r] = 1.0f;
     }
@@ -2115,37 +2051,42 @@ __global__ __launch_bounds__(64) void k_row_argmax2(const float* pv, const uint3
 
 // ---- host launchers ----------------------------------------------------------------
 
-size_t gemm_shared_bytes() { return sizeof(_Float16) * (size_t)(2 * kGM) * kGS; }
+bool gemm_needs_sums(int type, int k, int rows) { return gemm_int_sums(type) && !gemm_sk_applies(type, k, rows); }
 
-// k_gemm addresses the activation planes with 32-bit byte offsets
-bool gemm_planes_fit(const GemmArgs& a) { return a.t >= 1 && (int64_t)a.t * a.kpad * 2 <= (int64_t)UINT32_MAX; }
-
-// k_gemm<type, tj> on the stream; false for a type without an instance
-bool launch_gemm_tiles(const GemmArgs& a, int tj, dim3 grid, hipStream_t s) {
-  const size_t sh = gemm_shared_bytes();
-#define CHONK_GEMM_CASE(QT)                                                 \
-  case QT:                                                                  \
-    if (tj == 2)                                                            \
-      hipLaunchKernelGGL((k_gemm<QT, 2>), grid, dim3(kWg), sh, s, a);       \
-    else                                                                    \
-      hipLaunchKernelGGL((k_gemm<QT, 1>), grid, dim3(kWg), sh, s, a);       \
-    return true;
-  switch (a.w.type) {
-    CHONK_GEMM_CASE(QT_Q4_K)
-    CHONK_GEMM_CASE(QT_Q5_K)
-    CHONK_GEMM_CASE(QT_Q6_K)
-    CHONK_GEMM_CASE(QT_Q8_0)
-    CHONK_GEMM_CASE(QT_Q5_0)
-    CHONK_GEMM_CASE(QT_Q5_1)
-    default: return false;
-  }
-#undef CHONK_GEMM_CASE
-}
+// the GEMMs address the activation planes with 32-bit byte offsets
+bool gemm_planes_fit(const GemmArgs& a) { return a.t >= 1 && (int64_t)plane_rows(a.t) * a.kpad * 2 <= (int64_t)UINT32_MAX; }
 
 size_t fattn_shared_bytes(int hd) {
   return sizeof(_Float16) * ((size_t)kFaKeys * (hd + 8) + (size_t)hd * (kFaKeys + 8));
 }
 
+
+// Tiles and K split of a launch over the integer codes. The larger the tile, the
+// less each CU reads and dequantizes per product, as long as the grid covers the
+// device; a K split makes up for too few tiles but costs its partial sums twice.
+// Measured (us, Q4_K; weight rows x K at token rows: ni, tj, split):
+//   4096 x 1024 at 2047: 47.9 (8, 2, 1)  50.7 (4, 2, 1)  55.4 (4, 1, 1)
+//   1024 x 2048 at 2047: 26.8 (4, 2, 2)  28.5 (8, 2, 4)  29.9 (4, 1, 1)
+//   4096 x 1024 at 1200: 31.4 (8, 2, 2)  41.5 (8, 2, 1)  35.6 (4, 1, 1)
+//   4096 x 1024 at 288:  15.4 (4, 1, 1)  16.2 (4, 1, 2)  18.1 (8, 1, 1)
+//   1024 x 2048 at 288:  12.2 (4, 1, 4)  13.9 (4, 1, 7)  15.8 (8, 1, 7)
+//   1024 x 2048 at 80:    6.6 (4, 1, 8)   7.8 (4, 1, 4)   7.9 (8, 1, 8)
+// With one row tile (up to 64 rows), half the CUs: 32 rows of SmolLM2-135M Q8_0 take
+// 1.79 ms with 128 or 256 workgroups wanted, and the partial sums are half as many.
+struct IntTiles {
+  int ni, tj, ks;
+};
+IntTiles gemm_int_tiles(const GemmArgs& a, int n_rows, int64_t part_cap) {
+  auto tiles = [&](int ni, int tj) {
+    return ((n_rows + 16 * ni - 1) / (16 * ni)) * ((a.t + 64 * tj - 1) / (64 * tj));
+  };
+  const int tj = a.t > 512 ? 2 : 1, ni = tj == 2 && tiles(8, 2) >= 256 ? 8 : 4;
+  const int n = tiles(ni, tj), want = tj == 2 ? 512 : a.t > 64 ? 256 : 128;
+  const int step = gemm_int_step(a.w.type), nst = (a.w.k + step - 1) / step;
+  int ks = std::max(1, std::min({(want + n / 2) / n, nst, kMaxDeferSplit}));
+  while (ks > 1 && (int64_t)ks * a.t * n_rows > part_cap) --ks;
+  return {ni, tj, ks};
+}
 
 hipError_t launch_gemm(const GemmArgs& a0, hipStream_t s) {
   GemmArgs a = a0;
@@ -2172,22 +2113,13 @@ hipError_t launch_gemm(const GemmArgs& a0, hipStream_t s) {
     return hipGetLastError();
   }
   if (!gemm_planes_fit(a)) return hipErrorInvalidValue;
-  const int tj = gemm_tj(a.t), gt = gemm_tokens(tj);
-  const int tiles = ((a.w.n + kGM - 1) / kGM) * ((a.t + gt - 1) / gt);
-  const int nst = (a.w.k + kGK - 1) / kGK;
-  a.ksplit = 1;
-  if (a.part && tiles < 256) {
-    int ks = std::min(nst, (256 + tiles - 1) / tiles);
-    while (ks > 1 && (int64_t)ks * a.t * a.w.n > a.part_cap) --ks;
-    a.ksplit = ks;
-  }
-  const dim3 grid((a.w.n + kGM - 1) / kGM, (a.t + gt - 1) / gt, a.ksplit);
-  if (!launch_gemm_tiles(a, tj, grid, s)) return hipErrorInvalidValue;
-  if (a.ksplit > 1) {
-    const int64_t total = (int64_t)a.t * a.w.n;
-    const int blocks = (int)std::min<int64_t>((total + kWg - 1) / kWg, 4096);
-    hipLaunchKernelGGL(k_gemm_reduce, dim3(blocks), dim3(kWg), 0, s, a);
-  }
+  const IntTiles it = gemm_int_tiles(a, a.w.n, a.part ? a.part_cap : 0);
+  a.ksplit = it.ks;
+  const hipError_t e = launch_gemm_int(a, a.w.n, it.ni, it.tj, s);
+  if (e != hipSuccess || a.ksplit == 1) return e;
+  const int64_t total = (int64_t)a.t * a.w.n;
+  const int blocks = (int)std::min<int64_t>((total + kWg - 1) / kWg, 4096);
+  hipLaunchKernelGGL(k_gemm_reduce, dim3(blocks), dim3(kWg), 0, s, a);
   return hipGetLastError();
 }
 
@@ -2195,8 +2127,8 @@ hipError_t launch_gemm_deferred(const GemmArgs& a0, float* region, int64_t regio
   GemmArgs a = a0;
   const int N = a.n_all ? a.n_all : a.w.n;
   if (a.n_all) {
-    // fused segments: one type and K, starts on tile boundaries, in order
-    if (a.n1 <= 0 || a.n1 % kGM || a.n2 < a.n1 || a.n2 % kGM || a.n_all < a.n2 || a.w2.type != a.w.type ||
+    // fused segments: one type and K, in order, at multiples of 64 rows
+    if (a.n1 <= 0 || a.n1 % kSkRows || a.n2 < a.n1 || a.n2 % kSkRows || a.n_all < a.n2 || a.w2.type != a.w.type ||
         a.w3.type != a.w.type || a.w2.k != a.w.k || a.w3.k != a.w.k || a.w.n != a.n1 ||
         (a.n2 > a.n1 && a.w2.n != a.n2 - a.n1) || (a.n_all > a.n2 && a.w3.n != a.n_all - a.n2))
       return hipErrorInvalidValue;
@@ -2230,40 +2162,37 @@ hipError_t launch_gemm_deferred(const GemmArgs& a0, float* region, int64_t regio
     return e;
   }
   if (!gemm_planes_fit(a)) return hipErrorInvalidValue;
-  const int tj = gemm_tj(a.t), gt = gemm_tokens(tj);
-  const int tiles = ((N + kGM - 1) / kGM) * ((a.t + gt - 1) / gt);
-  const int nst = (a.w.k + kGK - 1) / kGK;
-  // split K until about four workgroups per CU are queued (passes of 128-row
-  // tiles; two with 64-row tiles); a decode batch (one row tile) runs faster
-  // with half the CUs busy, as fewer, longer-running
-  // workgroups amortise the stage pipeline's start (64 rows of the Qwen3-0.6B
-  // shapes: 3.86 ms per step at 128, 3.99 at 512, 4.39 at 64)
-  const int target = a.t <= 64 ? 128 : (tj == 2 ? 1024 : 512);
-  int ks = tiles < target ? std::min(std::min(nst, kMaxDeferSplit), (target + tiles - 1) / tiles) : 1;
-  while (ks > 1 && (int64_t)ks * a.t * N > region_cap) --ks;
-  a.ksplit = ks;
-  a.part = region;
-  a.defer = 1;
-  const dim3 grid((N + kGM - 1) / kGM, (a.t + gt - 1) / gt, ks);
-  if (!launch_gemm_tiles(a, tj, grid, s)) return hipErrorInvalidValue;
   out->p = region;
   out->n = N;
   out->ld = N;
-  out->ks = ks;
   out->zs = (int64_t)a.t * N;
-  return hipGetLastError();
+  const IntTiles it = gemm_int_tiles(a, N, region_cap);
+  a.ksplit = out->ks = it.ks;
+  a.part = region;
+  a.defer = 1;
+  return launch_gemm_int(a, N, it.ni, it.tj, s);
+}
+
+hipError_t launch_gemm_glu(const GemmArgs& a0, float* region, int64_t region_cap, PartSum* out, hipStream_t s) {
+  GemmArgs a = a0;
+  *out = PartSum{};
+  if (gemm_sk_applies(a) || !gemm_planes_fit(a)) return hipSuccess;
+  const IntTiles it = gemm_int_tiles(a, a.n2, region_cap);
+  if (it.ks != 1 || (it.ni == 4 && it.tj == 2) || (int64_t)a.t * a.n1 > region_cap) return hipSuccess;
+  a.ksplit = 1;
+  a.part = region;
+  a.defer = 1;
+  const hipError_t e = launch_gemm_int(a, a.n2, it.ni, it.tj, s);
+  if (e != hipSuccess) return e;
+  out->p = region;
+  out->n = out->ld = a.n1;
+  out->ks = 1;
+  out->zs = (int64_t)a.t * a.n1;
+  return hipSuccess;
 }
 
 hipError_t init_gemm_attributes() {
-  const size_t sh = gemm_shared_bytes();
-  const void* fns[12] = {(const void*)k_gemm<QT_Q4_K, 1>, (const void*)k_gemm<QT_Q5_K, 1>, (const void*)k_gemm<QT_Q6_K, 1>,
-                         (const void*)k_gemm<QT_Q8_0, 1>, (const void*)k_gemm<QT_Q5_0, 1>, (const void*)k_gemm<QT_Q5_1, 1>,
-                         (const void*)k_gemm<QT_Q4_K, 2>, (const void*)k_gemm<QT_Q5_K, 2>, (const void*)k_gemm<QT_Q6_K, 2>,
-                         (const void*)k_gemm<QT_Q8_0, 2>, (const void*)k_gemm<QT_Q5_0, 2>, (const void*)k_gemm<QT_Q5_1, 2>};
-  for (const void* f : fns) {
-    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh);
-    if (e != hipSuccess) return e;
-  }
+  if (const hipError_t e = init_gemm_int_attributes(); e != hipSuccess) return e;
   for (const void* f : {(const void*)k_gemm_sk<QT_Q4_K>, (const void*)k_gemm_sk<QT_Q6_K>,
                         (const void*)k_gemm_sk1<QT_Q4_K>, (const void*)k_gemm_sk1<QT_Q6_K>}) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_sk_shared_bytes());
@@ -2282,26 +2211,38 @@ hipError_t init_gemm_attributes() {
   return hipSuccess;
 }
 
-// the instance of a per-row kernel that holds a row of kpad elements
-#define CHONK_ROW_CASE(kpad, ...)                       \
-  do {                                                  \
-    if ((kpad) > kPfRowMax) return hipErrorInvalidValue; \
-    if ((kpad) <= 4 * kRowT) {                          \
-      constexpr int E = 4;                              \
-      __VA_ARGS__;                                      \
-    } else {                                            \
-      constexpr int E = 8;                              \
-      __VA_ARGS__;                                      \
-    }                                                   \
-    return hipGetLastError();                           \
+// The instance of a per-row kernel for `rows` rows of kpad elements: a wave per
+// row once those cover the device a few times over (kRowWave rows), else the
+// row over two or four waves.
+constexpr int kRowWave = 1024;
+#define CHONK_ROW_INST(tpr, e, ...)                              \
+  {                                                              \
+    constexpr int TPR = tpr, E = e;                              \
+    const dim3 grid((rows + kWg / TPR - 1) / (kWg / TPR));       \
+    __VA_ARGS__;                                                 \
+    return hipGetLastError();                                    \
+  }
+#define CHONK_ROW_CASE(kpad, ...)                                        \
+  do {                                                                   \
+    if ((kpad) > kPfRowMax) return hipErrorInvalidValue;                 \
+    if (rows >= kRowWave && (kpad) <= 3072) {                            \
+      if ((kpad) <= 1024) CHONK_ROW_INST(64, 2, __VA_ARGS__)             \
+      if ((kpad) <= 2048) CHONK_ROW_INST(64, 4, __VA_ARGS__)             \
+      CHONK_ROW_INST(64, 6, __VA_ARGS__)                                 \
+    }                                                                    \
+    if ((kpad) <= 1024) CHONK_ROW_INST(128, 1, __VA_ARGS__)              \
+    if ((kpad) <= 2048) CHONK_ROW_INST(256, 1, __VA_ARGS__)              \
+    if ((kpad) <= 4096) CHONK_ROW_INST(256, 2, __VA_ARGS__)              \
+    CHONK_ROW_INST(256, 4, __VA_ARGS__)                                  \
   } while (0)
 
 hipError_t launch_pf_split(const PfSplitArgs& a, int rows, hipStream_t s) {
+  if (a.k % 32 != 0 || a.ldx % 4 != 0 || ((uintptr_t)a.x & 15)) return hipErrorInvalidValue;
   if (a.norm_b || a.add_bias) {
     if ((a.w && !a.norm_b) || (a.add.p && !a.add_bias)) return hipErrorInvalidValue;
-    CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_split<E, true>), dim3(rows), dim3(kRowT), 0, s, a));
+    CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_split<TPR, E, true>), grid, dim3(kWg), 0, s, a, rows));
   }
-  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_split<E, false>), dim3(rows), dim3(kRowT), 0, s, a));
+  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_split<TPR, E, false>), grid, dim3(kWg), 0, s, a, rows));
 }
 hipError_t launch_pf_embed(const QMat& embed, const int32_t* tok, float scale, const float* pos, int p0, int k,
                            float* x, int rows, hipStream_t s) {
@@ -2310,7 +2251,7 @@ hipError_t launch_pf_embed(const QMat& embed, const int32_t* tok, float scale, c
 }
 hipError_t launch_pf_conv(const PfConvArgs& a, int rows, hipStream_t s) {
   if (rows < 1 || a.p.n < 3 * a.k) return hipErrorInvalidValue;
-  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_conv<E>), dim3(rows), dim3(kRowT), 0, s, a));
+  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_conv<TPR, E>), grid, dim3(kWg), 0, s, a, rows));
 }
 hipError_t launch_pf_conv_state(const PfConvArgs& a, int rows, hipStream_t s) {
   if (rows < 1 || a.p.n < 3 * a.k) return hipErrorInvalidValue;
@@ -2328,14 +2269,14 @@ hipError_t launch_pf_mamba(const PfMambaArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 hipError_t launch_pf_gate(const PfGateArgs& a, int rows, hipStream_t s) {
-  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_gate<E>), dim3(rows), dim3(kRowT), 0, s, a));
+  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_gate<TPR, E>), grid, dim3(kWg), 0, s, a, rows));
 }
 hipError_t launch_pf_norm_add(const float* d, const float* w, float eps, int k, float* x, int rows, hipStream_t s) {
   hipLaunchKernelGGL(k_pf_norm_add, dim3(rows), dim3(kWg), 0, s, d, w, eps, k, x);
   return hipGetLastError();
 }
 hipError_t launch_pf_glu_split(const PfGluArgs& a, int rows, hipStream_t s) {
-  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_glu_split<E>), dim3(rows), dim3(kRowT), 0, s, a));
+  CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_glu_split<TPR, E>), grid, dim3(kWg), 0, s, a, rows));
 }
 hipError_t launch_pf_rope_kv(const PfRopeArgs& a, int rows, hipStream_t s) {
   const int nh = a.heads + a.kv_heads;
