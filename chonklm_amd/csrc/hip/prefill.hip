@@ -1374,9 +1374,11 @@ __global__ __launch_bounds__(kWg) void k_pf_attn(PfAttnArgs a) {
 // transposed so that no operand needs a shuffle: per block of 64 keys,
 //   S^T = K Q^T  (v_mfma 16x16x32: K rows from LDS, q split into fp16 hi + lo),
 // whose accumulator layout (lane: query lane % 16, keys 4 (lane / 16) + i of
-// each 16-key tile) is the B operand layout of the 16x16x16 product, so
+// each 16-key tile) is a B operand layout with the keys permuted, so
 //   O^T += V^T P^T  (P split into hi + lo; V^T staged in LDS, V exact)
-// takes P straight from the registers, and every lane keeps the running
+// takes P straight from the registers as 16x16x32 products too (twice the rate
+// of the 16x16x16 shape): the lane's eight k of a 32-key step are keys 4 quad + i
+// of the step's two 16-key tiles, and V^T is staged with its keys in that order, and every lane keeps the running
 // maximum, sum and output of its own query. Scores are kept in log2 units
 // (scale * log2 e folded into one multiply) and the exponent base is only
 // raised when a block's maximum exceeds it by more than 8 (P <= 2^8 stays
@@ -1389,9 +1391,6 @@ __global__ __launch_bounds__(kWg) void k_pf_attn(PfAttnArgs a) {
 // (id mod 8), so with 8 kv heads each XCD's L2 holds one head's K/V.
 constexpr int kFaKeys = 64;
 
-__device__ __forceinline__ float4_t mfma16(half4_t a, half4_t b, float4_t c) {
-  return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
-}
 // max / sum over the four lanes of one query (lanes l, l ^ 16, l ^ 32, l ^ 48)
 __device__ __forceinline__ float xquad_max(float v) {
   float a, b;
@@ -1409,7 +1408,7 @@ __device__ __forceinline__ float xquad_sum(float v) {
 }
 
 template <int HD, bool PAGED>
-__global__ __launch_bounds__(kWg) void k_pf_fattn(PfAttnArgs a) {
+__global__ __launch_bounds__(kWg, HD <= 128 ? 2 : 1) void k_pf_fattn(PfAttnArgs a) {
   extern __shared__ __align__(16) _Float16 fsm[];
   constexpr int KS = HD + 8, VS = kFaKeys + 8;
   constexpr int NKP = HD / 32;                   // K pieces (8 halves) per thread and block
@@ -1457,8 +1456,9 @@ __global__ __launch_bounds__(kWg) void k_pf_fattn(PfAttnArgs a) {
   const int qpos = qok ? row_pos(a.kv, qt) : -1;
   const int qstart = (a.window != 0 && qpos + 1 > a.window) ? qpos + 1 - a.window : 0;
   // the wave's key range seen by every one of its queries (unused rows excluded)
-  const int wpos_min = (int)-wave_max(-(float)(qok ? qpos : 1 << 24));
-  const int wstart_max = (int)wave_max((float)(qok ? qstart : 0));
+  // (in scalar registers: the masking below is then a branch, not 48 instructions of every block)
+  const int wpos_min = __builtin_amdgcn_readfirstlane((int)-wave_max(-(float)(qok ? qpos : 1 << 24)));
+  const int wstart_max = __builtin_amdgcn_readfirstlane((int)wave_max((float)(qok ? qstart : 0)));
   const float sl2 = a.scale * 1.44269504088896341f;
   const int t_last = min(t0 + TW, a.rows) - 1;
   const int pos_hi = row_pos(a.kv, t_last), pos_lo = row_pos(a.kv, t0);
@@ -1512,13 +1512,15 @@ __global__ __launch_bounds__(kWg) void k_pf_fattn(PfAttnArgs a) {
     for (int j = 0; j < NVI; ++j) {
       const int item = tid + kWg * j, kp = item % (kFaKeys / 2), d8 = (item / (kFaKeys / 2)) * 8;
       if (item < VITEMS) {
-        // dims d8 .. d8 + 7 of keys 2 kp and 2 kp + 1 as eight (key, key + 1) pairs
+        // dims d8 .. d8 + 7 of keys 2 kp and 2 kp + 1 as eight (key, key + 1) pairs;
+        // key 32 s + 16 h + 4 q + i of the block sits at 32 s + 8 q + 4 h + i
+        const int key = 2 * kp, at = (key & 32) + 8 * ((key & 15) >> 2) + 4 * ((key >> 4) & 1) + (key & 3);
         const uint32_t* w0 = (const uint32_t*)&vreg[j][0];
         const uint32_t* w1 = (const uint32_t*)&vreg[j][1];
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-          *(uint32_t*)(vt + (d8 + 2 * d) * VS + 2 * kp) = (w0[d] & 0xffffu) | (w1[d] << 16);
-          *(uint32_t*)(vt + (d8 + 2 * d + 1) * VS + 2 * kp) = (w0[d] >> 16) | (w1[d] & 0xffff0000u);
+          *(uint32_t*)(vt + (d8 + 2 * d) * VS + at) = (w0[d] & 0xffffu) | (w1[d] << 16);
+          *(uint32_t*)(vt + (d8 + 2 * d + 1) * VS + at) = (w0[d] >> 16) | (w1[d] & 0xffff0000u);
         }
       }
     }
@@ -1536,19 +1538,20 @@ __global__ __launch_bounds__(kWg) void k_pf_fattn(PfAttnArgs a) {
     stage();
     __syncthreads();
     fetch(min(kb + 1, kb_hi));  // the next block (the last one again at the end: cache hits)
-    // S^T for the block's 64 keys x the wave's 16 queries (four 16 x 16 tiles)
-    float s[4][4];
+    // S^T for the block's 64 keys x the wave's 16 queries (four 16 x 16 tiles,
+    // their chains interleaved: no MFMA waits on the one before it)
+    float4_t sa[4];
 #pragma unroll
-    for (int kt = 0; kt < 4; ++kt) {
-      float4_t acc = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < 4; ++kt) sa[kt] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int k = 0; k < HD / 32; ++k) {
-        const half8_t kk = *(const half8_t*)(ks + (16 * kt + col) * KS + 32 * k + 8 * quad);
-        acc = mfma32(kk, qh[k], acc);
-        acc = mfma32(kk, ql[k], acc);
-      }
+    for (int k = 0; k < HD / 32; ++k) {
+      half8_t kk[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) s[kt][i] = acc[i] * sl2;
+      for (int kt = 0; kt < 4; ++kt) kk[kt] = *(const half8_t*)(ks + (16 * kt + col) * KS + 32 * k + 8 * quad);
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) sa[kt] = mfma32(kk[kt], qh[k], sa[kt]);
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) sa[kt] = mfma32(kk[kt], ql[k], sa[kt]);
     }
     if (!(k0 >= wstart_max && k0 + kFaKeys - 1 <= wpos_min)) {
       // some query of the wave sees only part of the block
@@ -1557,43 +1560,56 @@ __global__ __launch_bounds__(kWg) void k_pf_fattn(PfAttnArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int key = k0 + 16 * kt + 4 * quad + i;
-          s[kt][i] = key >= qstart && key <= qpos ? s[kt][i] : -INFINITY;
+          sa[kt][i] = key >= qstart && key <= qpos ? sa[kt][i] : -INFINITY;
         }
     }
     float mb = -INFINITY;
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mb = fmaxf(mb, s[kt][i]);
-    mb = xquad_max(mb);
+      for (int i = 0; i < 4; ++i) mb = fmaxf(mb, sa[kt][i]);
+    mb = xquad_max(mb) * sl2;  // (log2 units; the scale is positive)
     const bool upd = mb > m_use + 8.0f;
     const float alpha = !upd ? 1.0f : (m_use == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_use - mb));
     m_use = upd ? mb : m_use;
     const float base = m_use == -INFINITY ? 0.f : m_use;  // masked scores give exp2(-inf) = 0
     float lb = 0.f;
-    half4_t ph[4], pl[4];
+    half8_t ph[2], pl[2];  // of the block's two 32-key steps
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float p = __builtin_amdgcn_exp2f(s[kt][i] - base);
-        lb += p;
-        ph[kt][i] = (_Float16)p;
-        pl[kt][i] = (_Float16)(p - (float)ph[kt][i]);
+      for (int i = 0; i < 4; i += 2) {
+        // (pairs, for the packed conversion)
+        const float2_t p = {__builtin_amdgcn_exp2f(fmaf(sa[kt][i], sl2, -base)),
+                            __builtin_amdgcn_exp2f(fmaf(sa[kt][i + 1], sl2, -base))};
+        lb += p[0] + p[1];
+        const half2_t h = __builtin_convertvector(p, half2_t);
+        const float2_t r = {p[0] - (float)h[0], p[1] - (float)h[1]};
+        const half2_t lo = __builtin_convertvector(r, half2_t);
+        ph[kt >> 1][4 * (kt & 1) + i] = h[0];
+        ph[kt >> 1][4 * (kt & 1) + i + 1] = h[1];
+        pl[kt >> 1][4 * (kt & 1) + i] = lo[0];
+        pl[kt >> 1][4 * (kt & 1) + i + 1] = lo[1];
       }
     l_run = l_run * alpha + xquad_sum(lb);
     if (__builtin_amdgcn_ballot_w64(upd) != 0) {
 #pragma unroll
       for (int d = 0; d < HD / 16; ++d) o[d] *= alpha;
     }
-    // O^T += V^T P^T over the block's keys (four 16-key steps)
+    // O^T += V^T P^T over the block's keys (two 32-key steps), DG dim tiles'
+    // chains interleaved
+    constexpr int DG = HD >= 64 ? 4 : 2;
 #pragma unroll
-    for (int d = 0; d < HD / 16; ++d) {
+    for (int d = 0; d < HD / 16; d += DG) {
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        const half4_t vv = *(const half4_t*)(vt + (16 * d + col) * VS + 16 * kt + 4 * quad);
-        o[d] = mfma16(vv, ph[kt], o[d]);
-        o[d] = mfma16(vv, pl[kt], o[d]);
+      for (int st = 0; st < 2; ++st) {
+        half8_t vv[DG];
+#pragma unroll
+        for (int e = 0; e < DG; ++e) vv[e] = *(const half8_t*)(vt + (16 * (d + e) + col) * VS + 32 * st + 8 * quad);
+#pragma unroll
+        for (int e = 0; e < DG; ++e) o[d + e] = mfma32(vv[e], ph[st], o[d + e]);
+#pragma unroll
+        for (int e = 0; e < DG; ++e) o[d + e] = mfma32(vv[e], pl[st], o[d + e]);
       }
     }
   }
