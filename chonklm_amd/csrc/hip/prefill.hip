@@ -1055,8 +1055,8 @@ __global__ __launch_bounds__(kWg) void k_pf_mamba_scan(PfMambaArgs a) {
   const int h = tid >> 5, l = tid & 31;
   const int ld = pf_mamba_ld(a.conv, a.heads);
   const int nx = n * kMbHd + c0;  // the workgroup's first channel
-  float4* sp = reinterpret_cast<float4*>(a.ssm_state + (size_t)(nx + h) * kMbStates) + l;
-  float4 s = *sp;
+  float4_t* sp = reinterpret_cast<float4_t*>(a.ssm_state + (size_t)(nx + h) * kMbStates) + l;
+  float4_t s = *sp;
   const float dsk = a.d[n];
   // the next window: entry r is the input of row rows - 3 + r, or the old window's
   auto window = [&](int c) {
@@ -1079,13 +1079,13 @@ __global__ __launch_bounds__(kWg) void k_pf_mamba_scan(PfMambaArgs a) {
 
   // staging roles: thread moves float4 (tid % 64) of rows tid / 64 + 4 i of
   // B | C, and (row tid / 8, channel tid % 8) of x, dt and decay
-  float4 rb[kMbSteps / 4];
+  float4_t rb[kMbSteps / 4];
   float rx, rdt, rdec;
   auto fetch = [&](int t0) {
 #pragma unroll
     for (int i = 0; i < kMbSteps / 4; ++i) {
       const int t = min(t0 + (tid >> 6) + 4 * i, a.rows - 1);
-      rb[i] = *reinterpret_cast<const float4*>(a.xbc + (size_t)t * ld + a.inner + 4 * (tid & 63));
+      rb[i] = *reinterpret_cast<const float4_t*>(a.xbc + (size_t)t * ld + a.inner + 4 * (tid & 63));
     }
     const float* r = a.xbc + (size_t)min(t0 + (tid >> 3), a.rows - 1) * ld;
     rx = r[nx + (tid & 7)];
@@ -1097,7 +1097,7 @@ __global__ __launch_bounds__(kWg) void k_pf_mamba_scan(PfMambaArgs a) {
     __syncthreads();  // the previous rows are consumed, their y written out
 #pragma unroll
     for (int i = 0; i < kMbSteps / 4; ++i)
-      *reinterpret_cast<float4*>(&sbc[(tid >> 6) + 4 * i][4 * (tid & 63)]) = rb[i];
+      *reinterpret_cast<float4_t*>(&sbc[(tid >> 6) + 4 * i][4 * (tid & 63)]) = rb[i];
     sx[tid >> 3][tid & 7] = rx;
     // (steps past the last row leave the state as it is)
     const bool live = t0 + (tid >> 3) < a.rows;
@@ -1106,25 +1106,48 @@ __global__ __launch_bounds__(kWg) void k_pf_mamba_scan(PfMambaArgs a) {
     __syncthreads();
     fetch(min(t0 + kMbSteps, a.rows - 1));
     const int nt = min(kMbSteps, a.rows - t0);
-    for (int tb = 0; tb < nt; tb += 4) {
+    // four steps at a time: the next four's LDS reads are in flight, and the four
+    // sums over the lanes interleave (a step by itself waits for every read and
+    // every lane exchange)
+    struct Steps {
+      float4_t B[4], C[4];
+      float dx[4], dec[4];
+    };
+    auto load = [&](Steps& g, int tb) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int t = tb + u;
-        const float4 B = *reinterpret_cast<const float4*>(&sbc[t][4 * l]);
-        const float4 C = *reinterpret_cast<const float4*>(&sbc[t][kMbStates + 4 * l]);
-        const float dx = sxd[t][h], dec = sdec[t];
-        s.x = fmaf(s.x, dec, dx * B.x);
-        s.y = fmaf(s.y, dec, dx * B.y);
-        s.z = fmaf(s.z, dec, dx * B.z);
-        s.w = fmaf(s.w, dec, dx * B.w);
-        float acc = fmaf(s.x, C.x, s.y * C.y) + fmaf(s.z, C.z, s.w * C.w);
-        acc = group_sum<32>(acc);
-        if (l == 0) sy[t][h] = __fadd_rn(acc, __fmul_rn(dsk, sx[t][h]));
+        g.B[u] = *reinterpret_cast<const float4_t*>(&sbc[tb + u][4 * l]);
+        g.C[u] = *reinterpret_cast<const float4_t*>(&sbc[tb + u][kMbStates + 4 * l]);
+        g.dx[u] = sxd[tb + u][h];
+        g.dec[u] = sdec[tb + u];
       }
+    };
+    auto walk = [&](const Steps& g, int tb) {
+      float acc[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = fmaf(s[q], g.dec[u], g.dx[u] * g.B[u][q]);
+        acc[u] = fmaf(s[0], g.C[u][0], s[1] * g.C[u][1]) + fmaf(s[2], g.C[u][2], s[3] * g.C[u][3]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[u] = group_sum<32>(acc[u]);
+      // lane u of the channel's 32 keeps step u
+      const float a01 = l == 1 ? acc[1] : acc[0], a23 = l == 3 ? acc[3] : acc[2];
+      if (l < 4) sy[tb + l][h] = l < 2 ? a01 : a23;
+    };
+    Steps g0, g1;
+    load(g0, 0);
+    for (int tb = 0; tb < nt; tb += 8) {
+      load(g1, tb + 4);
+      walk(g0, tb);
+      load(g0, min(tb + 8, kMbSteps - 4));
+      walk(g1, tb + 4);
     }
     __syncthreads();
     const int t = tid >> 3;
-    if (t < nt) a.y[(size_t)(t0 + t) * a.inner + nx + (tid & 7)] = sy[t][tid & 7];
+    if (t < nt)
+      a.y[(size_t)(t0 + t) * a.inner + nx + (tid & 7)] = __fadd_rn(sy[t][tid & 7], __fmul_rn(dsk, sx[t][tid & 7]));
   }
   *sp = s;
 }
@@ -2275,7 +2298,7 @@ hipError_t launch_pf_conv_state(const PfConvArgs& a, int rows, hipStream_t s) {
   return hipGetLastError();
 }
 hipError_t launch_pf_mamba(const PfMambaArgs& a, hipStream_t s) {
-  static_assert(kWg == 2 * kMbStates && kWg == kMbSteps * kMbCh && kWg == 32 * kMbCh, "scan geometry");
+  static_assert(kMbSteps % 8 == 0 && kWg == 2 * kMbStates && kWg == kMbSteps * kMbCh && kWg == 32 * kMbCh, "scan geometry");
   if (a.rows < 1 || a.inner != a.heads * kMbHd || a.conv != a.inner + 2 * kMbStates ||
       a.p.n < a.inner + a.conv + a.heads)
     return hipErrorInvalidValue;
