@@ -2572,6 +2572,8 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
       r.kn_w = c.qk_norm ? L.k_norm : nullptr;
       r.eps = c.qk_eps;
       r.rope_inv = rope_table(e, c.layer[i].theta, c.hd);
+      // (the decode attention's table, made with the engine)
+      r.rope_cs = e->dec_attn ? rope_cs_table(e, c.layer[i].theta, c.hd) : nullptr;
       r.kv = kv_addr(i);
       // decode batches: the page-walking attention (one workgroup per (kv head,
       // row) walking all of its pages also does the rotary/K-V write)

@@ -131,6 +131,7 @@ struct PfRopeArgs {
   const float* bias;      // [q | k | v] added to the projections first (null: none)
   float eps;
   const float* rope_inv;  // [hd/2]
+  const float2* rope_cs;  // [position][hd/2] (cos, sin) of those angles, or null
   KvAddr kv;
 };
 
