@@ -1,4 +1,4 @@
-// Decode attention over the fp16 K/V cache for one new token: the body of
+// Decode attention over the fp16 (KV32: fp32) K/V cache for one new token: the body of
 // k_attn_dec (attn_decode.hip, which describes its phases) and of the fused
 // q|k|v + attention launch (kernels.hip), where the group's q, k and v rows
 // arrive as tagged words from the q|k|v workgroups of the same launch instead
@@ -48,17 +48,18 @@ __device__ __forceinline__ float tag_val(uint64_t w) { return __uint_as_float((u
 // epoch a.cnt[kv], which the newest chunk advances when it is done.
 // WALK: the workgroup walks a.sub sub-chunks (long contexts); otherwise its
 // chunk is one sub-chunk and the code is that of a single chunk.
-template <int G, int HD, bool WALK, bool FUSED>
+template <int G, int HD, bool WALK, bool FUSED, bool KV32 = false>
 __device__ __forceinline__ void attn_dec_body(const AttnArgs& a, int kv, int c) {
   extern __shared__ __align__(16) float sm[];
   constexpr int HALF = HD / 2;
   constexpr int DPT = HD / 4;            // K dims per lane (four lanes per position)
-  constexpr int NKV = DPT / 8;           // 16-byte K vectors per lane
+  constexpr int KPV = KV32 ? 4 : 8;      // K dims per 16-byte vector
+  constexpr int NKV = DPT / KPV;         // 16-byte K vectors per lane
   constexpr int NPR = (HALF + 63) / 64;  // rotary pairs per lane
   // V: wave w owns dims [w * HD / 4, (w + 1) * HD / 4) of all 64 positions;
   // a lane holds VD consecutive dims (VW dwords) of NP positions
   constexpr int VD = HD >= 256 ? 4 : 2;
-  constexpr int VW = VD / 2;
+  constexpr int VW = KV32 ? VD : VD / 2;
   constexpr int DW = HD / 4 / VD;        // lanes per position row: 8 or 16
   constexpr int LDW = DW == 8 ? 3 : 4;
   constexpr int PG = 64 / DW;            // position groups
@@ -93,22 +94,29 @@ __device__ __forceinline__ void attn_dec_body(const AttnArgs& a, int kv, int c) 
   const int kd0 = (lane & 3) * DPT;
   const int pg = lane >> LDW;                    // this lane's V positions: pg + PG * j
   const int vd = wave * (HD / 4) + VD * (lane & (DW - 1));
-  const __half* kc = (const __half*)a.kc + (size_t)kv * a.ctx * HD;
-  const __half* vc = (const __half*)a.vc + (size_t)kv * a.ctx * HD;
+  constexpr int EB = KV32 ? 4 : 2;       // bytes per cache element
+  const uint8_t* kc = (const uint8_t*)a.kc + (size_t)kv * a.ctx * HD * EB;
+  const uint8_t* vc = (const uint8_t*)a.vc + (size_t)kv * a.ctx * HD * EB;
   uint4 kr[NKV];
   uint32_t vr[NP][VW];
   // K / V rows of the 64 positions from t0
   auto load_k = [&](int t0) {
     const int tk = min(t0 + kp, a.ctx - 1);
 #pragma unroll
-    for (int v = 0; v < NKV; ++v) kr[v] = ldg4(kc + (size_t)tk * HD + kd0 + 8 * v);
+    for (int v = 0; v < NKV; ++v) kr[v] = ldg4(kc + ((size_t)tk * HD + kd0 + KPV * v) * EB);
   };
   auto load_v = [&](int t0) {
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
-      const __half* p = vc + (size_t)min(t0 + pg + PG * j, a.ctx - 1) * HD + vd;
+      const uint8_t* p = vc + ((size_t)min(t0 + pg + PG * j, a.ctx - 1) * HD + vd) * EB;
       if constexpr (VW == 1) {
         vr[j][0] = ldg1(p);
+      } else if constexpr (VW == 4) {
+        const uint4 w = ldg4(p);
+        vr[j][0] = w.x;
+        vr[j][1] = w.y;
+        vr[j][VW - 2] = w.z;
+        vr[j][VW - 1] = w.w;
       } else {
         const uint2 w = ldg2(p);
         vr[j][0] = w.x;
@@ -253,6 +261,15 @@ __device__ __forceinline__ void attn_dec_body(const AttnArgs& a, int kv, int c) 
 #pragma unroll
         for (int j = 0; j < NPR; ++j)
           if (lane + 64 * j < HALF) {
+            if constexpr (KV32) {
+              if (c == c_hi) {
+                *gblw((float*)a.kc + kv_row + ia[j]) = y0[j];
+                *gblw((float*)a.kc + kv_row + ib[j]) = y1[j];
+              }
+              kx[ia[j]] = y0[j];
+              kx[ib[j]] = y1[j];
+              continue;
+            }
             const __half h0 = __float2half_rn(y0[j]), h1 = __float2half_rn(y1[j]);
             if (c == c_hi) {
               *gblw((unsigned short*)a.kc + kv_row + ia[j]) = __half_as_ushort(h0);
@@ -265,6 +282,10 @@ __device__ __forceinline__ void attn_dec_body(const AttnArgs& a, int kv, int c) 
     } else {
 #pragma unroll
       for (int d = lane; d < HD; d += 64) {
+        if constexpr (KV32) {
+          if (c == c_hi) *gblw((float*)a.vc + kv_row + d) = vx[d];
+          continue;
+        }
         const __half vh = __float2half_rn(vx[d]);
         if (c == c_hi) *gblw((unsigned short*)a.vc + kv_row + d) = __half_as_ushort(vh);
         vx[d] = __half2float(vh);
@@ -306,7 +327,14 @@ __device__ __forceinline__ void attn_dec_body(const AttnArgs& a, int kv, int c) 
       const uint32_t w[4] = {kr[v].x, kr[v].y, kr[v].z, kr[v].w};
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        const float4 q0 = *(const float4*)(qn + g * HD + kd0 + 8 * v);
+        const float4 q0 = *(const float4*)(qn + g * HD + kd0 + KPV * v);
+        if constexpr (KV32) {
+          s[g] = fmaf(q0.x, __uint_as_float(w[0]), s[g]);
+          s[g] = fmaf(q0.y, __uint_as_float(w[1]), s[g]);
+          s[g] = fmaf(q0.z, __uint_as_float(w[2]), s[g]);
+          s[g] = fmaf(q0.w, __uint_as_float(w[3]), s[g]);
+          continue;
+        }
         const float4 q1 = *(const float4*)(qn + g * HD + kd0 + 8 * v + 4);
         s[g] = fmaf(q0.x, h2f(w[0]), s[g]);
         s[g] = fmaf(q0.y, h2f(w[0] >> 16), s[g]);
@@ -371,8 +399,12 @@ __device__ __forceinline__ void attn_dec_body(const AttnArgs& a, int kv, int c) 
         float vf[VD];
 #pragma unroll
         for (int t = 0; t < VW; ++t) {
-          vf[2 * t] = h2f(vr[j][t]);
-          vf[2 * t + 1] = h2f(vr[j][t] >> 16);
+          if constexpr (KV32) {
+            vf[t] = __uint_as_float(vr[j][t]);
+          } else {
+            vf[2 * t] = h2f(vr[j][t]);
+            vf[2 * t + 1] = h2f(vr[j][t] >> 16);
+          }
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {

@@ -1852,6 +1852,7 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
     const char* av = std::getenv("CHONK_ATTN");
     e->dec_attn = !(av && std::strcmp(av, "chunked") == 0);
     e->dsub = attn_dec_sub(c.ctx, 128);
+    const bool kv32 = e->kv_elem == 4;
     if (e->dsub > 1) {
       // long contexts: each workgroup walks several 64-position chunks, as many
       // workgroups per kv head as stay resident together with the walking kernel
@@ -1859,7 +1860,7 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
       for (const LayerCfg& lc : c.layer) {
         if (lc.conv || lc.mamba) continue;
         const int lg = lc.heads / lc.kv_heads;
-        per_head = std::min(per_head, attn_dec_resident(e->device, lg, c.hd, attn_dec_shared_bytes(lg, c.hd, 128), true) /
+        per_head = std::min(per_head, attn_dec_resident(e->device, lg, c.hd, attn_dec_shared_bytes(lg, c.hd, 128), true, kv32) /
                                           std::max(1, lc.kv_heads));
       }
       e->dsub = attn_dec_sub(c.ctx, per_head);
@@ -1868,9 +1869,9 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
     for (const LayerCfg& lc : c.layer) {
       const int lg = lc.heads / lc.kv_heads;
       if (lc.conv || lc.mamba) continue;
-      if (e->dec_attn && (!attn_dec_supported(lg, c.hd, c.ctx, e->kv_elem == 2 ? 1 : 0) ||
-                          attn_dec_resident(e->device, lg, c.hd, attn_dec_shared_bytes(lg, c.hd, e->dnchunk), e->dsub > 1) <
-                              lc.kv_heads * e->dnchunk))
+      if (e->dec_attn && (!attn_dec_supported(lg, c.hd, c.ctx) ||
+                          attn_dec_resident(e->device, lg, c.hd, attn_dec_shared_bytes(lg, c.hd, e->dnchunk), e->dsub > 1,
+                                            kv32) < lc.kv_heads * e->dnchunk))
         e->dec_attn = false;
     }
     // (another engine on this GPU holds the spin-merging attention: k_attention)
@@ -1879,7 +1880,8 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
     // (build_steps checks the instance and the grid's residency per layer);
     // CHONK_FUSE=0 keeps them apart
     const char* fv = std::getenv("CHONK_FUSE");
-    e->fuse_qkv = e->dec_attn && e->dsub == 1 && !(fv && std::strcmp(fv, "0") == 0);
+    // (the fp32 cache's rows leave the joint launch no registers: separate launches)
+    e->fuse_qkv = e->dec_attn && e->dsub == 1 && !kv32 && !(fv && std::strcmp(fv, "0") == 0);
   }
   const size_t kv_bytes = (size_t)kvdim * c.ctx * e->kv_elem;
   const size_t bits_words = (size_t)(c.vocab + 31) / 32;

@@ -184,7 +184,7 @@ hipError_t launch_ssm(const SsmArgs& a, hipStream_t s);
 // The register-resident decode attention (attn_decode.hip): fp16 cache,
 // head_dim 64/128/256, GQA group <= 8 (group x head_dim <= 1536), at most 128
 // chunks of attn_dec_chunk() positions over the context.
-bool attn_dec_supported(int group, int hd, int ctx, int kv_f16);
+bool attn_dec_supported(int group, int hd, int ctx);
 int attn_dec_chunk();
 // 64-position sub-chunks per k_attn_dec workgroup at a context, with at most
 // min(128, per_head) workgroups per kv head.
@@ -193,7 +193,7 @@ size_t attn_dec_shared_bytes(int group, int hd, int nchunk);
 // Workgroups of k_attn_dec that fit on the device at once (its active chunks
 // wait for each other, so the whole grid must be resident); 0 for an instance
 // that spills registers to scratch, which the engine then does not use.
-int attn_dec_resident(int device, int group, int hd, size_t shmem, bool walk);
+int attn_dec_resident(int device, int group, int hd, size_t shmem, bool walk, bool kv32);
 hipError_t launch_attn_dec(const AttnArgs& a, size_t shmem, hipStream_t s);
 // The fused q|k|v matvec + decode attention launch (k_qkv_attn): the matvec's
 // nq workgroups (m planned for the row kernel, EPI_TAG, PRO_NORM) ahead of the
