@@ -3115,7 +3115,7 @@ int chonk_engine_prefill(chonk_engine* e, const int32_t* tokens, size_t n) {
     if ((int64_t)e->pos + (int64_t)n > e->cfg.ctx)
       throw context_exhausted(e);
     if (!e->batched_prefill) {
-      // token by token through the decode step (gpt2, or CHONK_PREFILL=token)
+      // token by token through the decode step (rows wider than kPfRowMax, or CHONK_PREFILL=token)
       for (size_t i = 0; i < n; ++i) run_token(e, tokens[i], false, nullptr, nullptr, 0, nullptr, 0);
       e->known_token_pos = -1;
       e->logits_valid = false;

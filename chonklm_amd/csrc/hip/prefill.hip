@@ -571,8 +571,9 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk(GemmArgs a) {
 // step's layer GEMMs): every load of the wave — its x operands, copied
 // straight into its own 16 KiB of LDS, and its weight bytes — is issued at
 // entry and awaited once, so the wave pays one memory round trip before its
-// two steps of products. LDS per wave: [plane][step][token][32 halves].
-template <int T>
+// two steps of products. LDS per wave: [plane][step][token tile][512 halves].
+// NT: token tiles computed, 1, 2 or 4 (up to 16, 32 or 64 rows).
+template <int T, int NT>
 __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
   extern __shared__ __align__(16) float ssm[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -592,9 +593,9 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
 #undef CHONK_PICK_W
   // this wave's block: one per wave, the workgroup's four in a row
   const int blk = (int)blockIdx.z * 4 + wave;
-  _Float16* xw = (_Float16*)ssm + (size_t)wave * (2 * 2 * 64 * 32);  // this wave's x operands
-  float* xs = ssm + 4 * 64 * kSkRed;                                 // the token rows' operand scales
-  // x: 16 copies of 1 KiB (a token tile's 32 columns, in operand order; tiles
+  _Float16* xw = (_Float16*)ssm + (size_t)wave * (2 * 2 * NT * 512);  // this wave's x operands
+  float* xs = ssm + 4 * 16 * NT * kSkRed;                             // the token rows' operand scales
+  // x: 4 NT copies of 1 KiB (a token tile's 32 columns, in operand order; tiles
   // past a.t repeat the last one: their sums are never written)
   {
 #pragma unroll
@@ -602,11 +603,11 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < NT; ++i) {
           const _Float16* src =
               (p ? a.xl : a.xh) + plane_at(16 * min(i, (a.t - 1) / 16), sk_col<T>(blk, s2), a.kpad) + 8 * lane;
-          __builtin_amdgcn_global_load_lds((gmem_void*)src, (lds_void*)(xw + ((p * 2 + s2) * 64 + 16 * i) * 32), 16,
-                                           0, 0);
+          __builtin_amdgcn_global_load_lds((gmem_void*)src, (lds_void*)(xw + ((p * 2 + s2) * NT + i) * 512), 16, 0,
+                                           0);
         }
   }
   const float wsc = ldexpf(1.0f, a.ws);
@@ -616,18 +617,18 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
   if (tid < a.t) xs[tid] = a.xscale[tid];
   __builtin_amdgcn_s_waitcnt(0);  // (the copies into LDS land before they are read)
   __syncthreads();
-  float4_t acc[4][4];
+  float4_t acc[NT][4];
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt)
+  for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) acc[tt][rt] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s2 = 0; s2 < 2; ++s2) {
-    half8_t ah[4], al[4];
+    half8_t ah[NT], al[NT];
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      ah[tt] = *(const half8_t*)(xw + ((0 * 2 + s2) * 64 + 16 * tt) * 32 + 8 * lane);
-      al[tt] = *(const half8_t*)(xw + ((1 * 2 + s2) * 64 + 16 * tt) * 32 + 8 * lane);
+    for (int tt = 0; tt < NT; ++tt) {
+      ah[tt] = *(const half8_t*)(xw + ((0 * 2 + s2) * NT + tt) * 512 + 8 * lane);
+      al[tt] = *(const half8_t*)(xw + ((1 * 2 + s2) * NT + tt) * 512 + 8 * lane);
     }
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) {
@@ -636,47 +637,48 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
       half8_t bh, bl;
       split8(w, bh, bl);
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) acc[tt][rt] = mfma32(ah[tt], bh, acc[tt][rt]);
+      for (int tt = 0; tt < NT; ++tt) acc[tt][rt] = mfma32(ah[tt], bh, acc[tt][rt]);
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) acc[tt][rt] = mfma32(al[tt], bh, acc[tt][rt]);
+      for (int tt = 0; tt < NT; ++tt) acc[tt][rt] = mfma32(al[tt], bh, acc[tt][rt]);
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) acc[tt][rt] = mfma32(ah[tt], bl, acc[tt][rt]);
+      for (int tt = 0; tt < NT; ++tt) acc[tt][rt] = mfma32(ah[tt], bl, acc[tt][rt]);
     }
   }
   __syncthreads();  // every wave has read its x operands (the area is reused below)
   // the four waves' tiles [wave][token][row] (rows padded to kSkRed floats, so
   // that neither the writes below nor the 16-byte reads after them collide on
-  // LDS banks); then thread (token tid / 4, rows 16 (tid % 4) .. + 15) sums its
-  // 16 outputs over the waves with 16-byte reads and stores them with 16-byte
-  // stores — one pass instead of 16 dependent rounds of single floats
+  // LDS banks); then thread (token tid / TPT, rows RPT (tid % TPT) .. + RPT - 1) sums
+  // its outputs over the waves with 16-byte reads and stores them with 16-byte
+  // stores — one pass instead of dependent rounds of single floats
+  constexpr int RPT = 4 * NT, TPT = 64 / RPT;
   float* red = ssm;
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt)
+  for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) red[(wave * 64 + 16 * tt + 4 * g + i) * kSkRed + 16 * rt + r16] = acc[tt][rt][i];
+      for (int i = 0; i < 4; ++i) red[(wave * 16 * NT + 16 * tt + 4 * g + i) * kSkRed + 16 * rt + r16] = acc[tt][rt][i];
   __syncthreads();
-  const int t = tid >> 2, q = tid & 3;
+  const int t = tid / TPT, q = tid % TPT;
   if (t < a.t) {
     const float sc = ldexpf(1.0f, -a.ws) * xs[t];
-    float4 v[4];
+    float4 v[NT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float* e = red + t * kSkRed + 16 * q + 4 * j;
-      const float4 w0 = *(const float4*)e, w1 = *(const float4*)(e + 64 * kSkRed);
-      const float4 w2 = *(const float4*)(e + 2 * 64 * kSkRed), w3 = *(const float4*)(e + 3 * 64 * kSkRed);
+    for (int j = 0; j < NT; ++j) {
+      const float* e = red + t * kSkRed + RPT * q + 4 * j;
+      const float4 w0 = *(const float4*)e, w1 = *(const float4*)(e + 16 * NT * kSkRed);
+      const float4 w2 = *(const float4*)(e + 2 * 16 * NT * kSkRed), w3 = *(const float4*)(e + 3 * 16 * NT * kSkRed);
       v[j] = make_float4((((w0.x + w1.x) + w2.x) + w3.x) * sc, (((w0.y + w1.y) + w2.y) + w3.y) * sc,
                          (((w0.z + w1.z) + w2.z) + w3.z) * sc, (((w0.w + w1.w) + w2.w) + w3.w) * sc);
     }
-    const int nq = n0 + 16 * q;
+    const int nq = n0 + RPT * q;
     float* dst = a.part + ((size_t)blockIdx.z * a.t + t) * N + nq;
-    if (nq + 16 <= N && (N & 3) == 0) {
+    if (nq + RPT <= N && (N & 3) == 0) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) *(float4*)(dst + 4 * j) = v[j];
+      for (int j = 0; j < NT; ++j) *(float4*)(dst + 4 * j) = v[j];
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < NT; ++j) {
         const float o[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
         for (int e2 = 0; e2 < 4; ++e2)
@@ -695,7 +697,8 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
 // weights of the next block and its x copies are issued, then this block's
 // copies are awaited (s_waitcnt counts the loads issued since) and the waves
 // meet at a barrier before the products.
-template <int T>
+// NT: token tiles computed, as for k_gemm_sk1.
+template <int T, int NT>
 __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
   extern __shared__ __align__(16) float ssm[];
   constexpr int W = T == QT_Q4_K ? 8 : 16;  // weight loads per block and wave (4 row tiles)
@@ -704,21 +707,21 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
   const int r16 = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * (4 * kSkRows) + wave * kSkRows;  // this wave's rows
   const int N = a.w.n, nblk = a.w.k / kSkBlockK;
-  _Float16* xb = (_Float16*)ssm;  // [buffer][plane][step][token][32 halves]
-  float* xs = (float*)(xb + 2 * (2 * 2 * 64 * 32));
+  _Float16* xb = (_Float16*)ssm;  // [buffer][plane][step][token tile][512 halves]
+  float* xs = (float*)(xb + 2 * (2 * 2 * NT * 512));
   const float wsc = ldexpf(1.0f, a.ws);
   int rows[4];
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) rows[rt] = min(n0 + 16 * rt + r16, N - 1);
-  // x of block b into buffer b & 1: this wave's four of its sixteen 1-KiB copies
+  // x of block b into buffer b & 1: this wave's NT of its 4 NT 1-KiB copies
   auto copy_x = [&](int b) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int c = wave * 4 + j, p = c >> 3, s2 = (c >> 2) & 1, i = c & 3;
+    for (int j = 0; j < NT; ++j) {
+      const int c = wave * NT + j, p = c / (2 * NT), s2 = (c / NT) & 1, i = c % NT;
       const _Float16* src =
           (p ? a.xl : a.xh) + plane_at(16 * min(i, (a.t - 1) / 16), sk_col<T>(b, s2), a.kpad) + 8 * lane;
       __builtin_amdgcn_global_load_lds((gmem_void*)src,
-                                       (lds_void*)(xb + (((b & 1) * 4 + p * 2 + s2) * 64 + 16 * i) * 32), 16, 0, 0);
+                                       (lds_void*)(xb + (((b & 1) * 4 + p * 2 + s2) * NT + i) * 512), 16, 0, 0);
     }
   };
   if (tid < a.t) xs[tid] = a.xscale[tid];
@@ -728,9 +731,9 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
   __builtin_amdgcn_sched_barrier(0);
   copy_x(0);
   __builtin_amdgcn_sched_barrier(0);
-  float4_t acc[4][4];
+  float4_t acc[NT][4];
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt)
+  for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) acc[tt][rt] = float4_t{0.f, 0.f, 0.f, 0.f};
   for (int b = 0; b < nblk; ++b) {
@@ -745,18 +748,18 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
     copy_x(bn);
     __builtin_amdgcn_sched_barrier(0);
     // this block's copies have landed once at most the loads issued after
-    // them are outstanding: the next block's W weight loads and 4 copies
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(W + 4));
+    // them are outstanding: the next block's W weight loads and NT copies
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(W + NT));
     // (a bare barrier: __syncthreads would also wait for the loads in flight)
     lds_barrier();
-    const _Float16* xc = xb + (size_t)(b & 1) * 4 * 64 * 32;
+    const _Float16* xc = xb + (size_t)(b & 1) * 4 * NT * 512;
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
-      half8_t ah[4], al[4];
+      half8_t ah[NT], al[NT];
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt) {
-        ah[tt] = *(const half8_t*)(xc + ((0 * 2 + s2) * 64 + 16 * tt) * 32 + 8 * lane);
-        al[tt] = *(const half8_t*)(xc + ((1 * 2 + s2) * 64 + 16 * tt) * 32 + 8 * lane);
+      for (int tt = 0; tt < NT; ++tt) {
+        ah[tt] = *(const half8_t*)(xc + ((0 * 2 + s2) * NT + tt) * 512 + 8 * lane);
+        al[tt] = *(const half8_t*)(xc + ((1 * 2 + s2) * NT + tt) * 512 + 8 * lane);
       }
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) {
@@ -765,11 +768,11 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
         half8_t bh, bl;
         split8(w, bh, bl);
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) acc[tt][rt] = mfma32(ah[tt], bh, acc[tt][rt]);
+        for (int tt = 0; tt < NT; ++tt) acc[tt][rt] = mfma32(ah[tt], bh, acc[tt][rt]);
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) acc[tt][rt] = mfma32(al[tt], bh, acc[tt][rt]);
+        for (int tt = 0; tt < NT; ++tt) acc[tt][rt] = mfma32(al[tt], bh, acc[tt][rt]);
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) acc[tt][rt] = mfma32(ah[tt], bl, acc[tt][rt]);
+        for (int tt = 0; tt < NT; ++tt) acc[tt][rt] = mfma32(ah[tt], bl, acc[tt][rt]);
       }
     }
     lds_barrier();  // every wave has read buffer b & 1 before block b + 2's copies overwrite it
@@ -779,7 +782,7 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
   const float wun = ldexpf(1.0f, -a.ws);
   const bool add = a.epi == GEMM_ADD;
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt)
+  for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int t = 16 * tt + 4 * g + i;
@@ -799,9 +802,29 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
     }
 }
 
-size_t gemm_lm_shared_bytes() { return sizeof(_Float16) * 2 * (2 * 2 * 64 * 32) + sizeof(float) * 64; }
+size_t gemm_lm_shared_bytes(int nt) { return sizeof(_Float16) * 2 * (2 * 2 * nt * 512) + sizeof(float) * 64; }
 
-size_t gemm_sk_shared_bytes() { return sizeof(float) * (4 * 64 * kSkRed + 64); }
+size_t gemm_sk_shared_bytes(int nt = 4) { return sizeof(float) * (4 * 16 * nt * kSkRed + 64); }
+
+// Token tiles a decode-batch launch computes: the four of 64 rows cost a batch of
+// a few sequences products, copies and sums it drops (Qwen3-0.6B shape, step of 2,
+// 16, 30 and 64 rows: 2.03, 2.12, 2.27, 2.30 ms with four always; 1.83, 1.92, 2.12,
+// 2.31 with as many as the rows need).
+int gemm_sk_tiles(int rows) { return rows <= 16 ? 1 : rows <= 32 ? 2 : 4; }
+
+// kernel<type, nt> for a decode-batch launch
+#define CHONK_SK_LAUNCH(kernel, type, nt, grid, sh, s, a)                                   \
+  do {                                                                                      \
+    if ((type) == QT_Q4_K) {                                                                \
+      if ((nt) == 1) hipLaunchKernelGGL((kernel<QT_Q4_K, 1>), grid, dim3(kWg), sh, s, a);   \
+      else if ((nt) == 2) hipLaunchKernelGGL((kernel<QT_Q4_K, 2>), grid, dim3(kWg), sh, s, a); \
+      else hipLaunchKernelGGL((kernel<QT_Q4_K, 4>), grid, dim3(kWg), sh, s, a);             \
+    } else {                                                                                \
+      if ((nt) == 1) hipLaunchKernelGGL((kernel<QT_Q6_K, 1>), grid, dim3(kWg), sh, s, a);   \
+      else if ((nt) == 2) hipLaunchKernelGGL((kernel<QT_Q6_K, 2>), grid, dim3(kWg), sh, s, a); \
+      else hipLaunchKernelGGL((kernel<QT_Q6_K, 4>), grid, dim3(kWg), sh, s, a);             \
+    }                                                                                       \
+  } while (0)
 
 // The decode-batch GEMM applies: at most 64 token rows and a K-quant type it covers.
 bool gemm_sk_applies(int type, int k, int rows) {
@@ -2136,10 +2159,8 @@ hipError_t launch_gemm(const GemmArgs& a0, hipStream_t s) {
   if (!a.n_all && gemm_sk_applies(a) && a.w.n >= 128 * 4 * kSkRows) {
     // many row groups (the lm_head): four per workgroup over the whole K, x shared in LDS
     const dim3 grid((a.w.n + 4 * kSkRows - 1) / (4 * kSkRows));
-    if (a.w.type == QT_Q4_K)
-      hipLaunchKernelGGL(k_gemm_lm<QT_Q4_K>, grid, dim3(kWg), gemm_lm_shared_bytes(), s, a);
-    else
-      hipLaunchKernelGGL(k_gemm_lm<QT_Q6_K>, grid, dim3(kWg), gemm_lm_shared_bytes(), s, a);
+    const int nt = gemm_sk_tiles(a.t);
+    CHONK_SK_LAUNCH(k_gemm_lm, a.w.type, nt, grid, gemm_lm_shared_bytes(nt), s, a);
     return hipGetLastError();
   }
   if (!a.n_all && gemm_sk_applies(a)) {
@@ -2189,10 +2210,8 @@ hipError_t launch_gemm_deferred(const GemmArgs& a0, float* region, int64_t regio
     hipError_t e;
     if (one) {
       const dim3 grid((N + kSkRows - 1) / kSkRows, 1, ks);
-      if (a.w.type == QT_Q4_K)
-        hipLaunchKernelGGL(k_gemm_sk1<QT_Q4_K>, grid, dim3(kWg), gemm_sk_shared_bytes(), s, a);
-      else
-        hipLaunchKernelGGL(k_gemm_sk1<QT_Q6_K>, grid, dim3(kWg), gemm_sk_shared_bytes(), s, a);
+      const int nt = gemm_sk_tiles(a.t);
+      CHONK_SK_LAUNCH(k_gemm_sk1, a.w.type, nt, grid, gemm_sk_shared_bytes(nt), s, a);
       e = hipGetLastError();
     } else {
       e = launch_gemm_sk(a, N, s);
@@ -2237,7 +2256,7 @@ hipError_t launch_gemm_glu(const GemmArgs& a0, float* region, int64_t region_cap
 hipError_t init_gemm_attributes() {
   if (const hipError_t e = init_gemm_int_attributes(); e != hipSuccess) return e;
   for (const void* f : {(const void*)k_gemm_sk<QT_Q4_K>, (const void*)k_gemm_sk<QT_Q6_K>,
-                        (const void*)k_gemm_sk1<QT_Q4_K>, (const void*)k_gemm_sk1<QT_Q6_K>}) {
+                        (const void*)k_gemm_sk1<QT_Q4_K, 4>, (const void*)k_gemm_sk1<QT_Q6_K, 4>}) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_sk_shared_bytes());
     if (e != hipSuccess) return e;
   }

@@ -71,3 +71,40 @@ def test_step_of_more_than_64_sequences(synth):
         assert rel_err(rows[i], small.read_logits(i)) <= 1e-3  # (fp16 K/V)
     small.close()
     eng.dispose()
+
+
+@pytest.mark.parametrize("tname", ["Q4_K", "Q6_K"])
+@pytest.mark.parametrize("n_tok", [1, 16, 17, 32, 33, 64])
+def test_head_gemm_token_tiles(tname, n_tok):
+    """The lm_head GEMM of a batch with one, two and four token tiles."""
+    n_rows, row_len = 32768 + 5, 512
+    rng = np.random.default_rng(n_tok)
+    blocks = random_blocks(TYPES[tname], n_rows * row_len, rng)
+    w = orc.dequant(TYPES[tname], blocks, n_rows * row_len).reshape(n_rows, row_len)
+    x = rng.standard_normal((n_tok, row_len)).astype(np.float32)
+    got, _ = gpu_gemm(TYPES[tname], blocks, n_rows, row_len, x)
+    rows = np.unique([0, n_tok // 2, n_tok - 1])
+    want = x[rows].astype(np.float64) @ w.T.astype(np.float64)
+    err = np.linalg.norm(got[rows] - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert err.max() <= 5e-6, f"{tname}: {err.max():.2e}"
+
+
+def test_step_rows_do_not_depend_on_the_batch(synth):
+    """1 to 40 rows (one, two and four token tiles): a row's logits are the same."""
+    w = WORKLOADS["tiny-qwen3"]
+    eng = load_llama_wgsl_model(w.model_def(synth("tiny-qwen3"))).engine
+    rng = np.random.default_rng(9)
+    prompts = [rng.integers(0, w.spec.vocab, 3 + s % 5).tolist() for s in range(40)]
+    batch = LlamaWgslBatch(eng, 40, 16)
+    want = None
+    for n in (40, 33, 32, 17, 16, 2, 1):
+        for s in range(n):
+            batch.prefill(s, prompts[s])
+        batch.step(list(range(n)), [7] * n)
+        rows = np.stack([batch.read_logits(s) for s in range(n)])
+        assert np.isfinite(rows).all()
+        want = rows if want is None else want
+        # (fp32 sums in another order at most: the attention splits few rows' pages)
+        assert rel_err(rows, want[:n]) <= 2e-5, f"{n} rows"
+    batch.close()
+    eng.dispose()
