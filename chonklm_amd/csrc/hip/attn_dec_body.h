@@ -36,6 +36,13 @@ __device__ __forceinline__ uint64_t tag_get(const tagged_t* p) {
 __device__ __forceinline__ bool tag_is(uint64_t w, uint32_t tag) { return (uint32_t)(w >> 32) == tag; }
 __device__ __forceinline__ float tag_val(uint64_t w) { return __uint_as_float((uint32_t)w); }
 
+// exp of a score minus its maximum. The scaled argument of exp_fast rounds, an
+// error of |x| 2^-24 that fp16 K/V hides and an fp32 cache's results would show.
+template <bool EXACT>
+__device__ __forceinline__ float dec_exp(float x) {
+  return EXACT ? expf(x) : exp_fast(x);
+}
+
 // LDS (floats): q_s[G][HD] (raw) | kx[HD] | vx[HD] | nq[HD] | nk[HD] |
 // qn[G][HD] (normalised, rotated q, shared by the waves) | wmx[4][G] (each
 // wave's score maximum) | ew[G][64] (the chunk's weights; position p at
@@ -361,9 +368,9 @@ __device__ __forceinline__ void attn_dec_body(const AttnArgs& a, int kv, int c) 
       // finite: the sub-chunk holds a cached position
       const float mp = fmaxf(fmaxf(wmx[g], wmx[G + g]), fmaxf(wmx[2 * G + g], wmx[3 * G + g]));
       const float mn = WALK ? fmaxf(mx[g], mp) : mp;
-      if constexpr (WALK) alpha[g] = exp_fast(mx[g] - mn);  // 0 on the first sub-chunk
+      if constexpr (WALK) alpha[g] = dec_exp<KV32>(mx[g] - mn);  // 0 on the first sub-chunk
       mx[g] = mn;
-      const float e = kvalid ? exp_fast(s[g] - mn) : 0.f;
+      const float e = kvalid ? dec_exp<KV32>(s[g] - mn) : 0.f;
       if ((lane & 3) == 0) ew[g * kDecChunk + ei] = e;
     }
     __syncthreads();
@@ -509,12 +516,12 @@ __device__ __forceinline__ void attn_dec_body(const AttnArgs& a, int kv, int c) 
     const float m0 = h0 ? tag_val(w[0]) : -INFINITY, m1 = h1 ? tag_val(w[3]) : -INFINITY;
     const float sn = hv[4 * g];
     const float M = fmaxf(group_max_n(fmaxf(m0, m1), tpi), sn);
-    const float f0 = m0 == -INFINITY ? 0.f : exp_fast(m0 - M);
-    const float f1 = m1 == -INFINITY ? 0.f : exp_fast(m1 - M);
+    const float f0 = m0 == -INFINITY ? 0.f : dec_exp<KV32>(m0 - M);
+    const float f1 = m1 == -INFINITY ? 0.f : dec_exp<KV32>(m1 - M);
     const float l = (h0 ? tag_val(w[1]) * f0 : 0.f) + (h1 ? tag_val(w[4]) * f1 : 0.f);
     const float s = (h0 ? tag_val(w[2]) * f0 : 0.f) + (h1 ? tag_val(w[5]) * f1 : 0.f);
     const float L = group_sum_n(l, tpi), S = group_sum_n(s, tpi);
-    const float fn = exp_fast(sn - M);
+    const float fn = dec_exp<KV32>(sn - M);
     if (el && sub == 0) a.out[(size_t)kv * G * HD + g * HD + d] = __fdiv_rn(S + fn * vx[d], L + fn);
   }
   if (late && tid == 0) st->error = 4;
