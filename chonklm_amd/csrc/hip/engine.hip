@@ -2954,10 +2954,15 @@ void generate(chonk_engine* e, const int32_t* prompt, size_t n_prompt, int32_t m
   }
 }
 
-// The reference loop (:266-313) stepped from the host through run_token.
+// The reference loop (:266-313) stepped from the host through run_token. A
+// streamed call steps through its prompt too: it is run_token by run_token to
+// the bit. (Through row batches a 301-token prompt and 16 tokens of the
+// Qwen3-0.6B shape take 14.6 ms instead of 214, but some fp16 K/V values round
+// the other way, the logits move by 1e-4, and 4 prompts of 1500 got other greedy
+// ids at a near tie.) prompt_rows: the prompt as row batches, as generate does.
 void generate_stepped(chonk_engine* e, const int32_t* prompt, size_t n_prompt, int32_t max_new,
-                      const chonk_sampling* s_in, chonk_token_callback cb, void* user, std::vector<int32_t>* out,
-                      chonk_gen_stats* stats) {
+                      const chonk_sampling* s_in, chonk_token_callback cb, void* user, bool prompt_rows,
+                      std::vector<int32_t>* out, chonk_gen_stats* stats) {
   // maxNewTokens ?? 128 (:255): a negative value stands for "not given"
   const int64_t max = std::min<int64_t>(max_new >= 0 ? max_new : 128, (int64_t)e->def.max_context - (int64_t)n_prompt);
   const chonk_sampling s = effective_sampling(e, s_in);
@@ -2980,11 +2985,9 @@ void generate_stepped(chonk_engine* e, const int32_t* prompt, size_t n_prompt, i
     next = e->cached_next;
   } else {
     size_t done = 0;
-    if (e->batched_prefill && n_suffix > 1) {
-      // all but the last prompt token as row batches (as generate does): a
-      // 300-token prompt of the Qwen3-0.6B shape in 6 ms instead of 300 steps
-      // of 0.7 ms. A prompt past the context fills it and then fails at the
-      // first token that does not fit, as token-by-token steps would.
+    if (prompt_rows && e->batched_prefill && n_suffix > 1) {
+      // all but the last prompt token. A prompt past the context fills it and
+      // then fails at the first token that does not fit, as single steps would.
       const size_t room = (size_t)(e->cfg.ctx - e->pos);
       done = std::min(n_suffix - 1, room);
       append_rows(e, prompt + prefix, done);
@@ -3168,7 +3171,7 @@ int chonk_engine_generate(chonk_engine* e, const int32_t* prompt, size_t n_promp
     std::vector<int32_t> ids;
     // GPT-2 follows generateGptWgsl from the host (one more step at the end)
     if (e->cfg.gpt)
-      generate_stepped(e, prompt, n_prompt, max_new_tokens, s, nullptr, nullptr, &ids, stats);
+      generate_stepped(e, prompt, n_prompt, max_new_tokens, s, nullptr, nullptr, true, &ids, stats);
     else
       generate(e, prompt, n_prompt, max_new_tokens, s, &ids, stats);
     const size_t n = std::min(ids.size(), out_cap);
@@ -3183,7 +3186,7 @@ int chonk_engine_generate_stepped(chonk_engine* e, const int32_t* prompt, size_t
   return api(e, [&] {
     if (!prompt && n_prompt) throw Error(CHONK_EINVAL, "null prompt");
     std::vector<int32_t> ids;
-    generate_stepped(e, prompt, n_prompt, max_new_tokens, s, callback, user, &ids, stats);
+    generate_stepped(e, prompt, n_prompt, max_new_tokens, s, callback, user, false, &ids, stats);
     const size_t n = std::min(ids.size(), out_cap);
     if (out_ids && n) std::memcpy(out_ids, ids.data(), n * 4);
     if (n_out) *n_out = ids.size();
