@@ -2421,7 +2421,7 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
     return ps;
   };
   // one launch over two or three matrices of one type and K whose results are
-  // column ranges of one partial-sum row (segments start on 64-row tiles);
+  // column ranges of one partial-sum row (segments start at multiples of 64 rows);
   // returns false (nothing launched) when the matrices do not qualify
   // (epi GEMM_SWIGLU / GEMM_GEGLU: gate and up, leaving the product, where a launch can)
   auto gemm_fused = [&](std::initializer_list<const DevMat*> ms, int rows, PartSum* out, int epi = GEMM_STORE,

@@ -16,8 +16,8 @@ enum GemmEpi : int32_t { GEMM_STORE = 0, GEMM_ADD = 1, GEMM_SWIGLU = 2, GEMM_GEG
 struct GemmArgs {
   QMat w;                 // striped weights, N = w.n rows of K = w.k
   // a fused launch over up to three matrices of one type and K (e.g. q | k | v):
-  // output rows [0, n1) come from w, [n1, n2) from w2, [n2, n_all) from w3; the
-  // segment starts are multiples of the 64-row tile. n_all = 0: w alone.
+  // output rows [0, n1) come from w, [n1, n2) from w2, [n2, n_all) from w3 (n_all =
+  // n2: two matrices); the segment starts are multiples of 64 rows. n_all = 0: w alone.
   QMat w2, w3;
   int32_t n1, n2, n_all, pad0;
   const _Float16* xh;     // activation planes (plane_at), zero past K

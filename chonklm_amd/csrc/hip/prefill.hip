@@ -2191,8 +2191,10 @@ hipError_t launch_gemm_deferred(const GemmArgs& a0, float* region, int64_t regio
   GemmArgs a = a0;
   const int N = a.n_all ? a.n_all : a.w.n;
   if (a.n_all) {
-    // fused segments: one type and K, in order, at multiples of 64 rows
-    if (a.n1 <= 0 || a.n1 % kSkRows || a.n2 < a.n1 || a.n2 % kSkRows || a.n_all < a.n2 || a.w2.type != a.w.type ||
+    // fused segments: one type and K, in order, starting at multiples of 64 rows
+    // (n2 starts a segment only where there is a third: k of two matrices may end anywhere)
+    if (a.n1 <= 0 || a.n1 % kSkRows || a.n2 < a.n1 || (a.n_all > a.n2 && a.n2 % kSkRows) || a.n_all < a.n2 ||
+        a.w2.type != a.w.type ||
         a.w3.type != a.w.type || a.w2.k != a.w.k || a.w3.k != a.w.k || a.w.n != a.n1 ||
         (a.n2 > a.n1 && a.w2.n != a.n2 - a.n1) || (a.n_all > a.n2 && a.w3.n != a.n_all - a.n2))
       return hipErrorInvalidValue;

@@ -11,7 +11,8 @@ import numpy as np
 import pytest
 
 from chonklm_amd import WORKLOADS, ChonkError, generate_llama_wgsl, load_llama_wgsl_model
-from chonklm_amd import runtime
+from chonklm_amd import runtime, write_synthetic_gguf
+from chonklm_amd.registry import SynthSpec, Workload
 from tests.conftest import rel_err
 
 pytestmark = pytest.mark.gpu
@@ -73,7 +74,7 @@ def _same_state(name, parts, synth, max_context=None):
     the next two steps. With the fp32 cache both sides are fp32-class sums of the same
     values in another order: 3e-7 apart per layer at most, over at most 32 layers and
     two linear branches each, so 2e-5 bounds them."""
-    w = WORKLOADS[name]
+    w = name if isinstance(name, Workload) else WORKLOADS[name]
     md = w.model_def(synth(name), kv_dtype="f32")
     if max_context:
         md.max_context = max_context
@@ -121,3 +122,14 @@ def test_prompt_of_two_passes_equals_steps(name, synth):
 def test_prompt_rows_of_the_workload_shapes_equal_steps(name, synth):
     """Feed-forward rows over 4096 elements (eight per thread) and 48 SSM heads."""
     _same_state(name, (70, 3), synth)
+
+
+@pytest.mark.parametrize("recipe", ["q4_k_m", "q8_0"])
+@pytest.mark.parametrize("heads,kv_heads", [(6, 3), (4, 1), (6, 2), (3, 1)])
+def test_prompt_rows_of_32_wide_heads_equal_steps(heads, kv_heads, recipe, tmp_path):
+    """q and k in one GEMM where k (32 or 96 rows) ends inside a 64-row tile; one row tile and several."""
+    spec = SynthSpec(arch="llama", recipe=recipe, hidden=256, layers=3, heads=heads, kv_heads=kv_heads, head_dim=32,
+                     ffn=512, vocab=600, context_length=512, seed=heads)
+    w = Workload("heads32", spec, max_context=300, eos_ids=[2], prompt_tokens=8, decode_tokens=8)
+    path = write_synthetic_gguf(w, str(tmp_path / "m.gguf"))
+    _same_state(w, (17, 200), lambda _: path)
