@@ -2,7 +2,7 @@
 //
 //   Q4_K, Q5_K  W = d (sc (q - z)) + c,   z = 8, 16,  c = z d sc - dmin m per 32 k
 //   Q6_K        W = d (sc (q - 32))
-//   Q8_0, Q5_0  W = d q,  d (q - 16)
+//   Q8_0, Q5_0  W = d q,  d (q - 16) per 32 k
 //   Q5_1        W = d q + m, formed in fp32
 //
 // sc (q - z) of Q4_K and Q5_K is an integer below 2^10, exact in one fp16 plane, so
@@ -10,17 +10,27 @@
 // per 16x16x32 step where fp16 hi + lo weights take three, and no rounded
 // weight): the sums of a 256-k super-block are scaled by d once, and c, which
 // is constant over 32 k, meets the sums of x over those 32 k in one more MFMA
-// per super-block. sc (q - 32) of Q6_K has 13 bits and d q up to 19, so the
-// other types keep two planes, split exactly (h = fp16(v), l = v - h by one fma).
-// Codes become fp16 by byte permutes under the exponent of 1024 and one or
-// two packed fp16 instructions per pair, about 1.5 VALU instructions per weight.
+// per super-block. The codes of Q8_0 and Q5_0 are exact in one plane too; their d
+// changes every 32 k, which is one 16x16x32 step: its two products start from
+// zero and join the sums of 256 k by one fma with d. sc (q - 32) of Q6_K has 13
+// bits and Q5_1's d q + m more, so these keep two planes, split exactly (h =
+// fp16(v), l = v - h). Codes become fp16 by byte permutes under the exponent of
+// 1024 and one or two packed fp16 instructions per pair, about 1.5 VALU
+// instructions per weight.
+//
+// Chains are kept short: the matrix core rounds several times per step at the
+// size of what it adds to. Q8_0 as two planes in one chain over K was 1.6e-7 to
+// 3.6e-7 from float64 (8.4e-8 to 9.6e-8 now; 9216 x 1024 at 300 rows 32.7 -> 29.9 us,
+// 3376 x 768 at 2047 49.3 -> 48.3, 1024 x 1024 at 200 13.8 -> 14.1), and the logits
+// after a Granite or LFM2 Q8_0 prompt (fp32 cache) 1.4e-6 or 2.6e-6, where a prompt
+// in decode steps leaves 8.5e-7 or 1.53e-6 (8.5e-7 and 1.53e-6 now).
 //
 // Against the three-product GEMM over fp32-dequantized hi + lo weights that it
-// replaces (MI355X, 2047 token rows): Q4_K 4096 x 1024 95.0 -> 47.9 us, 6144 x 1024
-// 139.5 -> 65.2, Q6_K 1024 x 3072 90.6 -> 41.2, Q8_0 3376 x 768 74.3 -> 41.1; error
-// against float64 3.6e-7 -> 1.4e-7 (Q4_K), 6.2e-7 -> 1.7e-7 (Q6_K). What is left:
-// 16 us of the 4096-row launch are its 34 MB of fp32 results, the rest is the
-// products at the rate the matrix cores sustain beside the staging.
+// replaced (MI355X, 2047 token rows): Q4_K 4096 x 1024 95.0 -> 47.9 us, 6144 x 1024
+// 139.5 -> 65.2, Q6_K 1024 x 3072 90.6 -> 41.2; error against float64 3.6e-7 -> 1.4e-7
+// (Q4_K), 6.2e-7 -> 1.7e-7 (Q6_K). What is left: 16 us of the 4096-row launch are its
+// 34 MB of fp32 results, the rest is the products at the rate the matrix cores
+// sustain beside the staging.
 #include <hip/hip_runtime.h>
 
 #include "kernel_common.h"
@@ -97,12 +107,15 @@ template <int T>
 constexpr bool gemm_int_sb = T == QT_Q4_K || T == QT_Q5_K || T == QT_Q6_K;
 template <int T>
 constexpr bool gemm_int_offsets = T == QT_Q4_K || T == QT_Q5_K;
+// codes alone in the plane, the sums of a 32-weight block scaled by its d
 template <int T>
-constexpr int gemm_int_planes() { return gemm_int_offsets<T> ? 1 : 2; }
+constexpr bool gemm_int_blocks = T == QT_Q8_0 || T == QT_Q5_0;
+template <int T>
+constexpr int gemm_int_planes() { return gemm_int_offsets<T> || gemm_int_blocks<T> ? 1 : 2; }
 template <int T, int NI>
 constexpr size_t gemm_int_shared() {
   return sizeof(_Float16) * gemm_int_planes<T>() * 16 * NI * kIS + (gemm_int_offsets<T> ? 16 * NI * 16 * sizeof(_Float16) : 0) +
-         (gemm_int_sb<T> ? 16 * NI * sizeof(float) : 0);
+         (gemm_int_sb<T> ? 16 * NI * sizeof(float) : 0) + (gemm_int_blocks<T> ? 4 * 16 * NI * sizeof(float) : 0);
 }
 
 // 16 NI weight rows x 64 TJ token rows per workgroup; wave w owns token rows
@@ -117,14 +130,16 @@ constexpr size_t gemm_int_shared() {
 // (64-byte pieces of 16 rows at a time cost 15 us more at 4096 x 1024 x 2047).
 // GLU: the first half of the weight rows are gate rows (a.w), the second the same
 // rows of up (a.w2).
+// (BLK at NI = 4: at most 168 registers, three workgroups per CU; with 198 the 9216 x
+// 1024 launch at 300 rows takes 36.5 us instead of 29.9)
 template <int T, int NI, int TJ, bool GLU>
-__global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
+__global__ __launch_bounds__(kWg, (gemm_int_blocks<T> && NI == 4 ? 3 : 2)) void k_gemm_int(GemmArgs a) {
   extern __shared__ __align__(16) _Float16 gism[];
   constexpr int R = 16 * NI, NP = gemm_int_planes<T>(), NG = NI / 4;
-  constexpr bool SB = gemm_int_sb<T>, OFF = gemm_int_offsets<T>;
+  constexpr bool SB = gemm_int_sb<T>, OFF = gemm_int_offsets<T>, BLK = gemm_int_blocks<T>;
   _Float16* wp = gism;                                   // [NP][R][kIS]
   _Float16* cs = wp + NP * R * kIS;                      // OFF: [R][16], c of eight sub-blocks hi | lo
-  float* ds = (float*)(cs + (OFF ? R * 16 : 0));  // [R] d 2^(ws - 5) (Q6_K: d 2^ws)
+  float* ds = (float*)(cs + (OFF ? R * 16 : 0));  // [R] d 2^(ws - 5) (Q6_K: d 2^ws; BLK: [4][R], the stage's blocks)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * R, t0 = blockIdx.y * 64 * TJ;
@@ -312,13 +327,16 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
         const int u = NG * wq + g;
-        const half2_t d = splat(4 * s + u < (K >> 5) ? h2f(f.d[g]) * wsc : 0.f);
+        // (odd blocks with both signs turned: the matrix core rounds down on average, and
+        // with one sign the products were all low by up to 4e-8 of their rms, in every row alike)
+        const float sg = u & 1 ? -1.0f : 1.0f;
+        ds[u * R + wr] = 4 * s + u < (K >> 5) ? sg * (h2f(f.d[g]) * wsc) : 0.f;
+        const half2_t one = splat(sg), z = splat(sg * (T == QT_Q8_0 ? -1152.0f : -1040.0f));
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           const uint4 q4 = f.q[T == QT_Q8_0 ? 2 * g + p : g];
           const uint32_t w[4] = {q4.x, q4.y, q4.z, q4.w};
-          const _Float16 z = T == QT_Q8_0 ? 1152 : 1040;
-          half2_t vh[8], vl[8];
+          half2_t v[8];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             uint32_t b;
@@ -329,14 +347,10 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
               const uint32_t x = (f.qh[g] >> (16 * p + 4 * i)) & 15u;
               b = ((w[i] >> (4 * p)) & 0x0f0f0f0fu) | (((x | x << 7 | x << 14 | x << 21) & 0x01010101u) << 4);
             }
-            const half2_t x0 = bytes01(b) - half2_t{z, z}, x1 = bytes23(b) - half2_t{z, z};
-            vh[2 * i] = x0 * d;
-            vh[2 * i + 1] = x1 * d;
-            vl[2 * i] = __builtin_elementwise_fma(x0, d, -vh[2 * i]);
-            vl[2 * i + 1] = __builtin_elementwise_fma(x1, d, -vh[2 * i + 1]);
+            v[2 * i] = __builtin_elementwise_fma(bytes01(b), one, z);
+            v[2 * i + 1] = __builtin_elementwise_fma(bytes23(b), one, z);
           }
-          put16(rh + 32 * u + 16 * p, vh);
-          put16(rl + 32 * u + 16 * p, vl);
+          put16(rh + 32 * u + 16 * p, v);
         }
       }
     }
@@ -358,7 +372,8 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
   const char* xlb = (const char*)a.xl;
   const char* xsb = (const char*)a.xs;
 
-  float4_t acc[NI][TJ], tmp[SB ? NI : 1][TJ];
+  // (tmp: the sums of 256 k; see the merge below)
+  float4_t acc[NI][TJ], tmp[NI][TJ];
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -391,42 +406,74 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
     // the products: weight fragment f is plane f % NP of row tile f / NP % NI and
     // 32-k step f / NP / NI; AD fragments are read from LDS ahead of their use
     // (left alone, the compiler reads one at a time and waits for it)
-    constexpr int NF = SPS * NI * NP, AD = 3;
+    constexpr int NF = SPS * NI * NP, AD = BLK && TJ == 2 ? 1 : 3;
     auto frag = [&](int fi) {
       const int p = fi % NP, i = fi / NP % NI, ks = fi / NP / NI;
       return *(const half8_t*)(wp + p * R * kIS + (16 * i + col) * kIS + ks * 32 + 8 * quad);
     };
     half8_t af[AD + 1];
+    // BLK: the products of a fragment and their blocks' scales, which join tmp
+    // while the next fragment's products are issued
+    float4_t us[3][TJ], dv[AD + 1];
+    auto scale = [&](int fi) { return *(const float4_t*)(ds + (fi / NI) * R + 16 * (fi % NI) + 4 * quad); };
+    auto join = [&](int fi) {
+      const int i = fi % NI;
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float d = dv[fi % (AD + 1)][q], u = us[fi % 3][j][q];
+          tmp[i][j][q] = PAR == 0 && fi < NI ? d * u : fmaf(d, u, tmp[i][j][q]);
+        }
+    };
+    // (the small products first; with one token tile those of the fragment ahead
+    // stand between them and the large ones, which add to their result)
+    auto small = [&](int fi) {
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+        us[fi % 3][j] = mfma32(af[fi % (AD + 1)], bl[(SPS * PAR + fi / NI) % NS][j], float4_t{0.f, 0.f, 0.f, 0.f});
+    };
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int fi = 0; fi < AD; ++fi) af[fi] = frag(fi);
+    for (int fi = 0; fi < AD; ++fi) {
+      af[fi] = frag(fi);
+      if constexpr (BLK) dv[fi] = scale(fi);
+    }
 #pragma unroll
     for (int fi = 0; fi < NF; ++fi) {
       const int p = fi % NP, i = fi / NP % NI, ks = fi / NP / NI, sl = (SPS * PAR + ks) % NS;
+      if constexpr (BLK) {
+        if (fi > 0) join(fi - 1);
+        if (fi + AD < NF) dv[(fi + AD) % (AD + 1)] = scale(fi + AD);
+      }
       if (fi + AD < NF) af[(fi + AD) % (AD + 1)] = frag(fi + AD);
       if (p == 0 && i == 0) load_x(SPS * s + ks + LA, (SPS * PAR + ks + LA) % NS);
       const half8_t w = af[fi % (AD + 1)];
-      auto& dst = [&]() -> auto& {
-        if constexpr (SB)
-          return tmp[i];
-        else
-          return acc[i];
-      }();
-      const bool first = SB && PAR == 0 && ks == 0 && p == 0;
+      if constexpr (BLK) {
+        if (TJ == 2 || fi == 0) small(fi);
+        if (TJ == 1 && fi + 1 < NF) small(fi + 1);
 #pragma unroll
-      for (int j = 0; j < TJ; ++j) dst[j] = mfma32(w, bh[sl][j], first ? float4_t{0.f, 0.f, 0.f, 0.f} : dst[j]);
+        for (int j = 0; j < TJ; ++j) us[fi % 3][j] = mfma32(w, bh[sl][j], us[fi % 3][j]);
+        continue;
+      }
+      const bool first = (!SB || PAR == 0) && ks == 0 && p == 0;
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) tmp[i][j] = mfma32(w, bh[sl][j], first ? float4_t{0.f, 0.f, 0.f, 0.f} : tmp[i][j]);
       if (p == 0) {
 #pragma unroll
-        for (int j = 0; j < TJ; ++j) dst[j] = mfma32(w, bl[sl][j], dst[j]);
+        for (int j = 0; j < TJ; ++j) tmp[i][j] = mfma32(w, bl[sl][j], tmp[i][j]);
       }
     }
-    // (schedule: AD LDS reads, then per fragment one read and its products)
-    __builtin_amdgcn_sched_group_barrier(0x100, AD, 0);
+    if constexpr (BLK) join(NF - 1);
+    // (schedule: AD LDS reads, then per fragment one read and its products; BLK:
+    // two reads, the products and the fused multiplies of the fragment before)
+    __builtin_amdgcn_sched_group_barrier(0x100, BLK ? 2 * AD : AD, 0);
 #pragma unroll
     for (int fi = 0; fi < NF; fi += NP) {
       if (fi % (NP * NI) == 0) __builtin_amdgcn_sched_group_barrier(0x20, 2 * TJ, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, BLK ? 2 : 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x8, 2 * TJ, 0);
+      if constexpr (BLK) __builtin_amdgcn_sched_group_barrier(0x2, 4 * TJ, 0);
       if constexpr (NP == 2) {
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x8, TJ, 0);
@@ -449,6 +496,15 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_int(GemmArgs a) {
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) acc[i][j][q] = fmaf(d4[q], tmp[i][j][q], acc[i][j][q]);
+      }
+    }
+    if constexpr (!SB) {
+      // The sums of 256 k (Q5_1: of 128, which are longer chains) join the total in one addition.
+      if (!BLK || PAR == 1 || s + 1 >= s_hi) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < TJ; ++j) acc[i][j] += tmp[i][j];
       }
     }
   };

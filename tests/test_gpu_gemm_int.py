@@ -41,6 +41,26 @@ def test_tiles_of_every_type(tname, row_len, n_rows, n_tok):
     assert err.max() <= 5e-6, f"{tname}: {err.max():.2e}"
 
 
+# Bars of the 2-norm against float64, in units of 2^-25 (rms of one rounding; a chain
+# of n sums of like size rounds as sqrt(n / 2) of them at the total's size). Codes alone
+# (Q8_0, Q5_0): one rounding per 32 k, chains of 8, K / 256 <= 12 of those: sqrt(1 + 4 +
+# 6) = 3.3, with the operands' 22 bits 3.6. Q5_1: chains of 12 matrix steps, about four
+# roundings each, K / 128 <= 24 of those: sqrt(24 + 12) = 6, with the dropped lo x lo 6.3.
+@pytest.mark.parametrize("n_rows,row_len,n_tok", [(1024, 1024, 200), (768, 3072, 200), (576, 576, 48), (3376, 768, 2047),
+                                                  (9216, 1024, 300), (130, 160, 515)])
+@pytest.mark.parametrize("tname,bar", [("Q8_0", 4.2), ("Q5_0", 4.2), ("Q5_1", 7.0)])
+def test_error_of_32_weight_blocks(tname, bar, n_rows, row_len, n_tok):
+    rng = np.random.default_rng(n_rows + row_len)
+    blocks = random_blocks(TYPES[tname], n_rows * row_len, rng)
+    w = orc.dequant(TYPES[tname], blocks, n_rows * row_len).reshape(n_rows, row_len).astype(np.float64)
+    x = rng.standard_normal((n_tok, row_len)).astype(np.float32)
+    got, _ = gpu_gemm(TYPES[tname], blocks, n_rows, row_len, x)
+    rows = np.unique(np.r_[0:16, n_tok // 2, n_tok - 8:n_tok])
+    want = x[rows].astype(np.float64) @ w.T
+    err = np.linalg.norm(got[rows] - want) / np.linalg.norm(want)
+    assert err <= bar * 2.0 ** -25, f"{tname}: {err:.2e}"
+
+
 @pytest.mark.parametrize("name,parts", [
     ("qwen3-0.6b-q4_k_m", (300, 600)),   # gate * up inside the GEMM (SwiGLU), one wave's and four waves' rows
     ("gemma3-270m-q4_k_m", (300,)),      # ... with GELU
