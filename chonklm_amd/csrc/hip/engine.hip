@@ -16,6 +16,7 @@
 // hipGraph per step kind (with / without logits) and replayed. Device-driven
 // generation appends sampled ids on the device and checks EOS there, so a
 // whole generate call needs no per-token host round trip.
+#include <climits>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -592,7 +593,7 @@ struct chonk_engine {
   int32_t cached_next = 0;
   uint64_t weight_bytes_per_token = 0;
   // batched prompt processing: row buffers allocated on first use
-  bool batched_prefill = true;
+  int rows_min = 1;  // fewest prompt tokens that go through the row-batch pass (fewer: decode steps)
   uint8_t* scratch = nullptr;  // device address of this GPU's no-allocation prompt-pass scratch
   int noalloc_rows = 0;        // rows one chonk_engine_prefill_noalloc call may take (0: none)
   void* pf_mem = nullptr;
@@ -2125,13 +2126,20 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
   const char* pv = std::getenv("CHONK_PREFILL");
   // (the row-batch glue kernels hold a row of at most kPfRowMax elements in registers)
   const int widest = std::max({c.hidden, c.heads * c.hd, c.ffn, c.ssm_inner});
-  e->batched_prefill = !(pv && std::strcmp(pv, "token") == 0) && widest <= kPfRowMax;
+  const bool batched = !(pv && std::strcmp(pv, "token") == 0) && widest <= kPfRowMax;
+  // One or two tokens run as decode steps (a pass costs its launches whatever its
+  // rows). Then one logits step, ms, as steps / as rows, for 1, 2, 3 tokens: GPT-2
+  // 0.72 / 1.05, 1.00 / 1.07, 1.28 / 1.06; LFM2 Q8_0 1.05 / 1.53, 1.47 / 1.56, 1.90 / 1.58;
+  // Granite Q8_0 1.74 / 2.67, 2.44 / 2.72, 3.16 / 2.76; OpenELM 1.02 / 1.45, 1.46 / 1.48,
+  // 1.90 / 1.48. Llama-family models with rows of at most 4096 elements take the pass
+  // at any length, as the no-allocation call and batches of theirs do.
+  const bool plain_rows = !c.gpt && !c.lfm && !c.granite && widest <= 4096;
+  e->rows_min = !batched ? INT_MAX : plain_rows ? 1 : 3;
   // the no-allocation prompt pass: as many rows (a multiple of 16, at most one
   // full pass) as fit the scratch with this model's row buffers (the llama
   // family, rows of at most 4096 elements)
   e->scratch = scratch_address(e->device);
-  e->noalloc_rows =
-      e->batched_prefill && !c.gpt && !c.lfm && !c.granite && widest <= 4096 ? noalloc_rows_for(c) : 0;
+  e->noalloc_rows = batched && plain_rows ? noalloc_rows_for(c) : 0;
   const char* ng = std::getenv("CHONK_NO_GRAPH");
   e->use_graph = !(ng && ng[0] == '1');
   for (const Launch& L : e->kernels_logits)
@@ -2868,7 +2876,7 @@ void generate(chonk_engine* e, const int32_t* prompt, size_t n_prompt, int32_t m
   } else {
     std::vector<int32_t> suf(prompt + prefix, prompt + n_prompt);
     HIP_OK(hipMemcpy(e->hist + e->pos, suf.data(), suf.size() * 4, hipMemcpyHostToDevice));
-    if (e->batched_prefill && n_suffix > 1) {
+    if (n_suffix > 1 && n_suffix - 1 >= (size_t)e->rows_min) {
       // all but the last prompt token as row batches, the last one as a step
       prefill_rows(e, suf.data(), (int)n_suffix - 1);
       st.pos = e->pos + (int)n_suffix - 1;
@@ -2985,7 +2993,7 @@ void generate_stepped(chonk_engine* e, const int32_t* prompt, size_t n_prompt, i
     next = e->cached_next;
   } else {
     size_t done = 0;
-    if (prompt_rows && e->batched_prefill && n_suffix > 1) {
+    if (prompt_rows && n_suffix > 1 && n_suffix - 1 >= (size_t)e->rows_min) {
       // all but the last prompt token. A prompt past the context fills it and
       // then fails at the first token that does not fit, as single steps would.
       const size_t room = (size_t)(e->cfg.ctx - e->pos);
@@ -3117,8 +3125,9 @@ int chonk_engine_prefill(chonk_engine* e, const int32_t* tokens, size_t n) {
     for (size_t i = 0; i < n; ++i) check_token(e, tokens[i]);
     if ((int64_t)e->pos + (int64_t)n > e->cfg.ctx)
       throw context_exhausted(e);
-    if (!e->batched_prefill) {
-      // token by token through the decode step (rows wider than kPfRowMax, or CHONK_PREFILL=token)
+    if (n < (size_t)e->rows_min) {
+      // token by token through the decode step (a few tokens, rows wider than
+      // kPfRowMax, or CHONK_PREFILL=token)
       for (size_t i = 0; i < n; ++i) run_token(e, tokens[i], false, nullptr, nullptr, 0, nullptr, 0);
       e->known_token_pos = -1;
       e->logits_valid = false;

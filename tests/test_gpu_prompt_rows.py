@@ -133,3 +133,55 @@ def test_prompt_rows_of_32_wide_heads_equal_steps(heads, kv_heads, recipe, tmp_p
     w = Workload("heads32", spec, max_context=300, eos_ids=[2], prompt_tokens=8, decode_tokens=8)
     path = write_synthetic_gguf(w, str(tmp_path / "m.gguf"))
     _same_state(w, (17, 200), lambda _: path)
+
+
+@pytest.mark.parametrize("name", ["tiny-gpt2", "tiny-lfm2", "tiny-granite", "openelm-270m-q4_k_m"])
+def test_one_or_two_tokens_are_steps(name, synth):
+    """Prompts of one and two tokens run as decode steps on these runtimes: the logits to the bit."""
+    w = WORKLOADS[name]
+    eng = _load(name, synth).engine
+    tokens = np.random.default_rng(1).integers(0, w.spec.vocab, 20).tolist()
+    for n in (1, 2):
+        got = []
+        for rows in (True, False):
+            eng.reset()
+            for t in tokens[:9]:
+                eng.run_token(t, False)
+            if rows:
+                eng.prefill(tokens[9:9 + n])
+            else:
+                for t in tokens[9:9 + n]:
+                    eng.run_token(t, False)
+            assert eng.position == 9 + n
+            eng.run_token(tokens[15], True)
+            got.append(eng.read_logits().copy())
+        assert (got[0] == got[1]).all(), f"{n} tokens"
+    eng.dispose()
+
+
+@pytest.mark.parametrize("more", [1, 2, 3])
+@pytest.mark.parametrize("name", ["tiny-gpt2", "tiny-lfm2", "tiny-granite"])
+def test_continued_conversation_equals_steps(name, more, synth):
+    """A second call whose prompt adds one to three tokens to the first call's: the ids and
+    logits of run_token over those tokens, to the bit."""
+    w = WORKLOADS[name]
+    loaded = _load(name, synth)
+    eng, generate = loaded.engine, GENERATE[loaded.runtime]
+    rng = np.random.default_rng(more)
+    first = rng.integers(0, w.spec.vocab, 12).tolist()
+    talk = first + generate(loaded, first, 4)["ids"]
+    added = rng.integers(0, w.spec.vocab, more).tolist()
+    got = generate(loaded, talk + added, 3)["ids"]
+    logits = eng.read_logits().copy()
+    eng.reset()
+    eng.prefill(first[:-1])
+    for t in first[-1:] + talk[len(first):] + added[:-1]:
+        eng.run_token(t, False)
+    want = [eng.run_token(added[-1], True)]
+    while len(want) < 3 and want[-1] not in w.eos_ids:
+        want.append(eng.run_token(want[-1], True))
+    if want[-1] not in w.eos_ids:
+        eng.run_token(want[-1], True)  # (these loops also run the last id)
+    assert got == want
+    assert (eng.read_logits() == logits).all()
+    eng.dispose()
