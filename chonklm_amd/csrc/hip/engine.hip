@@ -552,6 +552,8 @@ struct chonk_engine {
   uint32_t *pen_bits = nullptr, *seen_bits = nullptr;
   int groups = 0, chunk = 0, nchunk = 0;
   bool dec_attn = false;          // per-phase attention: k_attn_dec over dnchunk chunks
+  // k_attn_dec only while the engine is alone on its device, k_attention beside others (fp32 cache)
+  bool solo_attn = false;
   int dnchunk = 0;                // workgroup chunks of dsub x 64 positions
   int dsub = 1;
   tagged_t* dpart = nullptr;      // k_attn_dec chunk rows
@@ -567,15 +569,15 @@ struct chonk_engine {
   std::vector<Launch> step_logits, step_plain;
   hipGraph_t graph_logits = nullptr, graph_plain = nullptr;
   hipGraphExec_t exec_logits = nullptr, exec_plain = nullptr;
-  // the same steps with the q|k|v matvec and the attention as separate launches:
-  // what the engine replays while another engine lives on its device (fuse_qkv)
+  // what the engine replays while another engine lives on its device (fuse_qkv: the
+  // q|k|v matvec and the attention as separate launches; solo_attn: k_attention)
   std::vector<Launch> step_logits_sep, step_plain_sep;
   hipGraph_t graph_logits_sep = nullptr, graph_plain_sep = nullptr;
   hipGraphExec_t exec_logits_sep = nullptr, exec_plain_sep = nullptr;
   // kMultiSteps logits steps in one graph: what runs of consecutive steps with
   // no host work between them replay (one launch gap per kMultiSteps tokens)
-  hipGraph_t graph_multi = nullptr;
-  hipGraphExec_t exec_multi = nullptr;
+  hipGraph_t graph_multi = nullptr, graph_multi_sep = nullptr;  // (sep: solo_attn)
+  hipGraphExec_t exec_multi = nullptr, exec_multi_sep = nullptr;
   bool registered = false;  // counted in device_engines()
   // pinned host staging
   DevState* h_state = nullptr;
@@ -1068,8 +1070,9 @@ const float2* rope_cs_table(chonk_engine* e, uint32_t theta, int hd) {
   return p;
 }
 
-// fuse: join each qualifying layer's q|k|v matvec and attention (fuse_qkv engines)
-void build_steps(chonk_engine* e, bool fuse) {
+// fuse: join each qualifying layer's q|k|v matvec and attention (fuse_qkv engines);
+// dec: k_attn_dec (engines with dec_attn), else k_attention
+void build_steps(chonk_engine* e, bool fuse, bool dec) {
   const ModelCfg& c = e->cfg;
   const int H = c.hidden;
   auto mv_base = [&]() {
@@ -1300,7 +1303,7 @@ void build_steps(chonk_engine* e, bool fuse) {
       t.kc = Ld.kc;
       t.vc = Ld.vc;
       t.part = e->part;
-      t.cnt = e->cnt;
+      t.cnt = dec ? e->cnt : e->cnt + c.kv_heads;  // (epochs; arrivals, zero between launches)
       t.out = e->attn;
       t.st = e->st;
       t.heads = lc.heads;
@@ -1323,7 +1326,7 @@ void build_steps(chonk_engine* e, bool fuse) {
       t.tpp = attn_threads_per_position(c.hd, e->chunk, (int)e->kv_elem);
       L.shmem = attn_shared_bytes(G, c.hd, e->chunk, e->nchunk, e->kv_elem);
       L.grid = lc.kv_heads * e->nchunk;
-      if (e->dec_attn) {
+      if (dec) {
         t.variant = 1;
         t.tpart = e->dpart;
         t.rope_cs = rope_cs_table(e, c.layer[i].theta, c.hd);
@@ -1587,7 +1590,10 @@ void capture(chonk_engine* e, const std::vector<Launch>& steps, hipGraph_t* g, h
 // threads could together exceed the device and wait until the time bound.
 // The first engine on a device that qualifies claims the device; engines
 // created while the claim is held use the arrival-counter k_attention (no
-// waiting). The claim ends with the engine.
+// waiting). The claim ends with the engine. Engines with the fp32 cache claim
+// nothing, so that they take it from no fp16 engine: they run k_attn_dec while
+// they are alone on the device (solo_attn, under DeviceEngines' lock) and
+// k_attention otherwise.
 struct SpinClaims {
   std::mutex mu;
   std::map<int, const chonk_engine*> owner;
@@ -1618,7 +1624,8 @@ void release_spin(int device, const chonk_engine* e) {
 // its resident workgroups hold while the rest of the grid waits behind it, so
 // an engine replays its fused steps only while it is the only engine on its
 // device (under this lock, which also orders a new engine's registration after
-// the fused steps already queued: registration waits for them to finish).
+// the fused steps already queued: registration waits for them to finish). An
+// engine with solo_attn does the same with its k_attn_dec steps.
 struct DeviceEngines {
   std::mutex mu;
   std::map<int, std::vector<chonk_engine*>> live;
@@ -1634,6 +1641,12 @@ void register_engine(chonk_engine* e) {
   d.live[e->device].push_back(e);
   e->registered = true;
 }
+// Whether no other engine lives on e's device; none registers while l is held.
+bool alone(const chonk_engine* e, std::unique_lock<std::mutex>& l) {
+  DeviceEngines& d = device_engines();
+  l = std::unique_lock<std::mutex>(d.mu);
+  return d.live[e->device].size() <= 1;
+}
 void unregister_engine(chonk_engine* e) {
   if (!e->registered) return;
   DeviceEngines& d = device_engines();
@@ -1645,10 +1658,10 @@ void unregister_engine(chonk_engine* e) {
 
 void engine_free(chonk_engine* e) {
   if (!e) return;
-  unregister_engine(e);
-  release_spin(e->device, e);
   (void)hipSetDevice(e->device);
   if (e->stream) (void)hipStreamSynchronize(e->stream);
+  unregister_engine(e);
+  release_spin(e->device, e);
   if (e->exec_logits) (void)hipGraphExecDestroy(e->exec_logits);
   if (e->exec_plain) (void)hipGraphExecDestroy(e->exec_plain);
   if (e->graph_logits) (void)hipGraphDestroy(e->graph_logits);
@@ -1659,6 +1672,8 @@ void engine_free(chonk_engine* e) {
   if (e->graph_plain_sep) (void)hipGraphDestroy(e->graph_plain_sep);
   if (e->exec_multi) (void)hipGraphExecDestroy(e->exec_multi);
   if (e->graph_multi) (void)hipGraphDestroy(e->graph_multi);
+  if (e->exec_multi_sep) (void)hipGraphExecDestroy(e->exec_multi_sep);
+  if (e->graph_multi_sep) (void)hipGraphDestroy(e->graph_multi_sep);
   e->weights.release();
   e->state.release();
   uncached_pool().give_back(e->device, e->uncached);
@@ -1876,12 +1891,13 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
         e->dec_attn = false;
     }
     // (another engine on this GPU holds the spin-merging attention: k_attention)
-    if (e->dec_attn && !claim_spin(e->device, e.get())) e->dec_attn = false;
+    e->solo_attn = e->dec_attn && kv32;
+    if (e->dec_attn && !kv32 && !claim_spin(e->device, e.get())) e->dec_attn = false;
     // the q|k|v matvec joins the attention launch where the layer allows it
     // (build_steps checks the instance and the grid's residency per layer);
     // CHONK_FUSE=0 keeps them apart
     const char* fv = std::getenv("CHONK_FUSE");
-    // (the fp32 cache's rows leave the joint launch no registers: separate launches)
+    // (the joint launch reads an fp16 cache)
     e->fuse_qkv = e->dec_attn && e->dsub == 1 && !kv32 && !(fv && std::strcmp(fv, "0") == 0);
   }
   const size_t kv_bytes = (size_t)kvdim * c.ctx * e->kv_elem;
@@ -2081,10 +2097,10 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
   {
     const size_t rowf = ((size_t)G * (c.hd + 2) + 3) & ~(size_t)3;
     const size_t part_bytes = align256((size_t)c.kv_heads * std::max(e->nchunk, e->dnchunk) * rowf * 4);
-    e->uncached = uncached_pool().take(e->device, part_bytes + align256((size_t)c.kv_heads * 4));
+    e->uncached = uncached_pool().take(e->device, part_bytes + align256((size_t)2 * c.kv_heads * 4));
     e->part = (float*)e->uncached;
     e->cnt = (uint32_t*)((uint8_t*)e->uncached + part_bytes);
-    HIP_OK(hipMemset(e->cnt, 0, (size_t)c.kv_heads * 4));
+    HIP_OK(hipMemset(e->cnt, 0, (size_t)2 * c.kv_heads * 4));
   }
   if (e->dec_attn) e->dpart = (tagged_t*)e->state.take(dpart_bytes);
   if (e->fuse_qkv) e->qkv_tag = (tagged_t*)e->state.take(qkv_tag_bytes);
@@ -2111,11 +2127,13 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
 
   HIP_OK(init_kernel_attributes());
   HIP_OK(init_gemm_attributes());
-  build_steps(e.get(), false);
-  if (e->fuse_qkv) {
+  build_steps(e.get(), false, e->dec_attn && !e->solo_attn);
+  if (e->fuse_qkv || e->solo_attn) {
     e->step_logits_sep = e->kernels_logits;
     e->step_plain_sep = e->kernels_plain;
-    build_steps(e.get(), true);
+    build_steps(e.get(), e->fuse_qkv, true);
+  }
+  if (e->fuse_qkv) {
     bool any = false;
     for (const Launch& L : e->kernels_logits) any = any || L.kind == Launch::QKVATTN;
     e->fuse_qkv = any;  // (no layer qualified: one set of steps)
@@ -2142,17 +2160,20 @@ void create_engine(const chonk_model_def* def, std::unique_ptr<ByteSource> src, 
   e->noalloc_rows = batched && plain_rows ? noalloc_rows_for(c) : 0;
   const char* ng = std::getenv("CHONK_NO_GRAPH");
   e->use_graph = !(ng && ng[0] == '1');
-  for (const Launch& L : e->kernels_logits)
-    if (L.shmem > lds_limit())
-      throw Error(CHONK_EINVAL, "kernel " + L.name + " needs " + std::to_string(L.shmem) + " bytes of LDS, above the " +
-                                    std::to_string(lds_limit()) + "-byte limit of this device");
+  for (const std::vector<Launch>* steps : {&e->kernels_logits, &e->step_logits_sep})
+    for (const Launch& L : *steps)
+      if (L.shmem > lds_limit())
+        throw Error(CHONK_EINVAL, "kernel " + L.name + " needs " + std::to_string(L.shmem) + " bytes of LDS, above the " +
+                                      std::to_string(lds_limit()) + "-byte limit of this device");
   capture(e.get(), e->step_plain, &e->graph_plain, &e->exec_plain);
   capture(e.get(), e->step_logits, &e->graph_logits, &e->exec_logits);
   if (e->use_graph) capture(e.get(), e->step_logits, &e->graph_multi, &e->exec_multi, kMultiSteps);
-  if (e->fuse_qkv) {
+  if (e->fuse_qkv || e->solo_attn) {
     capture(e.get(), e->step_plain_sep, &e->graph_plain_sep, &e->exec_plain_sep);
     capture(e.get(), e->step_logits_sep, &e->graph_logits_sep, &e->exec_logits_sep);
   }
+  if (e->use_graph && e->solo_attn)
+    capture(e.get(), e->step_logits_sep, &e->graph_multi_sep, &e->exec_multi_sep, kMultiSteps);
   *out = e.release();
 }
 
@@ -2169,20 +2190,17 @@ void check_injected_failure(chonk_engine* e, const char* where) {
 // or (CHONK_NO_GRAPH=1, for profilers that cannot trace graph launches) the
 // same launches issued one by one. Runs of kMultiSteps logits steps replay the
 // multi-step graph. An engine with fused steps replays them (and the
-// multi-step graph) only while it is alone on its device.
+// multi-step graph) only while it is alone on its device, one with solo_attn its
+// k_attn_dec steps.
 void replay(chonk_engine* e, bool logits, int64_t n = 1) {
   while (n > 0) {
     check_injected_failure(e, "hipGraphLaunch");
     std::unique_lock<std::mutex> l;
-    bool sep = false;
-    if (e->fuse_qkv) {
-      DeviceEngines& d = device_engines();
-      l = std::unique_lock<std::mutex>(d.mu);
-      sep = d.live[e->device].size() > 1;
-    }
+    const bool sep = (e->fuse_qkv || e->solo_attn) && !alone(e, l);
     if (e->use_graph) {
-      if (logits && !sep && e->exec_multi && n >= kMultiSteps && !multi_off()) {
-        HIP_OK(hipGraphLaunch(e->exec_multi, e->stream));
+      const hipGraphExec_t multi = sep ? e->exec_multi_sep : e->exec_multi;
+      if (logits && multi && n >= kMultiSteps && !multi_off()) {
+        HIP_OK(hipGraphLaunch(multi, e->stream));
         n -= kMultiSteps;
         continue;
       }
@@ -2194,6 +2212,12 @@ void replay(chonk_engine* e, bool logits, int64_t n = 1) {
     }
     --n;
   }
+}
+
+// The logits step's kernels for timing one by one: of a solo_attn engine those a
+// replay would launch now (with l held until the last has finished).
+const std::vector<Launch>& timed_kernels(const chonk_engine* e, std::unique_lock<std::mutex>& l) {
+  return e->solo_attn && !alone(e, l) ? e->step_logits_sep : e->kernels_logits;
 }
 
 void upload_state_fields(chonk_engine* e, const DevState& s) {
@@ -3102,7 +3126,8 @@ int chonk_engine_info_get(const chonk_engine* e, chonk_engine_info* out) {
   out->kernels_per_step = (int32_t)e->kernels_logits.size();
   out->persistent_step = 0;  // (the one-launch-per-token step was retired: the graph ran twice as fast)
   out->noalloc_prefill_rows = e->noalloc_rows;
-  out->spin_attention = e->dec_attn ? 1 : 0;
+  std::unique_lock<std::mutex> l;
+  out->spin_attention = e->dec_attn && (!e->solo_attn || alone(e, l)) ? 1 : 0;
   out->fused_attention = 0;
   for (const Launch& L : e->kernels_logits) out->fused_attention += L.kind == Launch::QKVATTN ? 1 : 0;
   return CHONK_OK;
@@ -3347,10 +3372,12 @@ int chonk_engine_time_kernels(chonk_engine* e, const int32_t* ids, int32_t n_ids
   return api(e, [&] {
     const ModelCfg& c = e->cfg;
     if (!ids || n_ids <= 0 || rounds <= 0 || !us_per_launch) throw Error(CHONK_EINVAL, "bad kernel list or rounds");
+    std::unique_lock<std::mutex> l;
+    const std::vector<Launch>& kernels = timed_kernels(e, l);
     std::vector<Launch> run;
     for (int i = 0; i < n_ids; ++i) {
-      if (ids[i] < 0 || ids[i] >= (int32_t)e->kernels_logits.size()) throw Error(CHONK_EINVAL, "bad kernel id");
-      Launch L = e->kernels_logits[(size_t)ids[i]];
+      if (ids[i] < 0 || ids[i] >= (int32_t)kernels.size()) throw Error(CHONK_EINVAL, "bad kernel id");
+      Launch L = kernels[(size_t)ids[i]];
       if (L.kind == Launch::SEL) throw Error(CHONK_EINVAL, "the select kernel advances the position; not timed alone");
       if (L.kind == Launch::MV) L.mv.advance_pos = 0;
       run.push_back(L);
@@ -3385,9 +3412,11 @@ int chonk_engine_bench_kernel(chonk_engine* e, int32_t kernel_id, int32_t reps, 
                               size_t name_len, uint64_t* bytes) {
   return api(e, [&] {
     const ModelCfg& c = e->cfg;
-    if (kernel_id < 0 || kernel_id >= (int32_t)e->kernels_logits.size() || reps < 0)
+    std::unique_lock<std::mutex> l;
+    const std::vector<Launch>& kernels = timed_kernels(e, l);
+    if (kernel_id < 0 || kernel_id >= (int32_t)kernels.size() || reps < 0)
       throw Error(CHONK_EINVAL, "bad kernel id or repetitions");
-    const Launch& L = e->kernels_logits[(size_t)kernel_id];
+    const Launch& L = kernels[(size_t)kernel_id];
     if (reps > 0 && L.kind == Launch::SEL)
       throw Error(CHONK_EINVAL, "the select kernel advances the position; not timed alone");
     if (e->pos >= c.ctx) throw context_exhausted(e);
@@ -3439,9 +3468,11 @@ int chonk_engine_bench_kernel_cold(chonk_engine* e, int32_t kernel_id, int32_t r
                                    double* cold_us, double* warm_us) {
   return api(e, [&] {
     const ModelCfg& c = e->cfg;
-    if (kernel_id < 0 || kernel_id >= (int32_t)e->kernels_logits.size() || reps <= 0)
+    std::unique_lock<std::mutex> l;
+    const std::vector<Launch>& kernels = timed_kernels(e, l);
+    if (kernel_id < 0 || kernel_id >= (int32_t)kernels.size() || reps <= 0)
       throw Error(CHONK_EINVAL, "bad kernel id or repetitions");
-    const Launch& L = e->kernels_logits[(size_t)kernel_id];
+    const Launch& L = kernels[(size_t)kernel_id];
     if (L.kind == Launch::SEL) throw Error(CHONK_EINVAL, "the select kernel advances the position; not timed alone");
     if (e->pos >= c.ctx) throw context_exhausted(e);
     flush_bytes = std::max<uint64_t>(flush_bytes, (uint64_t)512 << 20);

@@ -7,10 +7,12 @@ and outside Gemma-3's window, and past 128 chunks, where workgroups walk several
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from chonklm_amd import WORKLOADS, load_llama_wgsl_model
+from chonklm_amd import WORKLOADS, _lib, load_llama_wgsl_model
 from tests.conftest import rel_err
 
 pytestmark = pytest.mark.gpu
@@ -46,4 +48,61 @@ def test_fp32_decode_attention_equals_chunked(name, ctx, positions, synth, monke
     assert info["spin_attention"] == 1 and ref_info["spin_attention"] == 0
     for i, (a, b) in enumerate(zip(got, want)):
         assert np.isfinite(a).all()
+        assert rel_err(a, b) <= 2e-5, f"step {i}: {rel_err(a, b):.2e}"
+
+
+def test_fp32_engine_leaves_the_attention_to_an_fp16_engine(synth, monkeypatch):
+    """An fp32 engine decodes with k_attn_dec while it is alone, with k_attention beside another
+    engine, and with k_attn_dec again afterwards: the logits of the chunked kernel throughout.
+    An fp16 engine created beside it has the spin-merging attention all the same."""
+    name, ctx = "tiny-qwen3", 400
+    monkeypatch.delenv("CHONK_ATTN", raising=False)
+
+    def load(kv):
+        md = WORKLOADS[name].model_def(synth(name), kv_dtype=kv)
+        md.max_context = ctx
+        return load_llama_wgsl_model(md).engine
+
+    def steps(eng, tok):
+        out = []
+        for _ in range(11):  # (a run of eight steps and more)
+            tok = eng.run_token(tok, True)
+            out.append(eng.read_logits().copy())
+        return out, tok
+
+    def walk(eng, beside):
+        eng.fake_context(120, seed=5)
+        a, tok = steps(eng, 9)
+        with_other = beside()
+        b, tok = steps(eng, tok)
+        eng.bench_decode(0, 17)  # runs of steps: the multi-step graph
+        if with_other:
+            with_other.dispose()
+        c, tok = steps(eng, tok)
+        return a + b + c
+
+    def spin(eng):  # (engine.info is as of the load)
+        info = _lib.EngineInfoC()
+        _lib.check(_lib.lib().chonk_engine_info_get(eng._h, C.byref(info)), eng._h)
+        return info.spin_attention
+
+    eng = load("f32")
+    assert spin(eng) == 1
+    seen = {}
+
+    def fp16():
+        other = load("f16")
+        seen.update(fp16=spin(other), fp32=spin(eng))
+        other.fake_context(50, seed=1)
+        other.run_token(3, True)
+        return other
+
+    got = walk(eng, fp16)
+    assert seen == dict(fp16=1, fp32=0) and spin(eng) == 1
+    eng.dispose()
+    monkeypatch.setenv("CHONK_ATTN", "chunked")
+    ref = load("f32")
+    want = walk(ref, lambda: None)
+    ref.dispose()
+    for i, (a, b) in enumerate(zip(got, want)):
         assert rel_err(a, b) <= 2e-5, f"step {i}: {rel_err(a, b):.2e}"
