@@ -61,6 +61,13 @@ __device__ __forceinline__ half2_t bytes01(uint32_t w) {
 __device__ __forceinline__ half2_t bytes23(uint32_t w) {
   return as_half2(__builtin_amdgcn_perm(0x64646464u, w, 0x04030402u));
 }
+// Orders the LDS accesses of a wave's lanes before and after it. The hardware keeps
+// them in order; this keeps the compiler from moving them.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 // sixteen halves at dst (16-byte aligned)
 __device__ __forceinline__ void put16(_Float16* dst, const half2_t (&v)[8]) {
   uint32_t u[8];
@@ -544,7 +551,7 @@ __global__ __launch_bounds__(kWg, (gemm_int_blocks<T> && NI == 4 ? 3 : 2)) void 
       }
       *(float4_t*)(tile + col * OS + 16 * i + 4 * quad) = v;
     }
-    // (the wave's own LDS accesses are in order)
+    wave_lds_order();  // the lanes read what other lanes wrote
 #pragma unroll
     for (int r = 0; r < 16; r += 64 / LPT) {
       const int tr = r + lane / LPT, cc = 4 * (lane % LPT), tt = tt0 + tr, n = c0 + cc;
@@ -565,6 +572,7 @@ __global__ __launch_bounds__(kWg, (gemm_int_blocks<T> && NI == 4 ? 3 : 2)) void 
           y[q] = a.epi == GEMM_ADD ? __fadd_rn(y[q], v[q]) : v[q];
       }
     }
+    wave_lds_order();  // the next token tile overwrites them
   }
 }
 
