@@ -502,6 +502,16 @@ struct LayerDev {
   void *kc = nullptr, *vc = nullptr;
 };
 
+// Device buffers of a row batch (rows <= cap).
+struct RowBufs {
+  float *x = nullptr, *qkv = nullptr, *att = nullptr, *xscale = nullptr, *part = nullptr;
+  float *xbc = nullptr, *y = nullptr;  // Mamba2 layers: the convolved rows, the scan's output
+  _Float16 *h = nullptr, *l = nullptr, *xs = nullptr;
+  int32_t* tok = nullptr;
+  int cap = 0;
+  int64_t part_cap = 0;  // floats in part
+};
+
 struct Launch {
   // QKVATTN: the q|k|v matvec (mv, nq workgroups) and the decode attention (at)
   // in one launch (k_qkv_attn)
@@ -598,10 +608,8 @@ struct chonk_engine {
   int rows_min = 1;  // fewest prompt tokens that go through the row-batch pass (fewer: decode steps)
   uint8_t* scratch = nullptr;  // device address of this GPU's no-allocation prompt-pass scratch
   int noalloc_rows = 0;        // rows one chonk_engine_prefill_noalloc call may take (0: none)
-  void* pf_mem = nullptr;
-  float *pf_x = nullptr, *pf_qkv = nullptr, *pf_att = nullptr, *pf_g = nullptr, *pf_u = nullptr, *pf_d = nullptr, *pf_xscale = nullptr, *pf_part = nullptr;
-  _Float16 *pf_h = nullptr, *pf_l = nullptr, *pf_xs = nullptr;
-  int32_t* pf_tok = nullptr;
+  void *pf_mem = nullptr, *pf_part = nullptr;
+  RowBufs pf;
   // status
   std::atomic<bool> busy{false};
   bool lost = false;
@@ -1678,6 +1686,7 @@ void engine_free(chonk_engine* e) {
   e->state.release();
   uncached_pool().give_back(e->device, e->uncached);
   if (e->pf_mem) (void)hipFree(e->pf_mem);
+  if (e->pf_part) (void)hipFree(e->pf_part);
   if (e->flush) (void)hipFree(e->flush);
   for (auto& t : e->rope_cs) (void)hipFree(t.second);
   if (e->h_state) (void)hipHostFree(e->h_state);
@@ -2335,15 +2344,6 @@ Error device_error(chonk_engine* e, const DevState& st) {
 constexpr int kPrefillRows = 2048;  // prompt rows per pass (longer prompts take several)
 constexpr int64_t kPartFloats = (int64_t)4 << 20;  // K-split partial sums
 
-// Device buffers of a row batch (rows <= cap).
-struct RowBufs {
-  float *x = nullptr, *qkv = nullptr, *att = nullptr, *g = nullptr, *u = nullptr, *d = nullptr, *xscale = nullptr, *part = nullptr;
-  _Float16 *h = nullptr, *l = nullptr, *xs = nullptr;
-  int32_t* tok = nullptr;
-  int cap = 0;
-  int64_t part_cap = 0;  // floats in part
-};
-
 // Floats of the partial-sum buffer for `rows` rows: room for every deferred
 // GEMM result of a layer without a K split, and at least kPartFloats.
 int64_t row_part_floats(const ModelCfg& c, int rows) {
@@ -2354,21 +2354,21 @@ int64_t row_part_floats(const ModelCfg& c, int rows) {
   return std::max<int64_t>({kPartFloats, R * qkv, 2 * R * c.ffn, R * c.hidden, R * in_proj});
 }
 
-// Sizes the buffers of `rows` rows for the engine's model; returns the bytes
-// needed and, with base != null, carves them from base.
-size_t row_bufs_layout(const ModelCfg& c, int rows, uint8_t* base, RowBufs* out) {
+// Sizes the buffers of `rows` rows for the engine's model and part_floats floats
+// of partial sums (0: kept elsewhere); returns the bytes needed and, with base !=
+// null, carves them from base.
+size_t row_bufs_layout(const ModelCfg& c, int rows, int64_t part_floats, uint8_t* base, RowBufs* out) {
   const size_t R = rows;
   const size_t H = c.hidden, qdim = (size_t)c.heads * c.hd, kvdim = (size_t)c.kv_heads * c.hd, F = c.ffn;
-  // (Mamba2 layers: the convolved rows in g, the scan's output in u)
-  const size_t inner = c.ssm_inner, G = std::max(F, inner ? (size_t)pf_mamba_ld(c.ssm_conv, c.ssm_heads) : 0);
+  const size_t inner = c.ssm_inner, xbc = inner ? (size_t)pf_mamba_ld(c.ssm_conv, c.ssm_heads) : 0;
   const size_t kmax = gemm_kpad((int)std::max({H, qdim, F, inner}));
-  const size_t sizes[12] = {R * H * 4, R * (qdim + 2 * kvdim) * 4, R * qdim * 4, R * G * 4,
-                            R * std::max(F, inner) * 4, std::max(R * F * 4, R * (kmax / 32) * 4),
-                            R * H * 4, R * 4, (size_t)row_part_floats(c, rows) * 4, plane_rows(rows) * kmax * 2,
-                            plane_rows(rows) * kmax * 2, R * 4};
+  const size_t plane = plane_rows(rows) * kmax * 2;
+  const size_t sizes[11] = {R * H * 4,          R * (qdim + 2 * kvdim) * 4, R * qdim * 4, R * xbc * 4,
+                            R * inner * 4,      R * (kmax / 32) * 4,        R * 4,        (size_t)part_floats * 4,
+                            plane,              plane,                      R * 4};
   size_t off = 0;
-  void* ptr[12];
-  for (int i = 0; i < 12; ++i) {
+  void* ptr[11];
+  for (int i = 0; i < 11; ++i) {
     ptr[i] = base ? base + off : nullptr;
     off += align256(sizes[i]);
   }
@@ -2376,17 +2376,16 @@ size_t row_bufs_layout(const ModelCfg& c, int rows, uint8_t* base, RowBufs* out)
     out->x = (float*)ptr[0];
     out->qkv = (float*)ptr[1];
     out->att = (float*)ptr[2];
-    out->g = (float*)ptr[3];
-    out->u = (float*)ptr[4];
+    out->xbc = (float*)ptr[3];
+    out->y = (float*)ptr[4];
     out->xs = (_Float16*)ptr[5];
-    out->d = (float*)ptr[6];
-    out->xscale = (float*)ptr[7];
-    out->part = (float*)ptr[8];
-    out->h = (_Float16*)ptr[9];
-    out->l = (_Float16*)ptr[10];
-    out->tok = (int32_t*)ptr[11];
+    out->xscale = (float*)ptr[6];
+    out->part = (float*)ptr[7];
+    out->h = (_Float16*)ptr[8];
+    out->l = (_Float16*)ptr[9];
+    out->tok = (int32_t*)ptr[10];
     out->cap = rows;
-    out->part_cap = row_part_floats(c, rows);
+    out->part_cap = part_floats;
   }
   return off;
 }
@@ -2549,13 +2548,13 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
       m.d = L.d_w;
       m.conv_state = L.mconv_state;
       m.ssm_state = L.ssm_state;
-      m.xbc = b.g;
-      m.y = b.u;
+      m.xbc = b.xbc;
+      m.y = b.y;
       HIP_OK(launch_pf_mamba(m, s));
       if (last_kv) break;
       PfGateArgs gt{};
       gt.z = columns(m.p, 0, c.ssm_inner);
-      gt.y = b.u;
+      gt.y = b.y;
       gt.w = L.ssm_norm;
       gt.k = c.ssm_inner;
       gt.kpad = gemm_kpad(c.ssm_inner);
@@ -2698,47 +2697,28 @@ void run_rows(chonk_engine* e, const RowBufs& b, const RowKv& kvs, const RowPlac
 // the no-allocation scratch (0 when not even 16 rows fit).
 int noalloc_rows_for(const ModelCfg& c) {
   for (int r = kPrefillRows; r >= 16; r -= 16)
-    if (row_bufs_layout(c, r, nullptr, nullptr) <= kNoAllocScratchBytes) return r;
+    if (row_bufs_layout(c, r, row_part_floats(c, r), nullptr, nullptr) <= kNoAllocScratchBytes) return r;
   return 0;
 }
 
-void prefill_alloc(chonk_engine* e) {
-  if (e->pf_mem) return;
-  RowBufs b;
-  const size_t bytes = row_bufs_layout(e->cfg, kPrefillRows, nullptr, nullptr);
-  HIP_OK(hipMalloc(&e->pf_mem, bytes));
-  row_bufs_layout(e->cfg, kPrefillRows, (uint8_t*)e->pf_mem, &b);
-  e->pf_x = b.x;
-  e->pf_qkv = b.qkv;
-  e->pf_att = b.att;
-  e->pf_g = b.g;
-  e->pf_u = b.u;
-  e->pf_xs = b.xs;
-  e->pf_d = b.d;
-  e->pf_xscale = b.xscale;
-  e->pf_part = b.part;
-  e->pf_h = b.h;
-  e->pf_l = b.l;
-  e->pf_tok = b.tok;
-}
-
-RowBufs engine_row_bufs(const chonk_engine* e) {
-  RowBufs b;
-  b.x = e->pf_x;
-  b.qkv = e->pf_qkv;
-  b.att = e->pf_att;
-  b.g = e->pf_g;
-  b.u = e->pf_u;
-  b.xs = e->pf_xs;
-  b.d = e->pf_d;
-  b.xscale = e->pf_xscale;
-  b.part = e->pf_part;
-  b.h = e->pf_h;
-  b.l = e->pf_l;
-  b.tok = e->pf_tok;
-  b.cap = kPrefillRows;
-  b.part_cap = row_part_floats(e->cfg, kPrefillRows);
-  return b;
+// The engine's row buffers for a prompt of n tokens: made on the first call, made
+// larger (a power of two of rows, at least 256) by a longer prompt. The partial
+// sums are those of a full pass from the start, as they decide how K is split: a
+// pass gives the same values whatever came before it.
+void prefill_alloc(chonk_engine* e, int n) {
+  const int want = std::min(n, kPrefillRows);
+  if (e->pf.cap >= want) return;
+  int rows = 256;
+  while (rows < want) rows *= 2;
+  const int64_t part = row_part_floats(e->cfg, kPrefillRows);
+  if (!e->pf_part) HIP_OK(hipMalloc(&e->pf_part, (size_t)part * 4));
+  e->pf = RowBufs{};
+  if (e->pf_mem) HIP_OK(hipFree(e->pf_mem));  // (no pass is in flight: each is waited for)
+  e->pf_mem = nullptr;
+  HIP_OK(hipMalloc(&e->pf_mem, row_bufs_layout(e->cfg, rows, 0, nullptr, nullptr)));
+  row_bufs_layout(e->cfg, rows, 0, (uint8_t*)e->pf_mem, &e->pf);
+  e->pf.part = (float*)e->pf_part;
+  e->pf.part_cap = part;
 }
 
 // K/V of every layer for tokens[0, n) at positions e->pos .. e->pos + n - 1,
@@ -2749,8 +2729,8 @@ void prefill_rows_in(chonk_engine* e, const RowBufs& b, const int32_t* tokens, i
 
 void prefill_rows(chonk_engine* e, const int32_t* tokens, int n) {
   if (n <= 0) return;
-  prefill_alloc(e);
-  prefill_rows_in(e, engine_row_bufs(e), tokens, n);
+  prefill_alloc(e, n);
+  prefill_rows_in(e, e->pf, tokens, n);
 }
 
 // The same pass with row buffers b (passes of at most b.cap rows).
@@ -3185,7 +3165,7 @@ int chonk_engine_prefill_noalloc(chonk_engine* e, const int32_t* tokens, size_t 
     // pass has finished on the device)
     std::lock_guard<std::mutex> scratch_turn(scratch_lock(e->device));
     RowBufs b;
-    row_bufs_layout(e->cfg, e->noalloc_rows, e->scratch, &b);
+    row_bufs_layout(e->cfg, e->noalloc_rows, row_part_floats(e->cfg, e->noalloc_rows), e->scratch, &b);
     HIP_OK(hipMemcpy(e->hist + e->pos, tokens, n * 4, hipMemcpyHostToDevice));
     prefill_rows_in(e, b, tokens, (int)n);
     e->pos += (int)n;
@@ -3832,12 +3812,13 @@ void batch_create(chonk_engine* e, int max_seqs, int max_tokens, chonk_batch** o
     b->kvs.kc.push_back((uint8_t*)b->kv_mem + pool * 2 * i);
     b->kvs.vc.push_back((uint8_t*)b->kv_mem + pool * (2 * i + 1));
   }
-  const size_t rb = row_bufs_layout(c, b->rows_cap, nullptr, nullptr);
+  const int64_t part = row_part_floats(c, b->rows_cap);
+  const size_t rb = row_bufs_layout(c, b->rows_cap, part, nullptr, nullptr);
   const size_t tab = align256(n_pages * 4), arr = align256((size_t)b->rows_cap * 4);
   const size_t lg = align256((size_t)max_seqs * c.vocab * 4);
   HIP_OK(hipMalloc(&b->row_mem, rb + tab + 3 * arr + lg));
   uint8_t* p = (uint8_t*)b->row_mem;
-  row_bufs_layout(c, b->rows_cap, p, &b->b);
+  row_bufs_layout(c, b->rows_cap, part, p, &b->b);
   p += rb;
   b->pages = (int32_t*)p;
   p += tab;

@@ -7,6 +7,8 @@ follow it.
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -185,3 +187,30 @@ def test_continued_conversation_equals_steps(name, more, synth):
     assert got == want
     assert (eng.read_logits() == logits).all()
     eng.dispose()
+
+
+def _free_mib():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL("libamdhip64.so").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value / 2 ** 20
+
+
+# MiB of a short prompt's buffers: 256 rows of (x, q|k|v, attention, block sums, two planes)
+# floats or halves, and the partial sums of 2048 rows of the widest result, 2 ffn (or in_proj)
+@pytest.mark.parametrize("name,most", [("gpt2-124m-q4_k_m", 60), ("lfm2.5-350m-q4_k_m", 90),
+                                       ("openelm-270m-q4_k_m", 100), ("qwen3-0.6b-q4_k_m", 70)])
+def test_short_prompts_take_little_memory(name, most, synth):
+    w = WORKLOADS[name]
+    eng = _load(name, synth).engine
+    tokens = np.random.default_rng(1).integers(0, w.spec.vocab, 20).tolist()
+    eng.run_token(tokens[0], True)
+    before = _free_mib()
+    eng.prefill(tokens)
+    assert before - _free_mib() <= most
+    eng.dispose()
+
+
+@pytest.mark.parametrize("name", ["tiny-qwen3", "tiny-lfm2", "tiny-granite-q8"])
+def test_longer_prompts_make_the_buffers_larger(name, synth):
+    """20, 300 and 900 rows: each call's buffers replace smaller ones; the states stay."""
+    _same_state(name, (20, 300, 900), synth, max_context=1300)
