@@ -585,12 +585,10 @@ hipError_t launch_one(const GemmArgs& a, int n_rows, hipStream_t s) {
 
 template <int T>
 hipError_t launch_type(const GemmArgs& a, int n_rows, int ni, int tj, hipStream_t s) {
-  if (a.epi == GEMM_SWIGLU || a.epi == GEMM_GEGLU) {
-    if (ni == 8) return tj == 2 ? launch_one<T, 8, 2, true>(a, n_rows, s) : launch_one<T, 8, 1, true>(a, n_rows, s);
-    return tj == 2 ? hipErrorInvalidValue : launch_one<T, 4, 1, true>(a, n_rows, s);
-  }
-  if (ni == 8) return tj == 2 ? launch_one<T, 8, 2, false>(a, n_rows, s) : launch_one<T, 8, 1, false>(a, n_rows, s);
-  return tj == 2 ? launch_one<T, 4, 2, false>(a, n_rows, s) : launch_one<T, 4, 1, false>(a, n_rows, s);
+  const bool glu = a.epi == GEMM_SWIGLU || a.epi == GEMM_GEGLU;
+  if (ni == 8 && tj == 2) return glu ? launch_one<T, 8, 2, true>(a, n_rows, s) : launch_one<T, 8, 2, false>(a, n_rows, s);
+  if (ni == 4 && tj == 1) return glu ? launch_one<T, 4, 1, true>(a, n_rows, s) : launch_one<T, 4, 1, false>(a, n_rows, s);
+  return ni == 4 && tj == 2 && !glu ? launch_one<T, 4, 2, false>(a, n_rows, s) : hipErrorInvalidValue;
 }
 
 template <int T, int NI, int TJ, bool GLU>
@@ -600,9 +598,8 @@ hipError_t init_one() {
 }
 template <int T>
 hipError_t init_type() {
-  for (hipError_t e : {init_one<T, 8, 2, false>(), init_one<T, 8, 1, false>(), init_one<T, 4, 2, false>(),
-                       init_one<T, 4, 1, false>(), init_one<T, 8, 2, true>(), init_one<T, 8, 1, true>(),
-                       init_one<T, 4, 1, true>()})
+  for (hipError_t e : {init_one<T, 8, 2, false>(), init_one<T, 4, 2, false>(), init_one<T, 4, 1, false>(),
+                       init_one<T, 8, 2, true>(), init_one<T, 4, 1, true>()})
     if (e != hipSuccess) return e;
   return hipSuccess;
 }

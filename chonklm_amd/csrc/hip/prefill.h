@@ -172,7 +172,8 @@ __host__ __device__ inline size_t plane_at(int row, int col, int kpad) {
 constexpr int gemm_kpad(int k) { return (k + 127) / 128 * 128; }
 
 // The GEMM over the weights' integer codes (gemm_int.hip): 16 ni weight rows x
-// 64 tj token rows per workgroup (ni 4 or 8, tj 1 or 2), a.ksplit and the output
+// 64 tj token rows per workgroup ((ni, tj) of (8, 2), (4, 1) or, without a GLU
+// epilogue, (4, 2)), a.ksplit and the output
 // as set by the caller. K splits are whole steps of gemm_int_step columns; types
 // with block offsets (gemm_int_sums) need a.xs.
 bool gemm_int_sums(int type);
@@ -202,7 +203,6 @@ hipError_t launch_pf_conv(const PfConvArgs& a, int rows, hipStream_t s);
 hipError_t launch_pf_conv_state(const PfConvArgs& a, int rows, hipStream_t s);
 hipError_t launch_pf_mamba(const PfMambaArgs& a, hipStream_t s);
 hipError_t launch_pf_gate(const PfGateArgs& a, int rows, hipStream_t s);
-hipError_t launch_pf_norm_add(const float* d, const float* w, float eps, int k, float* x, int rows, hipStream_t s);
 hipError_t launch_pf_glu_split(const PfGluArgs& a, int rows, hipStream_t s);
 hipError_t launch_pf_rope_kv(const PfRopeArgs& a, int rows, hipStream_t s);
 hipError_t launch_pf_attn(const PfAttnArgs& a, int rows, hipStream_t s);

@@ -688,8 +688,6 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_sk1(GemmArgs a) {
   }
 }
 
-// s_waitcnt immediate that waits for vmcnt <= n only (gfx9 encoding: vmcnt in
-// bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
 // The same for a matrix with many row groups (the lm_head): a workgroup owns
 // 4 x 64 weight rows over the whole K, the four waves sharing each 64-k block
 // of x operands, copied into LDS one block ahead (two buffers; each wave
@@ -888,23 +886,6 @@ __global__ __launch_bounds__(kWg) void k_pf_embed(QMat embed, const int32_t* tok
       }
     }
   });
-}
-
-// x = clamp(x + RMSNorm(d) * w, +-65000) per token row (the Gemma-3 sandwich
-// residual, as the decode prologue PRO_RES_NORM computes it).
-__global__ __launch_bounds__(kWg) void k_pf_norm_add(const float* d, const float* w, float eps, int k, float* x) {
-  __shared__ float red[8];
-  const int t = blockIdx.x, tid = threadIdx.x;
-  const float* dr = d + (size_t)t * k;
-  float* xr = x + (size_t)t * k;
-  float ss = 0.f;
-  for (int i = tid; i < k; i += kWg) ss += dr[i] * dr[i];
-  ss = block_sum(ss, red);
-  const float inv = 1.0f / sqrtf(ss / (float)k + eps);
-  for (int i = tid; i < k; i += kWg) {
-    const float nd = __fmul_rn(__fmul_rn(dr[i], inv), w[i]);
-    xr[i] = fminf(fmaxf(__fadd_rn(xr[i], nd), -65000.0f), 65000.0f);
-  }
 }
 
 // silu(g) * u, gelu_tanh(g) * u or (GPT-2) gelu_tanh(u + bias) per element (or
@@ -2334,10 +2315,6 @@ hipError_t launch_pf_mamba(const PfMambaArgs& a, hipStream_t s) {
 }
 hipError_t launch_pf_gate(const PfGateArgs& a, int rows, hipStream_t s) {
   CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_gate<TPR, E>), grid, dim3(kWg), 0, s, a, rows));
-}
-hipError_t launch_pf_norm_add(const float* d, const float* w, float eps, int k, float* x, int rows, hipStream_t s) {
-  hipLaunchKernelGGL(k_pf_norm_add, dim3(rows), dim3(kWg), 0, s, d, w, eps, k, x);
-  return hipGetLastError();
 }
 hipError_t launch_pf_glu_split(const PfGluArgs& a, int rows, hipStream_t s) {
   CHONK_ROW_CASE(a.kpad, hipLaunchKernelGGL((k_pf_glu_split<TPR, E>), grid, dim3(kWg), 0, s, a, rows));
