@@ -711,15 +711,15 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
   int rows[4];
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) rows[rt] = min(n0 + 16 * rt + r16, N - 1);
-  // x of block b into buffer b & 1: this wave's NT of its 4 NT 1-KiB copies
-  auto copy_x = [&](int b) {
+  // x of block b into buffer buf: this wave's NT of its 4 NT 1-KiB copies
+  auto copy_x = [&](int b, int buf) {
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int c = wave * NT + j, p = c / (2 * NT), s2 = (c / NT) & 1, i = c % NT;
       const _Float16* src =
           (p ? a.xl : a.xh) + plane_at(16 * min(i, (a.t - 1) / 16), sk_col<T>(b, s2), a.kpad) + 8 * lane;
       __builtin_amdgcn_global_load_lds((gmem_void*)src,
-                                       (lds_void*)(xb + (((b & 1) * 4 + p * 2 + s2) * NT + i) * 512), 16, 0, 0);
+                                       (lds_void*)(xb + ((buf * 4 + p * 2 + s2) * NT + i) * 512), 16, 0, 0);
     }
   };
   if (tid < a.t) xs[tid] = a.xscale[tid];
@@ -727,7 +727,7 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
 #pragma unroll
   for (int rt = 0; rt < 4; ++rt) cur[rt] = sk_load<T>(a.w, rows[rt], 0, g);
   __builtin_amdgcn_sched_barrier(0);
-  copy_x(0);
+  copy_x(0, 0);
   __builtin_amdgcn_sched_barrier(0);
   float4_t acc[NT][4];
 #pragma unroll
@@ -735,15 +735,15 @@ __global__ __launch_bounds__(kWg, 2) void k_gemm_lm(GemmArgs a) {
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) acc[tt][rt] = float4_t{0.f, 0.f, 0.f, 0.f};
   for (int b = 0; b < nblk; ++b) {
-    // the next block's weights, then its x copies (the last block copies
-    // itself into the other buffer, which is not read again: the loop body
-    // stays branch-free, so every wait counts exactly)
+    // the next block's weights, then its x copies into the other buffer (the last
+    // block copies itself there, where nothing reads it: the loop body stays
+    // branch-free, so every wait counts exactly)
     const int bn = min(b + 1, nblk - 1);
     SkBlock<T> nxt[4];
 #pragma unroll
     for (int rt = 0; rt < 4; ++rt) nxt[rt] = sk_load<T>(a.w, rows[rt], bn, g);
     __builtin_amdgcn_sched_barrier(0);
-    copy_x(bn);
+    copy_x(bn, (b + 1) & 1);
     __builtin_amdgcn_sched_barrier(0);
     // this block's copies have landed once at most the loads issued after
     // them are outstanding: the next block's W weight loads and NT copies
