@@ -61,10 +61,15 @@ def test_error_of_32_weight_blocks(tname, bar, n_rows, row_len, n_tok):
     assert err <= bar * 2.0 ** -25, f"{tname}: {err:.2e}"
 
 
+# gate | up leave the GEMM as their product where its tiles are 64 x 64 or 128 x 128 and K is
+# not split; 64 x 128 tiles leave both
 @pytest.mark.parametrize("name,parts", [
-    ("qwen3-0.6b-q4_k_m", (300, 600)),   # gate * up inside the GEMM (SwiGLU), one wave's and four waves' rows
-    ("gemma3-270m-q4_k_m", (300,)),      # ... with GELU
-    ("smollm2-135m-q8_0", (1030,)),      # a wave per row in the glue kernels
+    ("qwen3-0.6b-q4_k_m", (300, 600)),   # 64 x 64 (Q4_K, SwiGLU), then 64 x 128; two and four waves per row in the glue
+    ("qwen3-0.6b-q4_k_m", (1030,)),      # 128 x 128, six rows in the last tile; a wave per row in the glue
+    ("gemma3-270m-q4_k_m", (300,)),      # 64 x 64, Q5_0, GELU
+    ("gemma3-270m-q4_k_m", (1301,)),     # 128 x 128, Q5_0, GELU
+    ("lfm2.5-350m-q8_0", (601,)),        # 128 x 128, Q8_0
+    ("smollm2-135m-q8_0", (1030,)),      # 64 x 128, Q8_0; K ends inside a stage
 ])
 def test_prompt_pass_of_the_workloads_equals_steps(name, parts, synth):
     _same_state(name, parts, synth, max_context=sum(parts) + 8)
