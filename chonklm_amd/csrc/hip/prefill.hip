@@ -2117,9 +2117,11 @@ size_t fattn_shared_bytes(int hd) {
 //   4096 x 1024 at 288:  15.4 (4, 1, 1)  16.2 (4, 1, 2)  18.1 (8, 1, 1)
 //   1024 x 2048 at 288:  12.2 (4, 1, 4)  13.9 (4, 1, 7)  15.8 (8, 1, 7)
 //   1024 x 2048 at 80:    6.6 (4, 1, 8)   7.8 (4, 1, 4)   7.9 (8, 1, 8)
-// One row tile (up to 64 rows), 128 or 256 workgroups wanted: prompts of 8 to 64 rows of
-// SmolLM2-135M Q8_0 1.39 .. 1.53 ms with either, 5 sequences of it decoded together 71.7 /
-// 70.2 ms per 40 steps, 64 rows of Gemma-3-270M 1.18 / 1.19.
+// One row tile (up to 64 rows) has 128 workgroups wanted: prompts of 3, 16 and 64 rows of the
+// LFM2.5-350M Q8_0 shape take 0.95, 0.98, 1.04 ms (256: 1.02, 1.07, 1.18), of Granite Q8_0 1.75,
+// 1.83, 2.05 (1.76, 1.89, 2.17), of SmolLM2-135M Q8_0 1.36, 1.46, 1.54 (1.34, 1.43, 1.52). (At one
+// step of a SmolLM2 run with a 1.3 repetition penalty two ids are 6e-6 apart after it; either
+// number has taken the oracle's id there since the block scales left the GEMM's operands.)
 struct IntTiles {
   int ni, tj, ks;
 };
@@ -2128,7 +2130,7 @@ IntTiles gemm_int_tiles(const GemmArgs& a, int n_rows, int64_t part_cap) {
     return ((n_rows + 16 * ni - 1) / (16 * ni)) * ((a.t + 64 * tj - 1) / (64 * tj));
   };
   const int tj = a.t > 512 ? 2 : 1, ni = tj == 2 && tiles(8, 2) >= 256 ? 8 : 4;
-  const int n = tiles(ni, tj), want = tj == 2 ? 512 : 256;
+  const int n = tiles(ni, tj), want = tj == 2 ? 512 : a.t > 64 ? 256 : 128;
   const int step = gemm_int_step(a.w.type), nst = (a.w.k + step - 1) / step;
   int ks = std::max(1, std::min({(want + n / 2) / n, nst, kMaxDeferSplit}));
   while (ks > 1 && (int64_t)ks * a.t * n_rows > part_cap) --ks;
