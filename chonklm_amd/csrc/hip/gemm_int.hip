@@ -20,17 +20,17 @@
 //
 // Chains are kept short: the matrix core rounds several times per step at the
 // size of what it adds to. Q8_0 as two planes in one chain over K was 1.6e-7 to
-// 3.6e-7 from float64 (8.4e-8 to 9.6e-8 now; 9216 x 1024 at 300 rows 32.7 -> 29.9 us,
-// 3376 x 768 at 2047 49.3 -> 48.3, 1024 x 1024 at 200 13.8 -> 14.1), and the logits
+// 3.6e-7 from float64 (8.4e-8 to 9.6e-8 now; 9216 x 1024 at 300 rows 32.7 -> 29.2 us,
+// 3376 x 768 at 2047 49.3 -> 48.3, 1024 x 1024 at 200 13.7 -> 13.7), and the logits
 // after a Granite or LFM2 Q8_0 prompt (fp32 cache) 1.4e-6 or 2.6e-6, where a prompt
 // in decode steps leaves 8.5e-7 or 1.53e-6 (8.5e-7 and 1.53e-6 now).
 //
 // Against the three-product GEMM over fp32-dequantized hi + lo weights that it
 // replaced (MI355X, 2047 token rows): Q4_K 4096 x 1024 95.0 -> 47.9 us, 6144 x 1024
 // 139.5 -> 65.2, Q6_K 1024 x 3072 90.6 -> 41.2; error against float64 3.6e-7 -> 1.4e-7
-// (Q4_K), 6.2e-7 -> 1.7e-7 (Q6_K). What is left: 16 us of the 4096-row launch are its
-// 34 MB of fp32 results, the rest is the products at the rate the matrix cores
-// sustain beside the staging.
+// (Q4_K), 6.2e-7 -> 1.7e-7 (Q6_K). What is left (6144 x 1024, gate * up, 60.4 us): the
+// matrix cores are busy 46% of the CUs' busy cycles and LDS 39%, the rest are the
+// stages' conversions and barriers.
 #include <hip/hip_runtime.h>
 
 #include "kernel_common.h"
@@ -473,14 +473,16 @@ __global__ __launch_bounds__(kWg, (gemm_int_blocks<T> && NI == 4 ? 3 : 2)) void 
     }
     if constexpr (BLK) join(NF - 1);
     // (schedule: AD LDS reads, then per fragment one read and its products; BLK:
-    // two reads, the products and the fused multiplies of the fragment before)
+    // two reads, the products and, with two token tiles, the fused multiplies of the
+    // fragment before. With one they find their own place: 3 rows of the LFM2.5-350M
+    // Q8_0 shape take 0.90 ms, 0.945 with a group for them)
     __builtin_amdgcn_sched_group_barrier(0x100, BLK ? 2 * AD : AD, 0);
 #pragma unroll
     for (int fi = 0; fi < NF; fi += NP) {
       if (fi % (NP * NI) == 0) __builtin_amdgcn_sched_group_barrier(0x20, 2 * TJ, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, BLK ? 2 : 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x8, 2 * TJ, 0);
-      if constexpr (BLK) __builtin_amdgcn_sched_group_barrier(0x2, 4 * TJ, 0);
+      if constexpr (BLK && TJ == 2) __builtin_amdgcn_sched_group_barrier(0x2, 4 * TJ, 0);
       if constexpr (NP == 2) {
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x8, TJ, 0);

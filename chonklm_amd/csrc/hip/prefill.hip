@@ -2118,8 +2118,8 @@ size_t fattn_shared_bytes(int hd) {
 //   1024 x 2048 at 288:  12.2 (4, 1, 4)  13.9 (4, 1, 7)  15.8 (8, 1, 7)
 //   1024 x 2048 at 80:    6.6 (4, 1, 8)   7.8 (4, 1, 4)   7.9 (8, 1, 8)
 // One row tile (up to 64 rows) has 128 workgroups wanted: prompts of 3, 16 and 64 rows of the
-// LFM2.5-350M Q8_0 shape take 0.95, 0.98, 1.04 ms (256: 1.02, 1.07, 1.18), of Granite Q8_0 1.75,
-// 1.83, 2.05 (1.76, 1.89, 2.17), of SmolLM2-135M Q8_0 1.36, 1.46, 1.54 (1.34, 1.43, 1.52). (At one
+// LFM2.5-350M Q8_0 shape take 0.90, 0.93, 0.99 ms (256: 1.00, 1.04, 1.16), of Granite Q8_0 1.70,
+// 1.79, 2.00 (1.73, 1.87, 2.14), of SmolLM2-135M Q8_0 1.34, 1.44, 1.51 (1.32, 1.42, 1.51). (At one
 // step of a SmolLM2 run with a 1.3 repetition penalty two ids are 6e-6 apart after it; either
 // number has taken the oracle's id there since the block scales left the GEMM's operands.)
 struct IntTiles {
