@@ -181,9 +181,10 @@ constexpr int kRowUnits = 4;
 hipError_t launch_matvec(const MvArgs& a, int grid, size_t shmem, hipStream_t s);
 hipError_t launch_attention(const AttnArgs& a, size_t shmem, hipStream_t s);
 hipError_t launch_ssm(const SsmArgs& a, hipStream_t s);
-// The register-resident decode attention (attn_decode.hip): fp16 cache,
+// The register-resident decode attention (attn_decode.hip): fp16 or fp32 cache,
 // head_dim 64/128/256, GQA group <= 8 (group x head_dim <= 1536), at most 128
-// chunks of attn_dec_chunk() positions over the context.
+// workgroups per kv head, each with one or (long contexts) several chunks of
+// attn_dec_chunk() positions.
 bool attn_dec_supported(int group, int hd, int ctx);
 int attn_dec_chunk();
 // 64-position sub-chunks per k_attn_dec workgroup at a context, with at most
